@@ -26,6 +26,13 @@
 //   big    int32[n_big]     spheres kept out of the tree (radius larger than
 //                           the region of the others, e.g. a ground sphere,
 //                           or non-finite data); tested by a flat loop first
+// For queries by whole waves (trace_tiles.h), the tree's spheres again, 32 to a
+// tile, neighbours together:
+//   tiles  uint4[n_tiles][128]  matrix operands in half precision
+//   tboxes float4[..][2]    box (centre, half size; tile units) of every tile,
+//                           then of every eight consecutive tiles
+//   tsph   float4[n_tree]   spheres in tile order (cx, cy, cz, r*r)
+//   tidx   int32[n_tree]    their index in the scene
 // Boxes are rounded outwards from double precision, so each contains its
 // spheres exactly.
 #pragma once
@@ -52,6 +59,13 @@ struct BvhDev {
     float sx, sy, sz;   // world size of one cell
     float isx, isy, isz;  // 1 / size (rounded)
     float ext;          // upper bound of 65535 * cell size over the axes
+    const uint4* tiles;
+    const float4* tboxes;
+    const float4* tsph;
+    const int32_t* tidx;
+    uint32_t n_tiles;
+    float ts;           // tile units per world unit (a power of two)
+    float t_lin;        // 2^-18 / smallest radius in tile units
 };
 
 }  // namespace atx

@@ -187,6 +187,128 @@ bool finite_sphere(const float* s)
            s[3] < 1e30f;
 }
 
+// Nearest half-precision number (ties to even); |x| < 65504.
+uint16_t half_bits(double x)
+{
+    const uint16_t sign = std::signbit(x) ? 0x8000u : 0u;
+    const double m = std::fabs(x);
+    if (m < 0x1p-14) return (uint16_t)(sign | (uint16_t)std::nearbyint(m * 0x1p24));   // subnormal: multiples of 2^-24
+    int e = 0;
+    const double f = std::frexp(m, &e);                       // m = f * 2^e, f in [0.5, 1)
+    const long q = (long)std::nearbyint(f * 2048.0);          // 11 significant bits
+    return (uint16_t)(sign | (uint16_t)(((e + 13) << 10) + q));   // a carry out of q moves the exponent up
+}
+
+double half_value(uint16_t h)
+{
+    const int e = (h >> 10) & 31, m = h & 1023;
+    const double v = e ? std::ldexp(1024.0 + m, e - 25) : std::ldexp((double)m, -24);
+    return h & 0x8000u ? -v : v;
+}
+
+// x as two halves: hi in the low 16 bits, the rest's nearest half above it.
+void half_split(double x, uint16_t& hi, uint16_t& lo)
+{
+    hi = half_bits(x);
+    lo = half_bits(x - half_value(hi));
+}
+
+// Orders spheres idx[b, e) so that every kTileSpheres of them lie close
+// together, and every eight such tiles too: halves along the longest side of
+// the centres' box, cut at a multiple of a tile (of eight tiles where there
+// are more than eight).
+void tile_order(const std::vector<float>& s, std::vector<uint32_t>& idx, size_t b, size_t e)
+{
+    const size_t tiles = (e - b + kTileSpheres - 1) / kTileSpheres;
+    if (tiles <= 1) return;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (size_t i = b; i < e; ++i)
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = std::min(lo[a], s[4 * idx[i] + a]);
+            hi[a] = std::max(hi[a], s[4 * idx[i] + a]);
+        }
+    int axis = 0;
+    for (int a = 1; a < 3; ++a)
+        if (hi[a] - lo[a] > hi[axis] - lo[axis]) axis = a;
+    const size_t unit = tiles > 8 ? 8 : 1;
+    const size_t left = ((tiles + 1) / 2 + unit - 1) / unit * unit;
+    const size_t m = std::min(e, b + left * kTileSpheres);
+    std::nth_element(idx.begin() + b, idx.begin() + m, idx.begin() + e, [&](uint32_t x, uint32_t y) {
+        return s[4 * x + axis] < s[4 * y + axis] || (s[4 * x + axis] == s[4 * y + axis] && x < y);
+    });
+    tile_order(s, idx, b, m);
+    tile_order(s, idx, m, e);
+}
+
+// Tiles of the tree's spheres (layout and error bound in trace_tiles.h).  Per
+// sphere 32 halves, of its centre c in tile units and w = |c|^2 - radius^2
+// (v = hi part, v' = lo part):
+//   twice each  xx yy zz 2xy 2xz 2yz 2x 2y 2z,  1 1 -w -w',
+//   xx' yy' zz' 2xy' 2xz' 2yz' 2x' 2y' 2z' 0
+// Lane l of a tile's k-th product (k = 0, 1) holds halves 16 k + 8 (l / 32) .. + 7
+// of the sphere in row l % 32.  Rows past the last sphere hold a sphere no ray
+// meets (-w far below zero, centre 0).
+void build_tiles(HostBvh* B)
+{
+    const uint32_t n = (uint32_t)B->lidx.size();
+    const double reach = ((double)B->rb + (double)B->r_max) * (1.0 + 0x1p-20);
+    int e = 0;
+    std::frexp(reach, &e);                                     // reach <= 2^e
+    const double ts = std::ldexp(1.0, 3 - e);                  // reach * ts <= 8
+    B->ts = (float)ts;
+    B->t_lin = round_up(std::min(0x1p-18 / std::max((double)B->r_min * ts, 1e-30), 1e6));
+    B->n_tiles = (n + kTileSpheres - 1) / kTileSpheres;
+    std::vector<uint32_t> order(n);
+    for (uint32_t k = 0; k < n; ++k) order[k] = k;
+    tile_order(B->lsph, order, 0, n);
+    B->tiles.assign((size_t)B->n_tiles * kTileWords, 0u);
+    const float centre[3] = {B->cx, B->cy, B->cz};
+    const uint32_t groups = (B->n_tiles + 7u) / 8u;
+    std::vector<double> lo(3 * (B->n_tiles + groups), INFINITY), hi(3 * (B->n_tiles + groups), -INFINITY);
+    for (uint32_t k = 0; k < B->n_tiles * kTileSpheres; ++k) {
+        const uint32_t t = k / kTileSpheres, g = B->n_tiles + t / 8u;
+        uint16_t v[32] = {};
+        v[18] = v[19] = half_bits(1.0);
+        if (k < n) {
+            const float* s = &B->lsph[4 * (size_t)order[k]];
+            B->tsph.insert(B->tsph.end(), s, s + 4);
+            B->tidx.push_back(B->lidx[order[k]]);
+            const double r = std::sqrt((double)s[3]) * ts * (1.0 + 0x1p-40);
+            double c[3], w = -(double)s[3] * ts * ts;
+            for (int a = 0; a < 3; ++a) {
+                c[a] = ((double)s[a] - (double)centre[a]) * ts;
+                w += c[a] * c[a];
+                for (uint32_t b : {t, g}) {
+                    lo[3 * b + a] = std::min(lo[3 * b + a], c[a] - r);
+                    hi[3 * b + a] = std::max(hi[3 * b + a], c[a] + r);
+                }
+            }
+            const double p[9] = {c[0] * c[0],       c[1] * c[1],       c[2] * c[2],
+                                 2.0 * c[0] * c[1], 2.0 * c[0] * c[2], 2.0 * c[1] * c[2],
+                                 2.0 * c[0],        2.0 * c[1],        2.0 * c[2]};
+            for (int j = 0; j < 9; ++j) {
+                half_split(p[j], v[2 * j], v[22 + j]);
+                v[2 * j + 1] = v[2 * j];
+            }
+            half_split(-w, v[20], v[21]);
+        } else {
+            v[20] = half_bits(-60000.0);
+        }
+        uint32_t* tile = &B->tiles[(size_t)t * kTileWords];
+        const uint32_t row = tile_row(k % kTileSpheres);
+        for (uint32_t j = 0; j < 32; j += 2)
+            tile[((j / 8) * 32u + row) * 4u + (j % 8) / 2] = v[j] | ((uint32_t)v[j + 1] << 16);
+    }
+    for (uint32_t b = 0; b < B->n_tiles + groups; ++b) {
+        float c[3], half[3];
+        for (int a = 0; a < 3; ++a) {
+            c[a] = (float)(0.5 * (lo[3 * b + a] + hi[3 * b + a]));
+            half[a] = round_up(std::max(hi[3 * b + a] - (double)c[a], (double)c[a] - lo[3 * b + a]));
+        }
+        B->tboxes.insert(B->tboxes.end(), {c[0], c[1], c[2], half[0], half[1], half[2], 0.0f, 0.0f});
+    }
+}
+
 }  // namespace
 
 void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
@@ -309,13 +431,17 @@ void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
     out->rb = round_up(rb * (1.0 + 0x1p-30));
     out->r_min = round_down(std::sqrt(r2_min) * (1.0 - 0x1p-30));
     out->r_max = round_up(std::sqrt(r2_max) * (1.0 + 0x1p-30));
+    build_tiles(out);
 }
 
 size_t bvh_device_bytes(uint64_t n)
 {
     const uint64_t nodes = n > 0 ? 2 * n - 1 : 0;
     return (size_t)(kBvhLayouts * nodes * 16 + 16) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16) +
-           (size_t)(4 * (kBvhMaxBig + 1) + 16);
+           (size_t)(4 * (kBvhMaxBig + 1) + 16) +
+           (n <= kBvhMaxTree + kBvhMaxBig
+                ? ((size_t)((n + 31) / 32) * (kTileWords * 4 + 36) + 64) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16)
+                : 0);
 }
 
 }  // namespace atx

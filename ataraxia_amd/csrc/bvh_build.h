@@ -14,6 +14,11 @@ constexpr uint32_t kBvhLeafMax = 4;      // spheres per leaf (2-bit count field)
 constexpr uint32_t kBvhMinSpheres = 16;  // smaller scenes use the flat loop only
 constexpr uint32_t kBvhMaxBig = 16;
 constexpr uint32_t kBvhMaxTree = 16382;  // tree spheres addressable by a 14-bit leaf index
+constexpr uint32_t kTileSpheres = 32;    // spheres per tile (rows of the matrix product)
+constexpr uint32_t kTileWords = 512;     // 32-bit words of one tile
+constexpr uint32_t kTileChunk = 8;       // tiles whose candidates are kept before they are tested
+constexpr uint32_t kTileRows = kTileChunk + 1;   // a wave's LDS rows: their masks, and their first spheres
+constexpr uint32_t kTileFlat = 16;       // with more tiles, every eight have a box of their own
 constexpr uint32_t kBvhGrid = 65535;     // node boxes are 16-bit cells of the tree's box
 
 // Node encoding (4 x u32 = 16 B): cell coordinates of the box corners,
@@ -32,7 +37,23 @@ struct HostBvh {
     float scale[3] = {1, 1, 1};  // world size of one cell per axis
     float inv_scale[3] = {1, 1, 1};
     float ext = 0;               // upper bound of kBvhGrid * scale over the axes
+    std::vector<uint32_t> tiles; // n_tiles * kTileWords, two halves per word
+    std::vector<float> tboxes;   // 8 per box: centre, half size, 0, 0; tiles, then groups of eight
+    std::vector<float> tsph;     // 4 per tree sphere, tile order
+    std::vector<int32_t> tidx;
+    uint32_t n_tiles = 0;
+    float ts = 0;                // tile units per world unit
+    float t_lin = 0;             // 2^-18 / smallest radius in tile units (capped)
 };
+
+// Row of a tile's matrix that holds its k-th sphere (k < kTileSpheres): the
+// product leaves row 8 * (i / 4) + 4 * h + i % 4 in register i of lane half h,
+// and the query collects register i of half h at bit 16 * h + 15 - i.
+inline uint32_t tile_row(uint32_t k)
+{
+    const uint32_t i = 15u - (k & 15u), h = k >> 4;
+    return 8u * (i / 4u) + 4u * h + i % 4u;
+}
 
 // Builds the tree over spheres given as (cx, cy, cz, r*r) quadruples, with
 // `layouts` traversal orders (1 or kBvhLayouts).  Scenes with fewer than

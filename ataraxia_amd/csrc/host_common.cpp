@@ -96,28 +96,32 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     build_bvh(L.sph.data(), (uint32_t)n, layouts, &T);
     out->bvh = BvhDev{};
     if (T.n_nodes > 0) {
-        ATX_HIP(out->bvh_nodes.reserve(T.nodes.size() * 4 + 16));
-        ATX_HIP(out->bvh_lsph.reserve(T.lsph.size() * 4 + 16));
-        ATX_HIP(out->bvh_lidx.reserve(T.lidx.size() * 4 + 16));
-        ATX_HIP(out->bvh_big.reserve(T.big.size() * 4 + 16));
-        ATX_HIP(hipMemcpy(out->bvh_nodes.get(), T.nodes.data(), T.nodes.size() * 4, hipMemcpyHostToDevice));
-        ATX_HIP(hipMemcpy(out->bvh_lsph.get(), T.lsph.data(), T.lsph.size() * 4, hipMemcpyHostToDevice));
-        ATX_HIP(hipMemcpy(out->bvh_lidx.get(), T.lidx.data(), T.lidx.size() * 4, hipMemcpyHostToDevice));
-        if (!T.big.empty())
-            ATX_HIP(hipMemcpy(out->bvh_big.get(), T.big.data(), T.big.size() * 4, hipMemcpyHostToDevice));
-        out->bvh = bvh_dev_from(T, out->bvh_nodes.get(), out->bvh_lsph.get(), out->bvh_lidx.get(),
-                                out->bvh_big.get());
+        const auto put = [](DevBuf& b, const void* src, size_t bytes) -> hipError_t {
+            const hipError_t e = b.reserve(bytes + 16);
+            return e != hipSuccess || bytes == 0 ? e : hipMemcpy(b.get(), src, bytes, hipMemcpyHostToDevice);
+        };
+        ATX_HIP(put(out->bvh_nodes, T.nodes.data(), T.nodes.size() * 4));
+        ATX_HIP(put(out->bvh_lsph, T.lsph.data(), T.lsph.size() * 4));
+        ATX_HIP(put(out->bvh_lidx, T.lidx.data(), T.lidx.size() * 4));
+        ATX_HIP(put(out->bvh_big, T.big.data(), T.big.size() * 4));
+        ATX_HIP(put(out->tiles, T.tiles.data(), T.tiles.size() * 4));
+        ATX_HIP(put(out->tile_boxes, T.tboxes.data(), T.tboxes.size() * 4));
+        ATX_HIP(put(out->tile_sph, T.tsph.data(), T.tsph.size() * 4));
+        ATX_HIP(put(out->tile_idx, T.tidx.data(), T.tidx.size() * 4));
+        out->bvh = bvh_dev_from(T, {out->bvh_nodes.get(), out->bvh_lsph.get(), out->bvh_lidx.get(), out->bvh_big.get(),
+                                    out->tiles.get(), out->tile_boxes.get(), out->tile_sph.get(),
+                                    out->tile_idx.get()});
     }
     return ATX_OK;
 }
 
-BvhDev bvh_dev_from(const HostBvh& T, const void* nodes, const void* lsph, const void* lidx, const void* big)
+BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at)
 {
     BvhDev b{};
-    b.nodes = static_cast<const uint4*>(nodes);
-    b.lsph = static_cast<const float4*>(lsph);
-    b.lidx = static_cast<const int32_t*>(lidx);
-    b.big = static_cast<const int32_t*>(big);
+    b.nodes = static_cast<const uint4*>(at.nodes);
+    b.lsph = static_cast<const float4*>(at.lsph);
+    b.lidx = static_cast<const int32_t*>(at.lidx);
+    b.big = static_cast<const int32_t*>(at.big);
     b.n_nodes = T.n_nodes;
     b.n_big = (uint32_t)T.big.size();
     b.layout_mask = T.layouts - 1u;
@@ -137,6 +141,13 @@ BvhDev bvh_dev_from(const HostBvh& T, const void* nodes, const void* lsph, const
     b.isy = T.inv_scale[1];
     b.isz = T.inv_scale[2];
     b.ext = T.ext;
+    b.tiles = static_cast<const uint4*>(at.tiles);
+    b.tboxes = static_cast<const float4*>(at.tboxes);
+    b.tsph = static_cast<const float4*>(at.tsph);
+    b.tidx = static_cast<const int32_t*>(at.tidx);
+    b.n_tiles = T.n_tiles;
+    b.ts = T.ts;
+    b.t_lin = T.t_lin;
     return b;
 }
 

@@ -175,18 +175,20 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 // sphere BVH (bvh.h; bvh.n_nodes = 0 when the scene has no tree).
 struct DevScene {
     DevBuf sph, sph_mat, mat, light;
-    DevBuf bvh_nodes, bvh_lsph, bvh_lidx, bvh_big;
+    DevBuf bvh_nodes, bvh_lsph, bvh_lidx, bvh_big, tiles, tile_boxes, tile_sph, tile_idx;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
     BvhDev bvh{};
     void use_pool(DevPool* pool)
     {
-        for (DevBuf* b : {&sph, &sph_mat, &mat, &light, &bvh_nodes, &bvh_lsph, &bvh_lidx, &bvh_big})
+        for (DevBuf* b : {&sph, &sph_mat, &mat, &light, &bvh_nodes, &bvh_lsph, &bvh_lidx, &bvh_big, &tiles, &tile_boxes, &tile_sph,
+                          &tile_idx})
             b->use_pool(pool);
     }
     size_t bytes() const
     {
         return sph.bytes() + sph_mat.bytes() + mat.bytes() + light.bytes() + bvh_nodes.bytes() +
-               bvh_lsph.bytes() + bvh_lidx.bytes() + bvh_big.bytes();
+               bvh_lsph.bytes() + bvh_lidx.bytes() + bvh_big.bytes() + tiles.bytes() + tile_boxes.bytes() +
+               tile_sph.bytes() + tile_idx.bytes();
     }
     // The tree to hand to a kernel: the scene's, or none for the flat loop.
     BvhDev accel(int mode) const
@@ -202,8 +204,11 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
                  const atx_light* lights, uint64_t l, DevScene* out);
 
 // Kernel view of a host-built tree whose arrays were copied to the given
-// device addresses (HostBvh::nodes, lsph, lidx and big, in that order).
-BvhDev bvh_dev_from(const HostBvh& T, const void* nodes, const void* lsph, const void* lidx, const void* big);
+// device addresses.
+struct BvhArrays {
+    const void *nodes, *lsph, *lidx, *big, *tiles, *tboxes, *tsph, *tidx;
+};
+BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at);
 
 // Device bytes a scene of this size occupies (geometry and tree).
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l);

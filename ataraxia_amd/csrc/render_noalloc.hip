@@ -132,7 +132,8 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     a.sc.n_mat = (uint32_t)num_materials;
     a.sc.n_light = (uint32_t)num_lights;
     if (T.n_nodes > 0)
-        a.sc.bvh = bvh_dev_from(T, base + off_nodes, base + off_lsph, base + off_lidx, base + off_big);
+        a.sc.bvh = bvh_dev_from(T, {base + off_nodes, base + off_lsph, base + off_lidx, base + off_big, nullptr, nullptr,
+                                    nullptr, nullptr});
     camera_inverse_matrices(cam->position, cam->direction, cam->fov_deg, cam->near_clip, cam->far_clip,
                             cam->width, cam->height, a.cam.inv_proj, a.cam.inv_view);
     memcpy(a.cam.pos, cam->position, sizeof(a.cam.pos));

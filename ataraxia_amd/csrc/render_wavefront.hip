@@ -37,20 +37,20 @@
 // path at once.  With the cache's hit list, jobs cover only the pixels
 // whose primary ray hits; k_accumulate adds the others' constant sample.
 //
-// Spheres and the scene table
-// are read with wave-uniform addresses through the constant address space,
-// which the compiler lowers to scalar loads (two spheres per s_load_dwordx8,
-// used directly as VALU operands).  A wave works on one scene at a time and
-// drains its lanes before it switches.
+// Rays of scenes with a tree are traced by whole waves (trace_tiles.h): all 64
+// lanes go through a query together, those without a ray as well.  In scenes
+// without one every ray tests every sphere.  Spheres, boxes and the scene
+// table are read with wave-uniform addresses through the constant address
+// space, which the compiler lowers to scalar loads.  A wave works on one scene
+// at a time and drains its lanes before it switches.
 //
-// Registers: the kernel is compiled twice, for 6 and for 7 resident waves
-// per SIMD (amdgpu_waves_per_eu: at most 80 and 72 VGPRs; the second
-// spills a few to scratch).  More waves hide more latency than the spills cost: launches that
-// traverse trees take the 6-wave instance, launches whose scenes all use the
-// flat loop the 7-wave one (the natural allocation, 93 VGPRs, allows 5).
+// Registers: launches whose scenes all use the flat loop have an instance for
+// each of 5 to 8 resident waves per SIMD (amdgpu_waves_per_eu; 7 by default),
+// launches with trees one for 5 (kWfWavesTree).
 #include "device_types.h"
 #include "trace_bvh.h"
 #include "trace_device.h"
+#include "trace_tiles.h"
 #include "wavefront.h"
 
 #include <stdlib.h>
@@ -228,21 +228,23 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
     }
 }
 
-template <uint32_t kWaves>
+template <uint32_t kWaves, bool kTree>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long lanes_below = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
     const uint32_t P = a.chunk_px;
-    // The instances for 7 and 8 resident waves per SIMD park the path state
-    // that a trace does not read (17 values per lane) in LDS while the trace
-    // runs: the state then needs no VGPRs there, and the trace fits the
-    // smaller register budget without spilling (17 KB of LDS per
-    // 256-lane workgroup, 136 KB per CU at 8 waves per SIMD).
-    constexpr bool kPark = kWaves >= 7;
+    // The instances for trees and for 7 and 8 resident waves per SIMD park the
+    // path state that a trace does not read (17 values per lane) in LDS while
+    // the trace runs: the state then needs no VGPRs there, and the trace fits
+    // its register budget without spilling (17 KB of LDS per 256-lane
+    // workgroup, 136 KB per CU at 8 waves per SIMD; a tile query's candidate
+    // masks take another 9 KB).
+    constexpr bool kPark = kWaves >= 7 || kTree;
     constexpr uint32_t kParked = 17;
     __shared__ uint32_t parked_all[4][kPark ? kParked : 1][64];
     uint32_t(*parked)[64] = parked_all[threadIdx.x >> 6];
+    __shared__ uint32_t tile_masks[4][kTree ? kTileRows : 1][64];
 
     // ---- wave-uniform scheduling state ----
     CScene* scenes = as_const(a.scenes);
@@ -447,10 +449,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         bool end_path = state == kCont && S->max_bounces <= 0;   // zero bounces: black sample
         const bool traces = tracing && !end_path;
         rays += (unsigned long long)__popcll(__ballot(traces));
-        if (traces) {
-            const bool shadow = state == kShadow;
-            const SphSrc flat{as_const(S->sph)};
-            Hit h;
+        const bool shadow = state == kShadow;
+        Hit h;
+        const bool tree = kTree && S && S->bvh.n_tiles != 0u;
+        const auto query = [&]() {
             if constexpr (kPark) {
                 const uint32_t v[kParked] = {__float_as_uint(col.x), __float_as_uint(col.y), __float_as_uint(col.z),
                                              __float_as_uint(tp.x),  __float_as_uint(tp.y),  __float_as_uint(tp.z),
@@ -462,23 +464,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 // keep the compiler from forwarding the stored values past the trace
                 __asm__ volatile("" ::: "memory");
             }
-            uint32_t dt = 0, db = 0;   // the trace's sphere and box tests
-            if (S->bvh.n_nodes) {
-                // the debug capture records the closest occluder; otherwise any proven one will do
+            const SphSrc flat{as_const(S->sph)};
+            // the debug capture records the closest occluder; otherwise any proven one will do
+            const float qd2 = (shadow && !(capture && S->dbg_shadow)) ? dist2 : -1.0f;
+            BvhQuery q;
+            if (tree) {
                 const BvhDev B = S->bvh;
-                BvhQuery q;
-                const float qd2 = (shadow && !(capture && S->dbg_shadow)) ? dist2 : -1.0f;
-                h = trace_bvh<true>(B, flat, S->n_sph, ro, rd, qd2, q);
-                if (q.exact)
-                    atomicAdd(a.counters + kCtrExact, (unsigned long long)q.exact);
-                dt = q.tests;
-                db = q.boxes;
+                h = trace_tiles(B, flat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
             } else {
-                uint32_t ex = 0;
-                h = trace_filtered(flat, S->n_sph, ro, rd, ex);
-                if (ex)
-                    atomicAdd(a.counters + kCtrExact, (unsigned long long)ex);
-                dt = S->n_sph;
+                h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
+                q.tests = S->n_sph;
             }
             if constexpr (kPark) {
                 __asm__ volatile("" ::: "memory");
@@ -497,9 +492,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 mid = (int32_t)parked[15][lane];
                 lidx = parked[16][lane];
             }
-            tests += dt;
-            boxes += db;
+            if (traces) {
+                if (q.exact)
+                    atomicAdd(a.counters + kCtrExact, (unsigned long long)q.exact);
+                tests += q.tests;
+                boxes += q.boxes;
+            }
+        };
 
+        const auto shade = [&]() {
             // ---------------- shading (divergent) ----------------
             if (!shadow) {
                 if (capture && S->dbg_hit && (uint32_t)bounce < S->dbg_bounces)
@@ -526,6 +527,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                     add_light(S, mid, lidx, nrm, vd, rd, tp, col);
                 end_bounce = true;
             }
+        };
+        if constexpr (kTree) {
+            if (tree || traces)   // every lane takes part in a tile query's matrix products
+                query();
+            if (traces)
+                shade();
+        } else if (traces) {
+            query();
+            shade();
         }
         if (end_bounce) {
             // the next ray leaves from the hit's offset origin, which ro holds
@@ -683,68 +693,82 @@ __global__ __launch_bounds__(256) void k_first_hit(FirstArgs a)
     const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
     const uint32_t ty = wave / tiles_x, tx = wave - ty * tiles_x;
     const uint32_t x = tx * 8u + (threadIdx.x & 7u), y = ty * 8u + ((threadIdx.x >> 3) & 7u);
-    if (x >= s.width || y >= s.height)
-        return;
-    const uint32_t px = y * s.width + x;
+    // lanes past the image's edge stay for the wave's tile queries
+    const bool in = x < s.width && y < s.height;
+    const uint32_t px = in ? y * s.width + x : 0u;
     const f3 ro = mk(s.cam_pos[0], s.cam_pos[1], s.cam_pos[2]);
     const float4 dv = s.dirs[px];
     const f3 rd = mk(dv.x, dv.y, dv.z);
     const SphSrc flat{as_const(s.sph)};
-    auto trace = [&](f3 o, f3 d, float d2) -> Hit {
-        if (s.bvh.n_nodes) {
-            BvhQuery q;
-            return trace_bvh(s.bvh, flat, s.n_sph, o, d, d2, q);
-        }
-        uint32_t ex = 0;
-        return trace_filtered(flat, s.n_sph, o, d, ex);
-    };
-    const Hit h = trace(ro, rd, -1.0f);
-    uint32_t slot = 0u;   // index in the hit list
-    {
-        // append this wave's hit pixels to the list (one atomic per wave)
-        const uint32_t lane = threadIdx.x & 63u;
-        const unsigned long long act = __ballot(1);
-        const unsigned long long hm = __ballot(h.id >= 0);
-        const uint32_t leader = (uint32_t)__ffsll((long long)act) - 1u;
-        uint32_t base = 0;
-        if (lane == leader && hm)
-            base = atomicAdd(a.n_hits, (uint32_t)__popcll(hm));
-        base = (uint32_t)__shfl((int)base, (int)leader, 64);
-        if (h.id >= 0) {
-            const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
-            slot = base + (uint32_t)__popcll(hm & below);
-            a.hits[slot] = px;
-        }
-    }
+    __shared__ uint32_t tile_masks[4][kTileRows][64];
+    const BvhDev B = s.bvh;
     const f3 one = mk(1.0f, 1.0f, 1.0f);
     const f3 zero = mk(0.0f, 0.0f, 0.0f);
-    f3 nrm = zero, so = zero, col = zero;
+    f3 pos = zero, nrm = zero, so = zero, col = zero;
+    Hit first;   // the primary hit
+    first.id = -1;
+    first.t = FLT_MAX;
     int32_t mid = 0;
     uint32_t mask = 0u;
-    if (h.id >= 0) {
-        f3 pos;
-        hit_frame(as_const(s.sph)[h.id], h, ro, rd, pos, nrm, so);
-        mid = s.sph_mat[h.id];
-        add_emission(s.mat, mid, one, col);
-        if (a.light) {
-            for (uint32_t l = 0; l < s.n_light; ++l) {
-                f3 L;
-                float dist2;
-                light_ray(s.light[2 * l], pos, L, dist2);
-                f3 term = zero;
-                if (lit_by(trace(so, L, dist2), dist2)) {
-                    mask |= 1u << l;
-                    term = light_term(s.mat, s.light, mid, l, nrm, rd, L, one);
-                }
-                a.light[(size_t)l * npx + px] = make_float4(term.x, term.y, term.z, 0.0f);
-            }
+    uint32_t slot = 0u;   // index in the hit list
+    // the primary ray, then a shadow ray towards each light (one query in the
+    // code: a second copy of it would take the registers of both)
+    const uint32_t n_rays = 1u + (a.light ? s.n_light : 0u);
+    for (uint32_t k = 0; k < n_rays; ++k) {
+        const bool hit = first.id >= 0, act = k == 0u ? in : hit;
+        f3 o = ro, d = rd;
+        float dist2 = -1.0f;
+        if (k > 0u) {
+            o = so;
+            d = one;
+            if (hit)
+                light_ray(s.light[2 * (k - 1u)], pos, d, dist2);
         }
-    } else if (a.light) {
-        for (uint32_t l = 0; l < s.n_light; ++l)
-            a.light[(size_t)l * npx + px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        Hit h;
+        h.id = -1;
+        h.t = FLT_MAX;
+        if (!__any(act)) {
+            // a wave of missing pixels has no shadow rays
+        } else if (B.n_tiles) {
+            BvhQuery q;
+            h = trace_tiles(B, flat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
+        } else {
+            uint32_t ex = 0;
+            h = trace_filtered(flat, s.n_sph, o, d, ex);
+        }
+        if (k == 0u) {
+            first = h;
+            if (!in)
+                first.id = -1;
+            // append this wave's hit pixels to the list (one atomic per wave)
+            const uint32_t lane = threadIdx.x & 63u;
+            const unsigned long long hm = __ballot(first.id >= 0);
+            uint32_t base = 0;
+            if (lane == 0 && hm)
+                base = atomicAdd(a.n_hits, (uint32_t)__popcll(hm));
+            base = (uint32_t)__shfl((int)base, 0, 64);
+            if (first.id >= 0) {
+                const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
+                slot = base + (uint32_t)__popcll(hm & below);
+                a.hits[slot] = px;
+                hit_frame(as_const(s.sph)[first.id], first, ro, rd, pos, nrm, so);
+                mid = s.sph_mat[first.id];
+                add_emission(s.mat, mid, one, col);
+            }
+        } else if (in) {
+            const uint32_t l = k - 1u;
+            f3 term = zero;
+            if (hit && lit_by(h, dist2)) {
+                mask |= 1u << l;
+                term = light_term(s.mat, s.light, mid, l, nrm, rd, d, one);
+            }
+            a.light[(size_t)l * npx + px] = make_float4(term.x, term.y, term.z, 0.0f);
+        }
     }
+    if (!in)
+        return;
     uint4* r = a.rec + 4 * (size_t)px;
-    r[0] = make_uint4((uint32_t)h.id, __float_as_uint(h.t), mask, (uint32_t)mid);
+    r[0] = make_uint4((uint32_t)first.id, __float_as_uint(first.t), mask, (uint32_t)mid);
     r[1] = make_uint4(__float_as_uint(nrm.x), __float_as_uint(nrm.y), __float_as_uint(nrm.z), __float_as_uint(so.x));
     r[2] = make_uint4(__float_as_uint(so.y), __float_as_uint(so.z), __float_as_uint(col.x), __float_as_uint(col.y));
     r[3] = make_uint4(__float_as_uint(col.z), slot, 0u, 0u);
@@ -754,6 +778,20 @@ __global__ void k_zero_u32(unsigned int* p, uint32_t n)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0u;
+}
+
+// The path kernel's instance for a launch (wf_waves).
+using PathKernel = void (*)(WfPass);
+PathKernel path_kernel(bool flat_only, uint32_t waves)
+{
+    if (!flat_only)
+        return k_render_wavefront<kWfWavesTree, true>;
+    switch (wf_waves(waves, flat_only)) {
+    case 5: return k_render_wavefront<5, false>;
+    case 6: return k_render_wavefront<6, false>;
+    case 7: return k_render_wavefront<7, false>;
+    default: return k_render_wavefront<8, false>;
+    }
 }
 
 }  // namespace
@@ -773,12 +811,7 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
         return hipErrorInvalidValue;
     // no jobs (every pixel's primary ray misses): k_accumulate alone
     if (p.total_chunks > 0) {
-        switch (wf_waves(l.waves, l.flat_only)) {
-        case 5: hipLaunchKernelGGL(k_render_wavefront<5>, dim3(l.workgroups), dim3(256), 0, stream, p); break;
-        case 6: hipLaunchKernelGGL(k_render_wavefront<6>, dim3(l.workgroups), dim3(256), 0, stream, p); break;
-        case 7: hipLaunchKernelGGL(k_render_wavefront<7>, dim3(l.workgroups), dim3(256), 0, stream, p); break;
-        default: hipLaunchKernelGGL(k_render_wavefront<8>, dim3(l.workgroups), dim3(256), 0, stream, p); break;
-        }
+        hipLaunchKernelGGL(path_kernel(l.flat_only, l.waves), dim3(l.workgroups), dim3(256), 0, stream, p);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && paths_done)
@@ -838,13 +871,8 @@ hipError_t launch_zero_u32(unsigned int* p, uint32_t n, hipStream_t stream)
 int wavefront_max_blocks_per_cu(bool flat_only, uint32_t waves)
 {
     int blocks = 0;
-    hipError_t e;
-    switch (wf_waves(waves, flat_only)) {
-    case 5: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_render_wavefront<5>, 256, 0); break;
-    case 6: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_render_wavefront<6>, 256, 0); break;
-    case 7: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_render_wavefront<7>, 256, 0); break;
-    default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_render_wavefront<8>, 256, 0); break;
-    }
+    const hipError_t e =
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, path_kernel(flat_only, waves), 256, 0);
     if (e != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;

@@ -124,7 +124,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     std::vector<uint32_t> launch_frames, launch_chunk;
     const bool wf = r->kernel == ATX_KERNEL_WAVEFRONT && frames > 0;
     bool use_first = false;
-    WfLaunch shape{0, false};
+    WfLaunch shape{0};
     if (wf) {
         uint32_t fi = r->frame_index, left = frames;
         const uint32_t fit = (uint32_t)std::max<size_t>(1, kSampleBufferBytes / (npx * kSampleBytes));
@@ -148,11 +148,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         for (const WfScene& e : table) most = std::max(most, launch_samples(&e, 1));
         ATX_HIP(r->wf_samples.reserve(most * kSampleBytes));
         shape.flat_only = wf_flat_only(table.data(), table.size());
-        // the instance: the caller's, else by the jobs of the largest launch
-        // (every pixel in every frame, an upper bound of the hit list's)
-        shape.waves = r->wf_waves ? r->wf_waves
-                      : shape.flat_only ? 0u
-                                        : wf_tree_waves((uint64_t)npx * launch_frames[0]);
+        shape.waves = r->wf_waves;
         shape.workgroups = wavefront_full_grid(shape.flat_only, shape.waves);
         // The first-bounce cache pays from two frames per camera on: a call
         // of one frame uses it once the camera has stayed the same since the

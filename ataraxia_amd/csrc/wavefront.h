@@ -173,29 +173,22 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
     return g * kJobGroupPx * frames + f * m + (k - g * kJobGroupPx);
 }
 
-// Resident waves per SIMD the path kernel's registers are budgeted for:
-// launches with trees, and launches whose scenes all use the flat loop.
-constexpr uint32_t kWfWavesTree = 6;
+// Resident waves per SIMD the path kernel's registers are budgeted for.
+// Launches whose scenes all use the flat loop have an instance for each of 5
+// to 8 (the batch autotuner tries them all).  Launches with trees have one,
+// for 5: a tile query holds 16 sums, 24 operands and its ray, which takes 96
+// VGPRs; the same kernel budgeted for 6 waves (80 VGPRs) spills 19 of them
+// (1080p, 256 frames: 22.5 ms of path kernel with 5, 24.7 with 6).
+constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
-
-// Register budgets the path kernel is compiled for (resident waves per
-// SIMD); a launch picks one (the batch autotuner tries them all).
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
-// Launches with trees of at least this many jobs take the 8-wave instance,
-// which parks the path state in LDS during traces (1080p workload, 1.37 M
-// jobs per frame, path kernel against 6 waves: 4 frames 4.5 % slower, 8
-// frames even, 12 / 16 / 20 frames 0.7 / 6.3 / 8.2 % faster, 256 frames 6.8 %
-// faster).
-constexpr uint64_t kWfWaves8MinJobs = uint64_t(12) << 20;
-__host__ __device__ __forceinline__ uint32_t wf_tree_waves(uint64_t jobs)
-{
-    return jobs >= kWfWaves8MinJobs ? 8u : kWfWavesTree;
-}
 // The instance a launch uses: `waves` when it names a compiled instance,
 // else the default for its scenes.
 __host__ __device__ __forceinline__ uint32_t wf_waves(uint32_t waves, bool flat_only)
 {
-    return waves >= kWfWavesMin && waves <= kWfWavesMax ? waves : (flat_only ? kWfWavesFlat : kWfWavesTree);
+    if (!flat_only)
+        return kWfWavesTree;
+    return waves >= kWfWavesMin && waves <= kWfWavesMax ? waves : kWfWavesFlat;
 }
 
 struct WfLaunch {
