@@ -47,6 +47,7 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
         out->sph_mat[i] = id;
     }
     out->mat.resize(12 * m);
+    out->mat_rr.resize(4 * m);
     for (uint64_t i = 0; i < m; ++i) {
         const atx_material& a = materials[i];
         float* o = &out->mat[12 * i];
@@ -54,6 +55,11 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
         o[4] = a.F0[0]; o[5] = a.F0[1]; o[6] = a.F0[2]; o[7] = a.metallic;
         o[8] = a.emission_color[0]; o[9] = a.emission_color[1]; o[10] = a.emission_color[2];
         o[11] = a.emission_intensity;
+        const f3 albedo = mk(a.albedo[0], a.albedo[1], a.albedo[2]);
+        const float p = gmax(0.1f, gmin(1.0f, length(albedo)));
+        const f3 tp = divs(albedo, p);
+        float* r = &out->mat_rr[4 * i];
+        r[0] = tp.x; r[1] = tp.y; r[2] = tp.z; r[3] = p;
     }
     out->light.resize(8 * l);
     for (uint64_t i = 0; i < l; ++i) {
@@ -67,7 +73,7 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l)
 {
-    return (16 * n + 16) + (4 * n + 16) + (48 * m + 16) + (32 * l + 16) + bvh_device_bytes(n);
+    return (16 * n + 16) + (4 * n + 16) + (48 * m + 16) + (16 * m + 16) + (32 * l + 16) + bvh_device_bytes(n);
 }
 
 int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
@@ -79,11 +85,14 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     ATX_HIP(out->sph.reserve(L.sph.size() * 4 + 16));
     ATX_HIP(out->sph_mat.reserve(L.sph_mat.size() * 4 + 16));
     ATX_HIP(out->mat.reserve(L.mat.size() * 4 + 16));
+    ATX_HIP(out->mat_rr.reserve(L.mat_rr.size() * 4 + 16));
     ATX_HIP(out->light.reserve(L.light.size() * 4 + 16));
     if (!L.sph.empty()) ATX_HIP(hipMemcpy(out->sph.get(), L.sph.data(), L.sph.size() * 4, hipMemcpyHostToDevice));
     if (!L.sph_mat.empty())
         ATX_HIP(hipMemcpy(out->sph_mat.get(), L.sph_mat.data(), L.sph_mat.size() * 4, hipMemcpyHostToDevice));
     if (!L.mat.empty()) ATX_HIP(hipMemcpy(out->mat.get(), L.mat.data(), L.mat.size() * 4, hipMemcpyHostToDevice));
+    if (!L.mat_rr.empty())
+        ATX_HIP(hipMemcpy(out->mat_rr.get(), L.mat_rr.data(), L.mat_rr.size() * 4, hipMemcpyHostToDevice));
     if (!L.light.empty())
         ATX_HIP(hipMemcpy(out->light.get(), L.light.data(), L.light.size() * 4, hipMemcpyHostToDevice));
     out->n_sph = (uint32_t)n;

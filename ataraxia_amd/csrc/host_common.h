@@ -162,6 +162,7 @@ struct HostSceneLayout {
     std::vector<float> sph;       // 4 per sphere: cx, cy, cz, r*r
     std::vector<int32_t> sph_mat; // material index per sphere (clamped)
     std::vector<float> mat;       // 12 per material
+    std::vector<float> mat_rr;    // 4 per material: albedo / p, p (see WfScene::mat_rr)
     std::vector<float> light;     // 8 per light
 };
 
@@ -174,19 +175,19 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 // One scene's geometry in HBM (device layout of device_types.h), with its
 // sphere BVH (bvh.h; bvh.n_nodes = 0 when the scene has no tree).
 struct DevScene {
-    DevBuf sph, sph_mat, mat, light;
+    DevBuf sph, sph_mat, mat, mat_rr, light;
     DevBuf bvh_nodes, bvh_lsph, bvh_lidx, bvh_big, tiles, tile_boxes, tile_sph, tile_idx;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
     BvhDev bvh{};
     void use_pool(DevPool* pool)
     {
-        for (DevBuf* b : {&sph, &sph_mat, &mat, &light, &bvh_nodes, &bvh_lsph, &bvh_lidx, &bvh_big, &tiles, &tile_boxes, &tile_sph,
+        for (DevBuf* b : {&sph, &sph_mat, &mat, &mat_rr, &light, &bvh_nodes, &bvh_lsph, &bvh_lidx, &bvh_big, &tiles, &tile_boxes, &tile_sph,
                           &tile_idx})
             b->use_pool(pool);
     }
     size_t bytes() const
     {
-        return sph.bytes() + sph_mat.bytes() + mat.bytes() + light.bytes() + bvh_nodes.bytes() +
+        return sph.bytes() + sph_mat.bytes() + mat.bytes() + mat_rr.bytes() + light.bytes() + bvh_nodes.bytes() +
                bvh_lsph.bytes() + bvh_lidx.bytes() + bvh_big.bytes() + tiles.bytes() + tile_boxes.bytes() +
                tile_sph.bytes() + tile_idx.bytes();
     }

@@ -58,7 +58,7 @@
 namespace atx {
 namespace {
 
-constexpr uint32_t kIdle = 0, kCont = 1, kShadow = 2;
+constexpr uint32_t kIdle = 0, kCont = 1, kShadow = 2, kNew = 3;
 
 // The scene table and the sphere arrays do not change during a launch; read
 // through the constant address space, wave-uniform loads from them become
@@ -185,25 +185,35 @@ __device__ __forceinline__ void add_light(CScene* S, int32_t mid, uint32_t lidx,
     col = add(col, light_term(S->mat, S->light, mid, lidx, nrm, rd, L, tp));
 }
 
-// Russian roulette and the next direction (Renderer.cu:362-381).  Returns
-// true when the path ends here.
-__device__ __forceinline__ bool next_bounce(CScene* S, int32_t mid, f3 nrm, f3 so, f3& tp, f3& ro, f3& rd,
-                                            int32_t& bounce, uint32_t& seed)
+// Throughput and Russian roulette at the end of a bounce (Renderer.cu:362-379).
+// Returns true when the path ends here, by the draw or at its last bounce.
+__device__ __forceinline__ bool roulette(CScene* S, int32_t mid, f3& tp, int32_t bounce, uint32_t& seed)
 {
-    const float4 m0 = S->mat[3 * mid + 0];
-    const float4 m1 = S->mat[3 * mid + 1];
-    tp = mul(tp, xyz(m0));
-    ro = so;
+    tp = mul(tp, xyz(S->mat[3 * mid]));
     const float p = gmax(0.1f, gmin(1.0f, length(tp)));
     if (pcg_float(seed) > p)
         return true;
     tp = divs(tp, p);
-    rd = sample_next(nrm, m1.w > 0.0f, m0.w, seed);
+    return bounce + 1 >= S->max_bounces;
+}
+
+// The same at bounce 0, where the throughput is 1: the scene holds p and
+// albedo / p per material (mat_rr), which saves a square root and three
+// divisions in every path.
+__device__ __forceinline__ bool roulette_first(CScene* S, int32_t mid, f3& tp, uint32_t& seed)
+{
+    const float4 rr = S->mat_rr[mid];
+    tp = xyz(rr);
+    return pcg_float(seed) > rr.w || S->max_bounces <= 1;
+}
+
+// The next direction of a path that goes on (Renderer.cu:381-384).
+__device__ __forceinline__ void next_direction(CScene* S, int32_t mid, f3 nrm, f3& rd, int32_t& bounce,
+                                               uint32_t& seed)
+{
+    rd = sample_next(nrm, S->mat[3 * mid + 1].w > 0.0f, S->mat[3 * mid].w, seed);
     ++bounce;
-    if (bounce >= S->max_bounces)
-        return true;
     seed += (uint32_t)bounce;
-    return false;
 }
 
 // The pixel of the scene's job `job` (`slots` jobs per frame): the path
@@ -370,7 +380,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                             state = kShadow;
                         } else {
                             nrm = mk(__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z));
-                            const f3 so = mk(__uint_as_float(r1.w), __uint_as_float(r2.x), __uint_as_float(r2.y));
+                            ro = mk(__uint_as_float(r1.w), __uint_as_float(r2.x), __uint_as_float(r2.y));
                             col = mk(__uint_as_float(r2.z), __uint_as_float(r2.w), __uint_as_float(r3.x));
                             mid = (int32_t)r0.w;
                             if (nl > 0u) {
@@ -380,7 +390,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                                 if ((r0.z >> lidx) & 1u)
                                     col = add(col, xyz(lt));
                             }
-                            done = next_bounce(S, mid, nrm, so, tp, ro, rd, bounce, seed);
+                            done = roulette_first(S, mid, tp, seed);
+                            state = kNew;
                         }
                         if (done) {
                             store_sample(S, slots, job, col);
@@ -442,6 +453,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         }
         if (!__any(state != kIdle) && qdone && pend < 0)
             break;
+        // The next direction of every path that goes on: those of the last
+        // round and those just handed out together, so that its 200
+        // instructions run once per round.  Where each hand-out and each
+        // bounce's end computed its own (about 3 per round at 1080p), the path
+        // kernel issued 1890 VALU instructions per round instead of 1600
+        // (1080p, 256 frames: 22.5 -> 20.0 ms).
+        if (state == kNew) {
+            next_direction(S, mid, nrm, rd, bounce, seed);
+            state = kCont;
+        }
 
         // ---------------- one closest-hit trace for every tracing lane ----------------
         const bool tracing = state == kCont || state == kShadow;
@@ -539,10 +560,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         }
         if (end_bounce) {
             // the next ray leaves from the hit's offset origin, which ro holds
-            if (next_bounce(S, mid, nrm, ro, tp, ro, rd, bounce, seed))
+            if (roulette(S, mid, tp, bounce, seed))
                 end_path = true;
             else
-                state = kCont;
+                state = kNew;
         }
         if (__any(tests >= 0x80000000u || boxes >= 0x80000000u))
             flush_counters(a.counters, lane, tests, boxes);

@@ -65,6 +65,7 @@ struct WfScene {
     const float4* sph;
     const int32_t* sph_mat;
     const float4* mat;
+    const float4* mat_rr;  // per material: albedo / p and p, the roulette at a path's first hit
     const float4* light;
     uint32_t n_sph;
     uint32_t n_mat;
@@ -178,7 +179,7 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
 // to 8 (the batch autotuner tries them all).  Launches with trees have one,
 // for 5: a tile query holds 16 sums, 24 operands and its ray, which takes 96
 // VGPRs; the same kernel budgeted for 6 waves (80 VGPRs) spills 19 of them
-// (1080p, 256 frames: 22.5 ms of path kernel with 5, 24.7 with 6).
+// (1080p, 256 frames: 20.0 ms of path kernel with 5, 23.2 with 6).
 constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;

@@ -19,6 +19,7 @@ inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_c
     out->sph = g.sph.as<float4>();
     out->sph_mat = g.sph_mat.as<int32_t>();
     out->mat = g.mat.as<float4>();
+    out->mat_rr = g.mat_rr.as<float4>();
     out->light = g.light.as<float4>();
     out->n_sph = g.n_sph;
     out->n_mat = g.n_mat;
