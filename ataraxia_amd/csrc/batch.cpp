@@ -55,7 +55,7 @@ struct Batch {
     std::vector<uint32_t> launch_chunk_px;  // jobs per chunk of launch l
     uint32_t launches = 0, chunk_px = 0, frames_per_launch = 0, grid = 0, max_spp = 0;
     uint64_t skipped = 0;   // primary rays of pixels left out of the jobs (hit lists), per render
-    bool flat_only = false;   // no scene has a tree: the flat-loop kernel instance
+    bool flat_only = false;   // no scene has tiles: the flat-loop kernel instance
     bool kahan = false;
     DevBuf d_samples;                     // sample buffer, shared by the launches (stream order)
     std::vector<uint32_t> launch_px;
@@ -264,7 +264,7 @@ int batch_accel(const Batch* b) { return b->accel; }
 bool batch_flat_only(const Batch* b)
 {
     for (const auto& e : b->scenes)
-        if (e->geo.accel(b->accel).n_nodes != 0)
+        if (e->geo.accel(b->accel).n_tiles != 0)
             return false;
     return true;
 }

@@ -191,11 +191,15 @@ struct DevScene {
                bvh_lsph.bytes() + bvh_lidx.bytes() + bvh_big.bytes() + tiles.bytes() + tile_boxes.bytes() +
                tile_sph.bytes() + tile_idx.bytes();
     }
-    // The tree to hand to a kernel: the scene's, or none for the flat loop.
+    // The tree to hand to a kernel: the scene's, or for ATX_ACCEL_NONE its tiles
+    // without nodes and boxes, so that every ray tests every sphere.
     BvhDev accel(int mode) const
     {
-        BvhDev b{};
-        if (mode == ATX_ACCEL_BVH) b = bvh;
+        BvhDev b = bvh;
+        if (mode != ATX_ACCEL_BVH) {
+            b.n_nodes = 0;
+            b.tboxes = nullptr;
+        }
         return b;
     }
 };

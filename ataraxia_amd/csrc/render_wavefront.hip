@@ -705,6 +705,7 @@ struct FirstArgs {
 // A wave takes an 8 x 8 tile of pixels: its rays stay closer together than
 // along a 64-pixel row (1080p: 0.586 -> 0.556 ms), and the hit list then
 // runs tile by tile.
+template <bool kTree>
 __global__ __launch_bounds__(256) void k_first_hit(FirstArgs a)
 {
     const WfScene& s = a.s;
@@ -721,7 +722,7 @@ __global__ __launch_bounds__(256) void k_first_hit(FirstArgs a)
     const float4 dv = s.dirs[px];
     const f3 rd = mk(dv.x, dv.y, dv.z);
     const SphSrc flat{as_const(s.sph)};
-    __shared__ uint32_t tile_masks[4][kTileRows][64];
+    __shared__ uint32_t tile_masks[4][kTree ? kTileRows : 1][64];
     const BvhDev B = s.bvh;
     const f3 one = mk(1.0f, 1.0f, 1.0f);
     const f3 zero = mk(0.0f, 0.0f, 0.0f);
@@ -748,12 +749,11 @@ __global__ __launch_bounds__(256) void k_first_hit(FirstArgs a)
         Hit h;
         h.id = -1;
         h.t = FLT_MAX;
-        if (!__any(act)) {
-            // a wave of missing pixels has no shadow rays
-        } else if (B.n_tiles) {
+        if constexpr (kTree) {
             BvhQuery q;
-            h = trace_tiles(B, flat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
-        } else {
+            if (__any(act))   // a wave of missing pixels has no shadow rays
+                h = trace_tiles(B, flat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
+        } else if (act) {
             uint32_t ex = 0;
             h = trace_filtered(flat, s.n_sph, o, d, ex);
         }
@@ -877,7 +877,8 @@ hipError_t launch_first_hits(const WfScene& s, hipStream_t stream)
     a.n_hits = v.n_hits;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, v.n_hits, 1u);
     const uint32_t tiles = ((s.width + 7u) / 8u) * ((s.height + 7u) / 8u);
-    hipLaunchKernelGGL(k_first_hit, dim3((tiles + 3u) / 4u), dim3(256), 0, stream, a);
+    const auto kernel = s.bvh.n_tiles ? k_first_hit<true> : k_first_hit<false>;
+    hipLaunchKernelGGL(kernel, dim3((tiles + 3u) / 4u), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

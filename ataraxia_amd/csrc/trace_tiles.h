@@ -38,7 +38,8 @@
 // error above allows (it is at most q / (2 r) and at most sqrt(q); r <= 8
 // here, and t_lin = 2^-18 / smallest radius, rounded up), and by 2^-18 (n + 16)
 // for the slab test's own rounding.  Tiles of more than kTileFlat tiles come in groups of eight with
-// a box of their own.  Distances are culled as in the tree.
+// a box of their own.  Distances are culled as in the tree.  Without boxes
+// (tboxes null: ATX_ACCEL_NONE) the product tests every sphere.
 //
 // What bounds it: VALU issue (0.31 instructions per cycle and SIMD in the path
 // kernel; minima, compares and shifts run at half the rate of multiply-adds),
@@ -51,7 +52,9 @@
 // flat loop over all spheres for a ray with an ambiguous pair), whole calls:
 // 1920x1080, 257 spheres, 20 frames 4.70 -> 3.40 ms, 256 frames 36.1 -> 25.5;
 // 1024x1024, 513 spheres, 64 frames 8.48 -> 6.08; 1600x900, 8001 spheres, 32
-// frames 31.1 -> 10.2 (k_first_hit alone 16.1 -> 1.25).
+// frames 31.1 -> 10.2 (k_first_hit alone 16.1 -> 1.25).  Testing every sphere by
+// the product instead of a loop of scalar loads: 853x481, 97 spheres, 8 frames
+// 1.33 -> 1.13 ms.
 #pragma once
 
 #include "bvh.h"
@@ -171,7 +174,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
         const int32_t id = B.big[j];
         tile_candidate(B, flat, flat((uint32_t)id), id, o, d, a, f, q);
     }
-    q.tests += B.n_big;
+    q.tests += B.tboxes ? B.n_big : n_all;   // without boxes every sphere is tested
 
     // the ray in tile units and its line's closest point to their origin
     const float ox = (o.x - B.cx) * B.ts, oy = (o.y - B.cy) * B.ts, oz = (o.z - B.cz) * B.ts;
@@ -243,13 +246,13 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
     const ATX_GLOBAL uint4* tiles = (const ATX_GLOBAL uint4*)(uintptr_t)B.tiles + lane;
     const ATX_GLOBAL float4* tsph = (const ATX_GLOBAL float4*)(uintptr_t)B.tsph;
     const uint32_t n_tiles = B.n_tiles;
-    const bool groups = n_tiles > kTileFlat;
+    const bool boxed = B.tboxes != nullptr, groups = n_tiles > kTileFlat;
     for (uint32_t t = 0; t < n_tiles;) {
         // candidates of up to kTileChunk touched tiles
         uint32_t nm = 0u, some = 0u;
         const float lim = act ? tlim * B.ts : -1.0f;   // a lane that does not act touches nothing
         for (;;) {
-            if (groups && !__any(touches(n_tiles + t / 8u, lim))) {
+            if (groups && boxed && !__any(touches(n_tiles + t / 8u, lim))) {
                 t += 8u;
                 if (t >= n_tiles)
                     break;
@@ -258,15 +261,20 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
             // which of the next eight tiles this lane's ray touches
             const uint32_t nt = n_tiles - t < 8u ? n_tiles - t : 8u;
             uint32_t touched = 0u, need = 0u;
+            if (boxed) {
 #pragma unroll
-            for (uint32_t k = 0; k < 8u; ++k) {
-                if (k < nt) {
-                    const bool touch = touches(t + k, lim);
-                    touched |= touch ? 1u << k : 0u;
-                    need |= __any(touch) ? 1u << k : 0u;
+                for (uint32_t k = 0; k < 8u; ++k) {
+                    if (k < nt) {
+                        const bool touch = touches(t + k, lim);
+                        touched |= touch ? 1u << k : 0u;
+                        need |= __any(touch) ? 1u << k : 0u;
+                    }
                 }
+                q.boxes += nt;
+            } else {
+                touched = act ? (1u << nt) - 1u : 0u;
+                need = __any(act) ? (1u << nt) - 1u : 0u;
             }
-            q.boxes += nt;
             if (nm + (uint32_t)__popc(need) > kTileChunk)
                 break;   // no room: test the candidates so far, then come back
             while (need != 0u) {
@@ -302,7 +310,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
             }
             const uint32_t k = base + (uint32_t)__builtin_ctz(m);
             m &= m - 1u;
-            ++q.tests;
+            q.tests += boxed ? 1u : 0u;
             if (tile_candidate(B, flat, tsph[k], kLeafSlot | (int32_t)k, o, d, a, f, q))
                 tlim = bvh_min_raw(tlim, f.best_hi * inv_a_up);
             // t of the best sphere <= tlim, and tlim*tlim < dist2 proves it occludes

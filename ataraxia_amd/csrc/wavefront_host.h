@@ -147,11 +147,11 @@ inline uint32_t wavefront_full_grid(bool flat_only, uint32_t waves = 0)
     return device_cus() * (uint32_t)wavefront_max_blocks_per_cu(flat_only, waves);
 }
 
-// True when no scene of the table has a tree (the flat-loop kernel instance).
+// True when no scene of the table has a tree or tiles (the flat-loop instances)
 inline bool wf_flat_only(const WfScene* tab, size_t n)
 {
     for (size_t k = 0; k < n; ++k)
-        if (tab[k].bvh.n_nodes != 0)
+        if (tab[k].bvh.n_nodes != 0 || tab[k].bvh.n_tiles != 0)
             return false;
     return true;
 }

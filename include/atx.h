@@ -102,8 +102,8 @@ ATX_STATIC_ASSERT(sizeof(atx_camera) == 44 && offsetof(atx_camera, fov_deg) == 2
 /* Which spheres a ray tests (Renderer.cu:251-285 tests all of them).  BVH
  * (the default) walks a bounding-volume hierarchy built at scene upload and
  * gives the same closest hit, bit for bit, including the lowest index among
- * equal distances; NONE is the flat loop over every sphere.  Scenes with
- * fewer than 16 spheres always use the flat loop.                           */
+ * equal distances; NONE tests every sphere.  Scenes with fewer than 16
+ * spheres always use the flat loop.                                         */
 #define ATX_ACCEL_BVH 0
 #define ATX_ACCEL_NONE 1
 
