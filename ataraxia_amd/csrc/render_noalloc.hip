@@ -1,13 +1,14 @@
 // render_noalloc.hip -- the allocation-free render entry point.
 //
-// atx_render_frames_noalloc renders frames of one scene with the plain kernel
-// (render_plain.hip) exactly as atx_renderer_render_frames does with
-// ATX_KERNEL_PLAIN, but allocates no device memory: the caller passes the
-// accumulation, compensation and image buffers, and everything else the
-// kernel reads (the scene in its device layout, the sphere tree, the
-// statistics counters) lives in one file-scope device array, `scratch`, of
-// kScratchBytes.  It is for callers that cannot call hipMalloc (serving
-// loops, harnesses that forbid allocation).
+// atx_render_frames_noalloc renders frames of one scene in place
+// (launch_in_place: every pixel's frames one after another in one lane, one
+// launch for all frames of the call), with the results of
+// atx_renderer_render_frames, but allocates no device memory: the caller
+// passes the accumulation, compensation and image buffers, and everything else
+// the kernel reads (the scene in its device layout, its tiles, the table entry,
+// the queue and the statistics counters) lives in one file-scope device array,
+// `scratch`, of kScratchBytes.  It is for callers that cannot call hipMalloc
+// (serving loops, harnesses that forbid allocation).
 //
 // Each device holds its own copy of `scratch` for the life of the process,
 // at its own address; that address is looked up once per device with
@@ -18,11 +19,12 @@
 // rendered, so consecutive calls on one thread do not overlap.
 #include <mutex>
 #include <string.h>
+#include <vector>
 
 #include "camera_host.h"
 #include "device_types.h"
 #include "host_common.h"
-#include "wavefront.h"
+#include "wavefront_host.h"
 
 namespace atx {
 namespace {
@@ -83,17 +85,21 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     HostBvh T;
     if (accel == ATX_ACCEL_BVH) build_bvh(L.sph.data(), (uint32_t)num_spheres, kBvhLayouts, &T);
 
-    // scratch layout: counters | spheres | material ids | materials | lights | tree
+    // scratch layout: counters | queue | table entry | spheres | material ids |
+    // materials | lights | tree
     const size_t off_ctr = 0;
-    const size_t off_sph = align256(off_ctr + kCtrCount * sizeof(unsigned long long));
+    const size_t off_queue = align256(off_ctr + kCtrCount * sizeof(unsigned long long));
+    const size_t off_table = align256(off_queue + sizeof(unsigned int));
+    const size_t off_sph = align256(off_table + sizeof(WfScene));
     const size_t off_smat = align256(off_sph + L.sph.size() * 4);
     const size_t off_mat = align256(off_smat + L.sph_mat.size() * 4);
     const size_t off_light = align256(off_mat + L.mat.size() * 4);
-    const size_t off_nodes = align256(off_light + L.light.size() * 4);
-    const size_t off_lsph = align256(off_nodes + T.nodes.size() * 4);
-    const size_t off_lidx = align256(off_lsph + T.lsph.size() * 4);
-    const size_t off_big = align256(off_lidx + T.lidx.size() * 4);
-    const size_t total = align256(off_big + T.big.size() * 4);
+    const size_t off_big = align256(off_light + L.light.size() * 4);
+    const size_t off_tiles = align256(off_big + T.big.size() * 4);
+    const size_t off_boxes = align256(off_tiles + T.tiles.size() * 4);
+    const size_t off_tsph = align256(off_boxes + T.tboxes.size() * 4);
+    const size_t off_tidx = align256(off_tsph + T.tsph.size() * 4);
+    const size_t total = align256(off_tidx + T.tidx.size() * 4);
     if (total > kScratchBytes) {
         set_error("scene needs %zu bytes of device scratch; atx_render_frames_noalloc holds at most %zu "
                   "(use atx_renderer_* for larger scenes)",
@@ -115,48 +121,46 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     ATX_HIP(put(off_smat, L.sph_mat.data(), L.sph_mat.size() * 4));
     ATX_HIP(put(off_mat, L.mat.data(), L.mat.size() * 4));
     ATX_HIP(put(off_light, L.light.data(), L.light.size() * 4));
-    ATX_HIP(put(off_nodes, T.nodes.data(), T.nodes.size() * 4));
-    ATX_HIP(put(off_lsph, T.lsph.data(), T.lsph.size() * 4));
-    ATX_HIP(put(off_lidx, T.lidx.data(), T.lidx.size() * 4));
     ATX_HIP(put(off_big, T.big.data(), T.big.size() * 4));
+    ATX_HIP(put(off_tiles, T.tiles.data(), T.tiles.size() * 4));
+    ATX_HIP(put(off_boxes, T.tboxes.data(), T.tboxes.size() * 4));
+    ATX_HIP(put(off_tsph, T.tsph.data(), T.tsph.size() * 4));
+    ATX_HIP(put(off_tidx, T.tidx.data(), T.tidx.size() * 4));
     // the counters start at zero in every call (a fill kernel, not a memset node)
     ATX_HIP(launch_zero_u32(reinterpret_cast<unsigned int*>(base + off_ctr),
                             (uint32_t)(kCtrCount * sizeof(unsigned long long) / 4), stream));
 
-    PlainArgs a{};
-    a.sc.sph = reinterpret_cast<const float4*>(base + off_sph);
-    a.sc.sph_mat = reinterpret_cast<const int32_t*>(base + off_smat);
-    a.sc.mat = reinterpret_cast<const float4*>(base + off_mat);
-    a.sc.light = reinterpret_cast<const float4*>(base + off_light);
-    a.sc.n_sph = (uint32_t)num_spheres;
-    a.sc.n_mat = (uint32_t)num_materials;
-    a.sc.n_light = (uint32_t)num_lights;
+    WfScene w{};
+    w.sph = reinterpret_cast<const float4*>(base + off_sph);
+    w.sph_mat = reinterpret_cast<const int32_t*>(base + off_smat);
+    w.mat = reinterpret_cast<const float4*>(base + off_mat);
+    w.light = reinterpret_cast<const float4*>(base + off_light);
+    w.n_sph = (uint32_t)num_spheres;
+    w.n_mat = (uint32_t)num_materials;
+    w.n_light = (uint32_t)num_lights;
     if (T.n_nodes > 0)
-        a.sc.bvh = bvh_dev_from(T, {base + off_nodes, base + off_lsph, base + off_lidx, base + off_big, nullptr, nullptr,
-                                    nullptr, nullptr});
-    camera_inverse_matrices(cam->position, cam->direction, cam->fov_deg, cam->near_clip, cam->far_clip,
-                            cam->width, cam->height, a.cam.inv_proj, a.cam.inv_view);
-    memcpy(a.cam.pos, cam->position, sizeof(a.cam.pos));
-    a.cam.width = cam->width;
-    a.cam.height = cam->height;
-    a.max_bounces = settings->max_bounces;
-    a.sky_light = settings->sky_light ? 1u : 0u;
-    a.accum = reinterpret_cast<float4*>(accum);
-    a.comp = accumulator == ATX_ACCUM_KAHAN ? reinterpret_cast<float4*>(comp) : nullptr;
-    a.image = image;
-    a.counters = reinterpret_cast<unsigned long long*>(base + off_ctr);
-
-    // the variant atx_renderer_render_frames picks for the plain kernel
-    uint32_t variant = 0;
-    if ((size_t)num_spheres * sizeof(float4) <= 64u * 1024u) variant |= kVarLds;
-    if (accumulator == ATX_ACCUM_KAHAN) variant |= kVarKahan;
-    if (a.sc.bvh.n_nodes) variant = (variant & ~(uint32_t)kVarLds) | kVarBvh;
-
-    uint32_t fi = first_frame;
-    for (uint32_t f = 0; f < frames; ++f) {
-        a.frame = fi;
-        ATX_HIP(launch_plain(a, variant, stream));
-        fi = settings->accumulation ? fi + 1u : 1u;   // Renderer.cu:245-248
+        w.bvh = bvh_dev_from(T, {nullptr, nullptr, nullptr, base + off_big, base + off_tiles, base + off_boxes,
+                                 base + off_tsph, base + off_tidx});
+    const bool kahan = accumulator == ATX_ACCUM_KAHAN;
+    // one launch for all frames; with accumulation off a launch per frame, the
+    // index back at 1 after the first (Renderer.cu:245-248).  The entries stay
+    // in place until their copies have run.
+    const uint32_t launches = settings->accumulation ? 1u : frames;
+    std::vector<WfScene> entries(launches, w);
+    for (uint32_t l = 0; l < launches; ++l) {
+        WfScene& w = entries[l];
+        const uint32_t n = settings->accumulation ? frames : 1u;
+        const uint32_t fi = l == 0 ? first_frame : 1u;
+        fill_wf_view(*settings, *cam, reinterpret_cast<float4*>(accum), kahan ? reinterpret_cast<float4*>(comp) : nullptr,
+                     image, kahan, fi, n, &w);
+        WfPass p{};
+        ATX_CHECK_ARG(layout_in_place(w, &p), "viewport too large");
+        p.scenes = reinterpret_cast<const WfScene*>(base + off_table);
+        p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
+        p.counters = reinterpret_cast<unsigned long long*>(base + off_ctr);
+        ATX_HIP(put(off_table, &w, sizeof(w)));
+        ATX_HIP(launch_zero_u32(p.queue, 1, stream));
+        ATX_HIP(launch_in_place(p, w.bvh.n_tiles == 0, stream));
     }
     // the host copies above read L and T, which end with this call
     ATX_HIP(hipStreamSynchronize(stream));

@@ -225,6 +225,72 @@ __device__ __forceinline__ uint32_t job_pixel(CScene* S, uint32_t slots, uint32_
     return S->hit_px ? S->hit_px[slot] : slot;
 }
 
+// In-place launches: the pixel of job j, whose 64 consecutive jobs are an 8 x 8
+// tile (past the image's edge: ~0).
+__device__ __forceinline__ uint32_t in_place_pixel(CScene* S, uint32_t j)
+{
+    const uint32_t W = S->width, tiles_x = (W + 7u) / 8u;
+    const uint32_t t = j >> 6, ty = t / tiles_x, tx = t - ty * tiles_x;
+    const uint32_t x = tx * 8u + (j & 7u), y = ty * 8u + ((j >> 3) & 7u);
+    return x < W && y < S->height ? y * W + x : ~0u;
+}
+
+__device__ __forceinline__ f3 primary_direction(CScene* S, uint32_t px)
+{
+    const uint32_t W = S->width;
+    const uint32_t y = px / W, x = px - y * W;
+    float ip[16], iv[16];
+    for (int k = 0; k < 16; ++k) {
+        ip[k] = S->inv_proj[k];
+        iv[k] = S->inv_view[k];
+    }
+    return camera_ray(ip, iv, x, y, W, S->height);
+}
+
+// Adds a sample to a channel's running sum (Renderer.cu:165), compensated if
+// kahan (c: the compensation).
+__device__ __forceinline__ void accumulate(bool kahan, float v, float& acc, float& c)
+{
+    if (kahan) {
+        const float y = v - c, t = acc + y;
+        c = (t - acc) - y;
+        acc = t;
+    } else {
+        acc = acc + v;
+    }
+}
+
+// Display value of a sum over `frame` frames (Renderer.cu:166-168, Renderer.h:70-78).
+__device__ __forceinline__ uint32_t display(float4 acc, uint32_t frame)
+{
+    const float fi = (float)frame;
+    return rgba8(gclamp(acc.x / fi, 0.0f, 1.0f), gclamp(acc.y / fi, 0.0f, 1.0f), gclamp(acc.z / fi, 0.0f, 1.0f),
+                 gclamp(acc.w / fi, 0.0f, 1.0f));
+}
+
+// In-place launches: the sample of pixel px in frame f of the launch goes to
+// the accumulation; the last frame's also to the image.
+__device__ __forceinline__ void add_sample(CScene* S, uint32_t px, uint32_t f, f3 col)
+{
+    const uint32_t frame = S->frame0 + f;
+    const bool kahan = S->kahan != 0u;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 acc = frame == 1u ? zero : S->accum[px];
+    float4 c = kahan && frame != 1u ? S->comp[px] : zero;
+    accumulate(kahan, col.x, acc.x, c.x);
+    accumulate(kahan, col.y, acc.y, c.y);
+    accumulate(kahan, col.z, acc.z, c.z);
+    accumulate(kahan, 1.0f, acc.w, c.w);
+    S->accum[px] = acc;
+    if (kahan)
+        S->comp[px] = c;
+    if (f + 1u == S->frames) {
+        S->image[px] = display(acc, frame);
+        if (S->dbg_radiance)
+            S->dbg_radiance[px] = make_float4(col.x, col.y, col.z, 1.0f);
+    }
+}
+
 // The sample of the scene's job `job` (`slots` jobs per frame), and the
 // last frame's debug capture.
 __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t job, f3 col)
@@ -238,7 +304,14 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
     }
 }
 
-template <uint32_t kWaves, bool kTree>
+// kInPlace: a job is a pixel, and its lane renders the launch's frames one
+// after another into the accumulation; no samples, no first-bounce cache.  A
+// kernel with one lane per pixel and frame, 64 pixels to a wave until its
+// longest path ended, took 0.62 ms per frame at 1280x720 with 129 spheres;
+// here lanes go on with their next frame or another pixel: a call of 4 frames
+// 2.68 -> 0.81 ms.  The tree instance is bound like
+// the sampling one, by VALU issue.
+template <uint32_t kWaves, bool kTree, bool kInPlace = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -255,6 +328,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     __shared__ uint32_t parked_all[4][kPark ? kParked : 1][64];
     uint32_t(*parked)[64] = parked_all[threadIdx.x >> 6];
     __shared__ uint32_t tile_masks[4][kTree ? kTileRows : 1][64];
+    // in place: the pixel's primary direction and the frame its path is in
+    __shared__ uint32_t own_all[4][kInPlace ? 4 : 1][64];
+    uint32_t(*own)[64] = own_all[threadIdx.x >> 6];
 
     // ---- wave-uniform scheduling state ----
     CScene* scenes = as_const(a.scenes);
@@ -288,6 +364,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     unsigned long long rays = 0, reused = 0;
     uint32_t tests = 0, boxes = 0;
 
+    // in place: starts pixel `job`'s path of the launch's frame f
+    const auto start_in_place = [&](uint32_t f, f3 dir) {
+        own[3][lane] = f;
+        ro = mk(S->cam_pos[0], S->cam_pos[1], S->cam_pos[2]);
+        rd = dir;
+        tp = mk(1.0f, 1.0f, 1.0f);
+        col = mk(0.0f, 0.0f, 0.0f);
+        seed = job * (S->frame0 + f);
+        bounce = 0;
+        state = kCont;
+        capture = (S->dbg_hit || S->dbg_shadow) && f + 1u == S->frames;
+        for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
+            if (S->dbg_hit) S->dbg_hit[(size_t)job * S->dbg_bounces + i] = -2;
+            if (S->dbg_shadow) S->dbg_shadow[(size_t)job * S->dbg_bounces + i] = -2;
+        }
+    };
+
     for (;;) {
         // ---------------- hand jobs to idle lanes (uniform control flow) ----------------
         for (;;) {
@@ -308,7 +401,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 const uint32_t rank = (uint32_t)__popcll(idle & lanes_below);
                 const uint32_t nidle = (uint32_t)__popcll(idle);
                 uint32_t cached_rays = 0;   // this lane's rays taken from the first-bounce cache
-                if (state == kIdle && rank < avail) {
+                if constexpr (kInPlace) {
+                    if (state == kIdle && rank < avail) {
+                        const uint32_t px = in_place_pixel(S, blk0 + blk_next + rank);
+                        if (px != ~0u) {
+                            job = px;
+                            const f3 dir = primary_direction(S, px);
+                            own[0][lane] = __float_as_uint(dir.x);
+                            own[1][lane] = __float_as_uint(dir.y);
+                            own[2][lane] = __float_as_uint(dir.z);
+                            start_in_place(0u, dir);
+                        }
+                    }
+                } else if (state == kIdle && rank < avail) {
                     job = blk0 + blk_next + rank;
                     uint32_t px, frame;
                     job_pixel_frame(job, slots, S->div_group, px, frame);
@@ -326,14 +431,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                         const float4 dv = S->dirs[px];
                         rd = mk(dv.x, dv.y, dv.z);
                     } else {
-                        const uint32_t W = S->width;
-                        const uint32_t y = px / W, x = px - y * W;
-                        float ip[16], iv[16];
-                        for (int k = 0; k < 16; ++k) {
-                            ip[k] = S->inv_proj[k];
-                            iv[k] = S->inv_view[k];
-                        }
-                        rd = camera_ray(ip, iv, x, y, W, S->height);
+                        rd = primary_direction(S, px);
                     }
                     tp = mk(1.0f, 1.0f, 1.0f);
                     col = mk(0.0f, 0.0f, 0.0f);
@@ -442,7 +540,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 slots = (uint32_t)__builtin_amdgcn_readfirstlane((int)job_slots(S->hit_px, S->width * S->height));
             }
             pend = -1;
-            const uint32_t jobs = slots * S->frames;
+            const uint32_t jobs = kInPlace ? in_place_jobs(S->width, S->height) : slots * S->frames;
             blk0 = ((uint32_t)c - S->chunk_begin) * P;
             blk_end = blk0 >= jobs ? 0u : (jobs - blk0 < P ? jobs - blk0 : P);
             blk_next = 0;
@@ -493,7 +591,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 const BvhDev B = S->bvh;
                 h = trace_tiles(B, flat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
             } else {
-                h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
+                if (kInPlace && S->exact)
+                    h = trace_exact(flat, S->n_sph, ro, rd);
+                else
+                    h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
                 q.tests = S->n_sph;
             }
             if constexpr (kPark) {
@@ -521,11 +622,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             }
         };
 
+        const auto pixel = [&]() { return kInPlace ? job : job_pixel(S, slots, job); };
         const auto shade = [&]() {
             // ---------------- shading (divergent) ----------------
             if (!shadow) {
                 if (capture && S->dbg_hit && (uint32_t)bounce < S->dbg_bounces)
-                    S->dbg_hit[(size_t)job_pixel(S, slots, job) * S->dbg_bounces + bounce] = h.id;
+                    S->dbg_hit[(size_t)pixel() * S->dbg_bounces + bounce] = h.id;
                 if (h.id < 0) {
                     if (S->sky_light)
                         col = add(col, mul(mk(0.6f, 0.7f, 0.9f), tp));
@@ -543,7 +645,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 }
             } else {
                 if (capture && S->dbg_shadow && (uint32_t)bounce < S->dbg_bounces)
-                    S->dbg_shadow[(size_t)job_pixel(S, slots, job) * S->dbg_bounces + bounce] = h.id;
+                    S->dbg_shadow[(size_t)pixel() * S->dbg_bounces + bounce] = h.id;
                 if (lit_by(h, dist2))
                     add_light(S, mid, lidx, nrm, vd, rd, tp, col);
                 end_bounce = true;
@@ -568,8 +670,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         if (__any(tests >= 0x80000000u || boxes >= 0x80000000u))
             flush_counters(a.counters, lane, tests, boxes);
         if (end_path) {
-            store_sample(S, slots, job, col);
             state = kIdle;
+            if constexpr (kInPlace) {
+                const uint32_t f = own[3][lane];
+                add_sample(S, job, f, col);
+                if (f + 1u < S->frames)
+                    start_in_place(f + 1u, mk(__uint_as_float(own[0][lane]), __uint_as_float(own[1][lane]),
+                                              __uint_as_float(own[2][lane])));
+            } else {
+                store_sample(S, slots, job, col);
+            }
         }
     }
 
@@ -667,9 +777,7 @@ __global__ __launch_bounds__(256) void k_accumulate(WfPass a)
         }
     }
     S.accum[px] = acc;
-    const float fi = (float)(S.frame0 + S.frames - 1u);
-    S.image[px] = rgba8(gclamp(acc.x / fi, 0.0f, 1.0f), gclamp(acc.y / fi, 0.0f, 1.0f),
-                        gclamp(acc.z / fi, 0.0f, 1.0f), gclamp(acc.w / fi, 0.0f, 1.0f));
+    S.image[px] = display(acc, S.frame0 + S.frames - 1u);
 }
 
 struct CamDirArgs {
@@ -840,6 +948,26 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
     if (e != hipSuccess)
         return e;
     hipLaunchKernelGGL(k_accumulate, dim3((p.total_px + 255u) / 256u), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_in_place(const WfPass& pass, bool flat_only, hipStream_t stream)
+{
+    WfPass p = pass;
+    p.refill_min = kRefillMin;
+    if (p.total_chunks == 0 || p.n_scenes != 1)
+        return hipErrorInvalidValue;
+    const PathKernel kernel = flat_only ? k_render_wavefront<kWfWavesFlat, false, true>
+                                        : k_render_wavefront<kWfWavesTree, true, true>;
+    int dev = 0, cus = 0, blocks = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 256, 0);
+    if (e != hipSuccess)
+        return e;
+    const uint32_t full = (uint32_t)(cus > 0 ? cus : 1) * (uint32_t)(blocks > 0 ? blocks : 1);
+    const uint32_t most = (p.total_chunks + 3u) / 4u;   // a first chunk for each wave
+    hipLaunchKernelGGL(kernel, dim3(full < most ? full : most), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -57,7 +57,6 @@ struct Renderer {
     atx_settings settings{1, 0, {0, 0}, 15};  // Scene.h:49-56 defaults
     uint32_t frame_index = 1;
     int accumulator = ATX_ACCUM_NAIVE;
-    size_t lds_budget = 64 * 1024;
     bool exact_loop = false;
     atx_render_stats stats{};
 };
@@ -79,44 +78,26 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     }
     ATX_CHECK_ARG(r->settings.max_bounces >= 0, "max_bounces must be >= 0");
 
-    PlainArgs a{};
-    a.sc.sph = r->geo.sph.as<float4>();
-    a.sc.sph_mat = r->geo.sph_mat.as<int32_t>();
-    a.sc.mat = r->geo.mat.as<float4>();
-    a.sc.light = r->geo.light.as<float4>();
-    a.sc.n_sph = r->geo.n_sph;
-    a.sc.n_mat = r->geo.n_mat;
-    a.sc.n_light = r->geo.n_light;
     const int accel = r->exact_loop ? ATX_ACCEL_NONE : r->accel;
-    a.sc.bvh = r->geo.accel(accel);
-    camera_inverse_matrices(cam->position, cam->direction, cam->fov_deg, cam->near_clip, cam->far_clip,
-                            cam->width, cam->height, a.cam.inv_proj, a.cam.inv_view);
-    memcpy(a.cam.pos, cam->position, sizeof(a.cam.pos));
-    a.cam.width = r->width;
-    a.cam.height = r->height;
-    a.max_bounces = r->settings.max_bounces;
-    a.sky_light = r->settings.sky_light ? 1u : 0u;
-    a.accum = r->accum.as<float4>();
-    a.comp = r->accumulator == ATX_ACCUM_KAHAN ? r->comp.as<float4>() : nullptr;
-    a.image = r->image.as<uint32_t>();
-    a.counters = r->counters.as<unsigned long long>();
-
     const size_t npx = (size_t)r->width * r->height;
+    float4* const accum = r->accum.as<float4>();
+    float4* const comp = r->accumulator == ATX_ACCUM_KAHAN ? r->comp.as<float4>() : nullptr;
     DevBuf& d_rad = r->dbg_rad;
     DevBuf& d_hit = r->dbg_hit;
     DevBuf& d_sh = r->dbg_sh;
-    uint32_t variant = 0;
-    if ((size_t)r->geo.n_sph * sizeof(float4) <= r->lds_budget) variant |= kVarLds;
-    if (r->accumulator == ATX_ACCUM_KAHAN) variant |= kVarKahan;
-    if (r->exact_loop) variant |= kVarExactLoop;
-    if (a.sc.bvh.n_nodes) variant = (variant & ~(uint32_t)kVarLds) | kVarBvh;
-    if (dbg_rad || dbg_hit || dbg_shadow) {
-        variant |= kVarDebug;
-        if (dbg_rad) { ATX_HIP(d_rad.reserve(npx * sizeof(float4))); a.dbg_radiance = d_rad.as<float4>(); }
-        if (dbg_hit) { ATX_HIP(d_hit.reserve(npx * dbg_bounces * 4)); a.dbg_hit = d_hit.as<int32_t>(); }
-        if (dbg_shadow) { ATX_HIP(d_sh.reserve(npx * dbg_bounces * 4)); a.dbg_shadow = d_sh.as<int32_t>(); }
-        a.dbg_bounces = dbg_bounces;
-    }
+    if (dbg_rad) ATX_HIP(d_rad.reserve(npx * sizeof(float4)));
+    if (dbg_hit) ATX_HIP(d_hit.reserve(npx * dbg_bounces * 4));
+    if (dbg_shadow) ATX_HIP(d_sh.reserve(npx * dbg_bounces * 4));
+    const auto entry = [&](uint32_t frame0, uint32_t n) {
+        WfScene e;
+        fill_wf_scene(r->geo, r->settings, *cam, accum, comp, r->image.as<uint32_t>(), comp != nullptr, frame0, n,
+                      accel, &e);
+        if (dbg_rad) e.dbg_radiance = d_rad.as<float4>();
+        if (dbg_hit) e.dbg_hit = d_hit.as<int32_t>();
+        if (dbg_shadow) e.dbg_shadow = d_sh.as<int32_t>();
+        e.dbg_bounces = dbg_bounces;
+        return e;
+    };
 
     // wavefront mode: launches of up to wf_frames frames each (one frame per
     // launch when accumulation is off: the frame index then stays 1)
@@ -131,13 +112,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         const uint32_t per_launch = std::min(r->wf_frames, fit);
         while (left > 0) {
             const uint32_t k = r->settings.accumulation ? (left < per_launch ? left : per_launch) : 1u;
-            WfScene e;
-            fill_wf_scene(r->geo, r->settings, *cam, a.accum, a.comp, a.image, a.comp != nullptr, fi, k, accel,
-                          &e);
-            e.dbg_radiance = a.dbg_radiance;
-            e.dbg_hit = a.dbg_hit;
-            e.dbg_shadow = a.dbg_shadow;
-            e.dbg_bounces = a.dbg_bounces;
+            const WfScene e = entry(fi, k);
             table.push_back(e);
             launch_frames.push_back(k);
             fi = r->settings.accumulation ? fi + k : 1u;
@@ -192,10 +167,6 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
                 return ATX_ERR_INVALID;
             }
         }
-        ATX_HIP(r->wf_table.reserve(table.size() * sizeof(WfScene)));
-        ATX_HIP(r->wf_queue.reserve(table.size() * sizeof(unsigned int)));
-        ATX_HIP(hipMemcpyAsync(r->wf_table.get(), table.data(), table.size() * sizeof(WfScene),
-                               hipMemcpyHostToDevice, r->stream));
         while (r->wf_ev.size() < 2 * table.size()) {
             hipEvent_t ev = nullptr;
             ATX_HIP(hipEventCreate(&ev));
@@ -203,8 +174,32 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         }
     }
 
+    // the plain kernel: an in-place launch per frame
+    std::vector<WfPass> passes;
+    if (!wf) {
+        for (uint32_t f = 0, fi = r->frame_index; f < frames; ++f) {
+            WfScene e = entry(fi, 1);
+            e.exact = r->exact_loop ? 1u : 0u;
+            if (r->exact_loop) e.bvh.n_tiles = 0;
+            WfPass p{};
+            if (!layout_in_place(e, &p)) {
+                set_error("render: %u x %u pixels exceed one launch", e.width, e.height);
+                return ATX_ERR_INVALID;
+            }
+            table.push_back(e);
+            passes.push_back(p);
+            if (r->settings.accumulation) ++fi;
+        }
+    }
+    const uint32_t n_launch = (uint32_t)table.size();
+    if (n_launch) {
+        ATX_HIP(r->wf_table.reserve(n_launch * sizeof(WfScene)));
+        ATX_HIP(r->wf_queue.reserve(n_launch * sizeof(unsigned int)));
+        ATX_HIP(hipMemcpyAsync(r->wf_table.get(), table.data(), n_launch * sizeof(WfScene), hipMemcpyHostToDevice,
+                               r->stream));
+        ATX_HIP(launch_zero_u32(r->wf_queue.as<unsigned int>(), n_launch, r->stream));
+    }
     ATX_HIP(hipMemsetAsync(r->counters.get(), 0, kCtrCount * sizeof(unsigned long long), r->stream));
-    if (wf) ATX_HIP(launch_zero_u32(r->wf_queue.as<unsigned int>(), (uint32_t)table.size(), r->stream));
     ATX_HIP(hipEventRecord(r->ev0, r->stream));
     if (wf) {
         for (size_t l = 0; l < table.size(); ++l) {
@@ -215,7 +210,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             wp.chunk_px = launch_chunk[l];
             wp.total_px = table[l].width * table[l].height;
             wp.queue = r->wf_queue.as<unsigned int>() + l;
-            wp.counters = a.counters;
+            wp.counters = r->counters.as<unsigned long long>();
             ATX_HIP(hipEventRecord(r->wf_ev[2 * l], r->stream));
             ATX_HIP(launch_wavefront(wp, shape, r->stream, r->wf_ev[2 * l + 1]));
             // Renderer.cu:245-248, once per frame of the launch
@@ -225,9 +220,13 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             }
         }
     } else {
+        const bool flat_only = n_launch == 0 || wf_flat_only(table.data(), 1);
         for (uint32_t f = 0; f < frames; ++f) {
-            a.frame = r->frame_index;
-            ATX_HIP(launch_plain(a, variant, r->stream));
+            WfPass wp = passes[f];
+            wp.scenes = r->wf_table.as<WfScene>() + f;
+            wp.queue = r->wf_queue.as<unsigned int>() + f;
+            wp.counters = r->counters.as<unsigned long long>();
+            ATX_HIP(launch_in_place(wp, flat_only, r->stream));
             // Renderer.cu:245-248
             if (r->settings.accumulation) r->frame_index++;
             else r->frame_index = 1;
@@ -305,7 +304,6 @@ int atx_renderer_create(atx_renderer** out)
         return ATX_ERR_HIP;
     }
     if (const char* env = getenv("ATX_EXACT_LOOP")) r->exact_loop = atoi(env) != 0;
-    if (const char* env = getenv("ATX_LDS_BUDGET")) r->lds_budget = (size_t)strtoull(env, nullptr, 10);
     if (const char* env = getenv("ATX_WF_CHUNK")) {
         const uint32_t c = (uint32_t)strtoul(env, nullptr, 10);
         if (c >= 64 && c % 64 == 0 && c <= kMaxChunkPx) r->wf_chunk = c;

@@ -80,6 +80,7 @@ struct WfScene {
     uint32_t n_chunks;     // ceil(width * height * frames / chunk_px)
     uint32_t kahan;        // 1: compensated accumulation (comp must be valid)
     uint32_t dbg_bounces;  // stride of the debug arrays
+    uint32_t exact;        // in-place launches without a tree: exact closest-hit loop
     uint32_t px_begin;     // first pixel of this scene in the launch's pixel range
     float inv_proj[16];
     float inv_view[16];
@@ -165,6 +166,13 @@ __host__ __device__ __forceinline__ void job_pixel_frame(uint32_t j, uint32_t pi
     px = kJobGroupPx * g + (w - frame * m);
 }
 
+// Jobs of an in-place launch: the pixels of whole 8 x 8 tiles.
+constexpr uint32_t kInPlaceChunk = 64;
+__host__ __device__ __forceinline__ uint32_t in_place_jobs(uint32_t width, uint32_t height)
+{
+    return ((width + 7u) / 8u) * ((height + 7u) / 8u) * 64u;
+}
+
 // The job of slot k in the launch's frame f (the inverse of job_pixel_frame).
 __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint32_t pixels, uint32_t frames)
 {
@@ -202,6 +210,11 @@ struct WfLaunch {
 // given, is recorded on the stream between the two.
 hipError_t launch_wavefront(const WfPass& p, const WfLaunch& l, hipStream_t stream,
                             hipEvent_t paths_done = nullptr);
+// In-place rendering of one scene (p.n_scenes 1, chunks of kInPlaceChunk jobs
+// laid out by layout_in_place): every pixel's frames one after another in one
+// lane, added to the accumulation as they end.  It needs neither samples nor
+// a first-bounce cache, so no memory beyond the scene's and the image's.
+hipError_t launch_in_place(const WfPass& p, bool flat_only, hipStream_t stream);
 hipError_t launch_zero_u32(unsigned int* p, uint32_t n, hipStream_t stream);
 // Writes the primary ray direction of every pixel of s's camera to dirs
 // (width * height float4, w = 0): camera_ray, computed once instead of per path.

@@ -11,19 +11,10 @@
 
 namespace atx {
 
-inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_camera& cam, float4* accum,
-                          float4* comp, uint32_t* image, bool kahan, uint32_t frame0, uint32_t frames,
-                          int accel, WfScene* out)
+// Everything of an entry but the scene's arrays.
+inline void fill_wf_view(const atx_settings& st, const atx_camera& cam, float4* accum, float4* comp, uint32_t* image,
+                         bool kahan, uint32_t frame0, uint32_t frames, WfScene* out)
 {
-    memset(out, 0, sizeof(*out));
-    out->sph = g.sph.as<float4>();
-    out->sph_mat = g.sph_mat.as<int32_t>();
-    out->mat = g.mat.as<float4>();
-    out->mat_rr = g.mat_rr.as<float4>();
-    out->light = g.light.as<float4>();
-    out->n_sph = g.n_sph;
-    out->n_mat = g.n_mat;
-    out->n_light = g.n_light;
     out->width = cam.width;
     out->height = cam.height;
     out->max_bounces = st.max_bounces;
@@ -39,6 +30,22 @@ inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_c
     out->accum = accum;
     out->comp = comp;
     out->image = image;
+}
+
+inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_camera& cam, float4* accum,
+                          float4* comp, uint32_t* image, bool kahan, uint32_t frame0, uint32_t frames,
+                          int accel, WfScene* out)
+{
+    memset(out, 0, sizeof(*out));
+    out->sph = g.sph.as<float4>();
+    out->sph_mat = g.sph_mat.as<int32_t>();
+    out->mat = g.mat.as<float4>();
+    out->mat_rr = g.mat_rr.as<float4>();
+    out->light = g.light.as<float4>();
+    out->n_sph = g.n_sph;
+    out->n_mat = g.n_mat;
+    out->n_light = g.n_light;
+    fill_wf_view(st, cam, accum, comp, image, kahan, frame0, frames, out);
     out->bvh = g.accel(accel);
 }
 
@@ -129,6 +136,24 @@ inline bool layout_launch(WfScene* tab, size_t n, uint32_t chunk_px, float3* sam
     p->total_chunks = (uint32_t)chunks;
     p->total_px = (uint32_t)px;
     p->chunk_px = chunk_px;
+    return true;
+}
+
+// The same for an in-place launch of one scene.  False when its jobs do not
+// fit 32 bits.
+inline bool layout_in_place(WfScene& w, WfPass* p)
+{
+    const uint64_t jobs = (((uint64_t)w.width + 7) / 8) * (((uint64_t)w.height + 7) / 8) * 64;
+    if (jobs + kInPlaceChunk >= 1ull << 32)
+        return false;
+    w.chunk_begin = w.px_begin = 0;
+    w.n_chunks = (uint32_t)(jobs / kInPlaceChunk);
+    w.div_group = udiv_make(kJobGroupPx * w.frames);
+    w.div_light = udiv_make(w.n_light ? w.n_light : 1u);
+    p->n_scenes = 1;
+    p->total_chunks = w.n_chunks;
+    p->total_px = w.width * w.height;
+    p->chunk_px = kInPlaceChunk;
     return true;
 }
 

@@ -130,7 +130,7 @@ const char* atx_version(void);
 int atx_device_count(int* count);
 int atx_device_synchronize(void);
 
-/* ---- Renderer: single scene, one frame per Render (the plain kernel) ----- */
+/* ---- Renderer: single scene, one frame per Render ------------------------ */
 typedef struct atx_renderer atx_renderer;
 
 int atx_renderer_create(atx_renderer** out);
@@ -187,7 +187,7 @@ int atx_renderer_reserve(atx_renderer* r, uint32_t frames);
 /* ---- Allocation-free rendering ---------------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (serving loops, harnesses that forbid hipMalloc): renders `frames`
- * frames of one scene with the plain kernel, exactly as
+ * frames of one scene, a lane per pixel, exactly as
  * atx_renderer_render_frames does with ATX_KERNEL_PLAIN, frame indices
  * first_frame, first_frame + 1, ... (with accumulation off the index returns
  * to 1 after the first frame, Renderer.cu:245-248; frame 1 starts the
