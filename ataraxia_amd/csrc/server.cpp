@@ -119,12 +119,15 @@ static double now_s(const Server* s)
 // Device bytes a request holds while admitted: scene, tree, accumulation,
 // compensation, image, primary ray directions, first-bounce cache, and its
 // share of the tick's sample buffer.
+static size_t sample_share(const Request& r, uint32_t frames_per_tick)
+{
+    return (size_t)r.cam.width * r.cam.height * std::min<size_t>(frames_per_tick, r.spp) * kSampleBytes;
+}
 static size_t request_bytes(const Request& r, bool kahan, uint32_t frames_per_tick)
 {
     const size_t npx = (size_t)r.cam.width * r.cam.height;
-    const size_t f = std::min<size_t>(frames_per_tick, r.spp);
     return scene_device_bytes(r.spheres.size(), r.materials.size(), r.lights.size()) +
-           npx * (16 + (kahan ? 16 : 0) + 4 + 16) + npx * f * kSampleBytes +
+           npx * (16 + (kahan ? 16 : 0) + 4 + 16) + sample_share(r, frames_per_tick) +
            (r.spp >= 2 ? first_cache_bytes(npx, (uint32_t)r.lights.size()) : 0);
 }
 
@@ -134,10 +137,8 @@ static size_t request_bytes(const Request& r, bool kahan, uint32_t frames_per_ti
 // budget, then charges this.
 static size_t held_bytes(const Request& r, uint32_t frames_per_tick)
 {
-    const size_t npx = (size_t)r.cam.width * r.cam.height;
-    const size_t f = std::min<size_t>(frames_per_tick, r.spp);
     return r.geo.bytes() + r.accum.bytes() + r.comp.bytes() + r.image.bytes() + r.dirs.bytes() + r.first.bytes() +
-           npx * f * kSampleBytes;
+           sample_share(r, frames_per_tick);
 }
 
 // A launch's paths must stay below 2^31 (the kernel's 32-bit job indices).
@@ -204,7 +205,13 @@ static void release_device(Server* s, Request& r)
     r.dirs.release();
     r.first.release();
     std::lock_guard<std::mutex> lk(s->mu);
-    s->stats.hbm_in_use -= r.device_bytes;
+    // its share of the tick's sample buffer stays allocated: it becomes excess,
+    // so that nothing is admitted on bytes the buffer still holds
+    const size_t excess =
+        std::max(s->samples_excess,
+                 std::min(s->samples_excess + sample_share(r, s->cfg.frames_per_tick), s->samples.bytes()));
+    s->stats.hbm_in_use = s->stats.hbm_in_use - r.device_bytes + (excess - s->samples_excess);
+    s->samples_excess = excess;
 }
 
 // Releases the device buffers of requests the retire thread has finished
@@ -287,9 +294,12 @@ static void admit_queued(Server* s)
                 }
             }
             auto r = s->queue[pick];
-            if (s->stats.hbm_in_use + r->device_bytes > s->cfg.hbm_budget_bytes) break;
+            // its share of the samples comes out of what the buffer holds too much
+            const size_t from_excess = std::min(s->samples_excess, sample_share(*r, F));
+            if (s->stats.hbm_in_use + r->device_bytes - from_excess > s->cfg.hbm_budget_bytes) break;
             if (tick_paths + tick_paths_of(*r, F) >= kMaxTickPaths) break;   // 32-bit job indices
-            s->stats.hbm_in_use += r->device_bytes;
+            s->stats.hbm_in_use += r->device_bytes - from_excess;
+            s->samples_excess -= from_excess;
             s->stats.hbm_high_water = std::max(s->stats.hbm_high_water, s->stats.hbm_in_use);
             tick_paths += tick_paths_of(*r, F);
             newly.push_back(r);
