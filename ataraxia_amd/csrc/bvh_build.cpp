@@ -1,6 +1,7 @@
-// bvh_build.cpp -- host construction of the sphere BVH (device layout in bvh.h).
+// bvh_build.cpp -- host construction of tiles (device layout in bvh.h) and, for
+// the host checks, of a sphere BVH.
 //
-// Binary tree, surface-area heuristic over sphere boxes, at most kBvhLeafMax
+// Tree: binary, surface-area heuristic over sphere boxes, at most kBvhLeafMax
 // spheres per leaf.  All geometry is evaluated in double precision; every box
 // is rounded outwards to float and then to 16-bit cells of the root box (one
 // extra cell on each side), so a node box contains each of its spheres
@@ -309,12 +310,48 @@ void build_tiles(HostBvh* B)
     }
 }
 
+// The tree's nodes in `layouts` orders; leaves P in leaf order.
+void build_nodes(std::vector<Prim>& P, uint32_t layouts, HostBvh* out)
+{
+    Builder B(P);
+    B.build(0, (int)P.size());
+    const uint32_t nn = (uint32_t)B.nodes.size();
+
+    // Cell grid over the root box: world = base + cell * scale, with scale a
+    // float so that the device's grid coordinates mean exactly the same boxes.
+    // Boxes round outwards and get one extra cell on each side.
+    Grid g;
+    for (int a = 0; a < 3; ++a) {
+        const double lo_a = B.nodes[0].lo[a], hi_a = B.nodes[0].hi[a];
+        const double span = hi_a - lo_a;
+        float sc = round_up(span > 0.0 ? span / (double)(kBvhGrid - 4) : 1.0);
+        if (!(sc > 0.0f)) sc = 1.0f;
+        g.base[a] = lo_a;
+        g.scale[a] = sc;
+        out->base[a] = B.nodes[0].lo[a];
+        out->scale[a] = sc;
+        out->inv_scale[a] = (float)(1.0 / (double)sc);
+    }
+    out->ext = round_up((double)kBvhGrid * std::max(std::max(g.scale[0], g.scale[1]), g.scale[2]) * (1.0 + 0x1p-30));
+    out->n_nodes = nn;
+    out->layouts = layouts;
+    out->nodes.assign((size_t)layouts * nn * 4, 0u);
+    for (uint32_t oct = 0; oct < layouts; ++oct) {
+        std::vector<uint32_t> lay((size_t)nn * 4);
+        uint32_t cur = 0;
+        emit(B.nodes, 0, oct, g, lay, cur);
+        std::copy(lay.begin(), lay.end(), out->nodes.begin() + (size_t)oct * nn * 4);
+    }
+    std::vector<Prim> ordered = std::move(B.leaf_order);
+    P.swap(ordered);
+}
+
 }  // namespace
 
 void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
 {
     *out = HostBvh();
-    layouts = layouts >= kBvhLayouts ? kBvhLayouts : 1u;
+    layouts = layouts >= kBvhLayouts ? kBvhLayouts : layouts;
     if (n < kBvhMinSpheres) return;
 
     std::vector<int32_t> big;
@@ -367,7 +404,8 @@ void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
         p.idx = (int32_t)i;
         P.push_back(p);
     }
-    if (big.size() > kBvhMaxBig || P.size() < kBvhMinSpheres || P.size() > kBvhMaxTree) return;
+    if (big.size() > kBvhMaxBig || P.size() < kBvhMinSpheres || P.size() > (layouts ? kBvhMaxTree : kTileMaxSpheres))
+        return;
     std::sort(big.begin(), big.end());
 
     // Region of the tree: centre of the centres' box, bounds of distance and radius.
@@ -390,36 +428,8 @@ void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
         rb = std::max(rb, std::sqrt(dx * dx + dy * dy + dz * dz));
     }
 
-    Builder B(P);
-    B.build(0, (int)P.size());
-    const uint32_t nn = (uint32_t)B.nodes.size();
-
-    // Cell grid over the root box: world = base + cell * scale, with scale a
-    // float so that the device's grid coordinates mean exactly the same boxes.
-    // Boxes round outwards and get one extra cell on each side.
-    Grid g;
-    for (int a = 0; a < 3; ++a) {
-        const double lo_a = B.nodes[0].lo[a], hi_a = B.nodes[0].hi[a];
-        const double span = hi_a - lo_a;
-        float sc = round_up(span > 0.0 ? span / (double)(kBvhGrid - 4) : 1.0);
-        if (!(sc > 0.0f)) sc = 1.0f;
-        g.base[a] = lo_a;
-        g.scale[a] = sc;
-        out->base[a] = B.nodes[0].lo[a];
-        out->scale[a] = sc;
-        out->inv_scale[a] = (float)(1.0 / (double)sc);
-    }
-    out->ext = round_up((double)kBvhGrid * std::max(std::max(g.scale[0], g.scale[1]), g.scale[2]) * (1.0 + 0x1p-30));
-    out->n_nodes = nn;
-    out->layouts = layouts;
-    out->nodes.assign((size_t)layouts * nn * 4, 0u);
-    for (uint32_t oct = 0; oct < layouts; ++oct) {
-        std::vector<uint32_t> lay((size_t)nn * 4);
-        uint32_t cur = 0;
-        emit(B.nodes, 0, oct, g, lay, cur);
-        std::copy(lay.begin(), lay.end(), out->nodes.begin() + (size_t)oct * nn * 4);
-    }
-    for (const Prim& p : B.leaf_order) {
+    if (layouts) build_nodes(P, layouts, out);
+    for (const Prim& p : P) {
         for (int a = 0; a < 4; ++a)
             out->lsph.push_back(sph4[4 * p.idx + a]);
         out->lidx.push_back(p.idx);
@@ -436,12 +446,10 @@ void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
 
 size_t bvh_device_bytes(uint64_t n)
 {
-    const uint64_t nodes = n > 0 ? 2 * n - 1 : 0;
-    return (size_t)(kBvhLayouts * nodes * 16 + 16) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16) +
-           (size_t)(4 * (kBvhMaxBig + 1) + 16) +
-           (n <= kBvhMaxTree + kBvhMaxBig
-                ? ((size_t)((n + 31) / 32) * (kTileWords * 4 + 36) + 64) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16)
-                : 0);
+    const uint64_t tiles = (n + kTileSpheres - 1) / kTileSpheres, boxes = tiles + (tiles + 7) / 8;
+    const size_t big = 4 * (kBvhMaxBig + 1) + 16;
+    if (n > kTileMaxSpheres + kBvhMaxBig) return big;
+    return (size_t)(tiles * kTileWords * 4 + boxes * 32 + 32) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16) + big;
 }
 
 }  // namespace atx

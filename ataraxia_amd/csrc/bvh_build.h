@@ -1,5 +1,5 @@
-// bvh_build.h -- host construction of the sphere BVH whose device layout is
-// described in bvh.h.  Plain C++ (no HIP types), so that host-side checks can
+// bvh_build.h -- host construction of a scene's tiles (device layout in bvh.h),
+// and of a binary tree over the same spheres that the host checks use.  Plain C++ (no HIP types), so that host-side checks can
 // build it with any C++ compiler.
 #pragma once
 
@@ -14,6 +14,7 @@ constexpr uint32_t kBvhLeafMax = 4;      // spheres per leaf (2-bit count field)
 constexpr uint32_t kBvhMinSpheres = 16;  // smaller scenes use the flat loop only
 constexpr uint32_t kBvhMaxBig = 16;
 constexpr uint32_t kBvhMaxTree = 16382;  // tree spheres addressable by a 14-bit leaf index
+constexpr uint32_t kTileMaxSpheres = 1u << 20;
 constexpr uint32_t kTileSpheres = 32;    // spheres per tile (rows of the matrix product)
 constexpr uint32_t kTileWords = 512;     // 32-bit words of one tile
 constexpr uint32_t kTileChunk = 8;       // tiles whose candidates are kept before they are tested
@@ -27,7 +28,7 @@ constexpr uint32_t kBvhGrid = 65535;     // node boxes are 16-bit cells of the t
 // else ((first + 1) << 2) | (count - 1)).
 struct HostBvh {
     std::vector<uint32_t> nodes; // layouts * n_nodes * 4
-    std::vector<float> lsph;     // 4 per tree sphere
+    std::vector<float> lsph;     // 4 per sphere, leaf order
     std::vector<int32_t> lidx;
     std::vector<int32_t> big;
     uint32_t n_nodes = 0;
@@ -39,7 +40,7 @@ struct HostBvh {
     float ext = 0;               // upper bound of kBvhGrid * scale over the axes
     std::vector<uint32_t> tiles; // n_tiles * kTileWords, two halves per word
     std::vector<float> tboxes;   // 8 per box: centre, half size, 0, 0; tiles, then groups of eight
-    std::vector<float> tsph;     // 4 per tree sphere, tile order
+    std::vector<float> tsph;     // 4 per sphere, tile order
     std::vector<int32_t> tidx;
     uint32_t n_tiles = 0;
     float ts = 0;                // tile units per world unit
@@ -55,10 +56,12 @@ inline uint32_t tile_row(uint32_t k)
     return 8u * (i / 4u) + 4u * h + i % 4u;
 }
 
-// Builds the tree over spheres given as (cx, cy, cz, r*r) quadruples, with
-// `layouts` traversal orders (1 or kBvhLayouts).  Scenes with fewer than
-// kBvhMinSpheres spheres, or more than kBvhMaxBig spheres that cannot go into
-// a tree, get no tree (n_nodes = 0).
+// Sorts out the spheres given as (cx, cy, cz, r*r) quadruples that cannot go
+// into tiles and builds tiles over the others; with `layouts` 1 or kBvhLayouts
+// also the tree, in that many traversal orders (the kernels do not use it:
+// 0).  Scenes with fewer than kBvhMinSpheres spheres, or more than kBvhMaxBig
+// spheres kept out, or more than kTileMaxSpheres (with a tree kBvhMaxTree)
+// others get neither (n_tiles = n_nodes = 0).
 void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out);
 
 // Device bytes of the tree of an n-sphere scene (upper bound).

@@ -100,25 +100,19 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     out->n_light = (uint32_t)l;
 
     HostBvh T;
-    uint32_t layouts = kBvhLayouts;
-    if (const char* env = getenv("ATX_BVH_LAYOUTS")) layouts = (uint32_t)atoi(env);
-    build_bvh(L.sph.data(), (uint32_t)n, layouts, &T);
+    build_bvh(L.sph.data(), (uint32_t)n, 0, &T);
     out->bvh = BvhDev{};
-    if (T.n_nodes > 0) {
+    if (T.n_tiles > 0) {
         const auto put = [](DevBuf& b, const void* src, size_t bytes) -> hipError_t {
             const hipError_t e = b.reserve(bytes + 16);
             return e != hipSuccess || bytes == 0 ? e : hipMemcpy(b.get(), src, bytes, hipMemcpyHostToDevice);
         };
-        ATX_HIP(put(out->bvh_nodes, T.nodes.data(), T.nodes.size() * 4));
-        ATX_HIP(put(out->bvh_lsph, T.lsph.data(), T.lsph.size() * 4));
-        ATX_HIP(put(out->bvh_lidx, T.lidx.data(), T.lidx.size() * 4));
-        ATX_HIP(put(out->bvh_big, T.big.data(), T.big.size() * 4));
+        ATX_HIP(put(out->big, T.big.data(), T.big.size() * 4));
         ATX_HIP(put(out->tiles, T.tiles.data(), T.tiles.size() * 4));
         ATX_HIP(put(out->tile_boxes, T.tboxes.data(), T.tboxes.size() * 4));
         ATX_HIP(put(out->tile_sph, T.tsph.data(), T.tsph.size() * 4));
         ATX_HIP(put(out->tile_idx, T.tidx.data(), T.tidx.size() * 4));
-        out->bvh = bvh_dev_from(T, {out->bvh_nodes.get(), out->bvh_lsph.get(), out->bvh_lidx.get(), out->bvh_big.get(),
-                                    out->tiles.get(), out->tile_boxes.get(), out->tile_sph.get(),
+        out->bvh = bvh_dev_from(T, {out->big.get(), out->tiles.get(), out->tile_boxes.get(), out->tile_sph.get(),
                                     out->tile_idx.get()});
     }
     return ATX_OK;
@@ -127,34 +121,17 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
 BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at)
 {
     BvhDev b{};
-    b.nodes = static_cast<const uint4*>(at.nodes);
-    b.lsph = static_cast<const float4*>(at.lsph);
-    b.lidx = static_cast<const int32_t*>(at.lidx);
-    b.big = static_cast<const int32_t*>(at.big);
-    b.n_nodes = T.n_nodes;
-    b.n_big = (uint32_t)T.big.size();
-    b.layout_mask = T.layouts - 1u;
-    b.cx = T.cx;
-    b.cy = T.cy;
-    b.cz = T.cz;
-    b.rb = T.rb;
-    b.r_min = T.r_min;
-    b.r_max = T.r_max;
-    b.bx = T.base[0];
-    b.by = T.base[1];
-    b.bz = T.base[2];
-    b.sx = T.scale[0];
-    b.sy = T.scale[1];
-    b.sz = T.scale[2];
-    b.isx = T.inv_scale[0];
-    b.isy = T.inv_scale[1];
-    b.isz = T.inv_scale[2];
-    b.ext = T.ext;
     b.tiles = static_cast<const uint4*>(at.tiles);
     b.tboxes = static_cast<const float4*>(at.tboxes);
     b.tsph = static_cast<const float4*>(at.tsph);
     b.tidx = static_cast<const int32_t*>(at.tidx);
+    b.big = static_cast<const int32_t*>(at.big);
     b.n_tiles = T.n_tiles;
+    b.n_nodes = (uint32_t)(T.tboxes.size() / 8);
+    b.n_big = (uint32_t)T.big.size();
+    b.cx = T.cx;
+    b.cy = T.cy;
+    b.cz = T.cz;
     b.ts = T.ts;
     b.t_lin = T.t_lin;
     return b;

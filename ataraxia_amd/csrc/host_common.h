@@ -173,33 +173,28 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
                        uint64_t m, const atx_light* lights, uint64_t l, HostSceneLayout* out);
 
 // One scene's geometry in HBM (device layout of device_types.h), with its
-// sphere BVH (bvh.h; bvh.n_nodes = 0 when the scene has no tree).
+// tiles (bvh.h; bvh.n_tiles = 0 when the scene has none).
 struct DevScene {
     DevBuf sph, sph_mat, mat, mat_rr, light;
-    DevBuf bvh_nodes, bvh_lsph, bvh_lidx, bvh_big, tiles, tile_boxes, tile_sph, tile_idx;
+    DevBuf big, tiles, tile_boxes, tile_sph, tile_idx;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
     BvhDev bvh{};
     void use_pool(DevPool* pool)
     {
-        for (DevBuf* b : {&sph, &sph_mat, &mat, &mat_rr, &light, &bvh_nodes, &bvh_lsph, &bvh_lidx, &bvh_big, &tiles, &tile_boxes, &tile_sph,
-                          &tile_idx})
+        for (DevBuf* b : {&sph, &sph_mat, &mat, &mat_rr, &light, &big, &tiles, &tile_boxes, &tile_sph, &tile_idx})
             b->use_pool(pool);
     }
     size_t bytes() const
     {
-        return sph.bytes() + sph_mat.bytes() + mat.bytes() + mat_rr.bytes() + light.bytes() + bvh_nodes.bytes() +
-               bvh_lsph.bytes() + bvh_lidx.bytes() + bvh_big.bytes() + tiles.bytes() + tile_boxes.bytes() +
-               tile_sph.bytes() + tile_idx.bytes();
+        return sph.bytes() + sph_mat.bytes() + mat.bytes() + mat_rr.bytes() + light.bytes() + big.bytes() +
+               tiles.bytes() + tile_boxes.bytes() + tile_sph.bytes() + tile_idx.bytes();
     }
-    // The tree to hand to a kernel: the scene's, or for ATX_ACCEL_NONE its tiles
-    // without nodes and boxes, so that every ray tests every sphere.
+    // The tiles to hand to a kernel; for ATX_ACCEL_NONE without their boxes, so
+    // that every ray tests every sphere.
     BvhDev accel(int mode) const
     {
         BvhDev b = bvh;
-        if (mode != ATX_ACCEL_BVH) {
-            b.n_nodes = 0;
-            b.tboxes = nullptr;
-        }
+        if (mode != ATX_ACCEL_BVH) b.n_nodes = 0;
         return b;
     }
 };
@@ -208,10 +203,10 @@ struct DevScene {
 int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
                  const atx_light* lights, uint64_t l, DevScene* out);
 
-// Kernel view of a host-built tree whose arrays were copied to the given
+// Kernel view of host-built tiles whose arrays were copied to the given
 // device addresses.
 struct BvhArrays {
-    const void *nodes, *lsph, *lidx, *big, *tiles, *tboxes, *tsph, *tidx;
+    const void *big, *tiles, *tboxes, *tsph, *tidx;
 };
 BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at);
 

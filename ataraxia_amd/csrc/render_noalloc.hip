@@ -29,10 +29,11 @@
 namespace atx {
 namespace {
 
-constexpr size_t kScratchBytes = 8u << 20;   // 8 MiB per device
+constexpr size_t kScratchBytes = 8u << 20;   // per device: 8 MiB for the scene
+constexpr size_t kControlBytes = 4096;       // and a page for counters, queue and table entry
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kControlBytes];
 
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
@@ -83,14 +84,20 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     int rc = build_scene_layout(spheres, num_spheres, materials, num_materials, lights, num_lights, &L);
     if (rc != ATX_OK) return rc;
     HostBvh T;
-    if (accel == ATX_ACCEL_BVH) build_bvh(L.sph.data(), (uint32_t)num_spheres, kBvhLayouts, &T);
+    build_bvh(L.sph.data(), (uint32_t)num_spheres, 0, &T);
+    // a scene that fits the scratch array only without its tiles has none
+    const size_t bare = (L.sph.size() + L.sph_mat.size() + L.mat.size() + L.light.size()) * 4;
+    if (bare + (T.tiles.size() + T.tboxes.size() + T.tsph.size() + T.tidx.size() + T.big.size()) * 4 + 16 * 256 >
+        kScratchBytes)
+        T = HostBvh();
 
-    // scratch layout: counters | queue | table entry | spheres | material ids |
-    // materials | lights | tree
-    const size_t off_ctr = 0;
+    // scratch layout: spheres | material ids | materials | lights | tiles, then
+    // past kScratchBytes counters | queue | table entry
+    const size_t off_ctr = kScratchBytes;
     const size_t off_queue = align256(off_ctr + kCtrCount * sizeof(unsigned long long));
     const size_t off_table = align256(off_queue + sizeof(unsigned int));
-    const size_t off_sph = align256(off_table + sizeof(WfScene));
+    static_assert(sizeof(WfScene) + 3 * 256 <= kControlBytes, "control page");
+    const size_t off_sph = 0;
     const size_t off_smat = align256(off_sph + L.sph.size() * 4);
     const size_t off_mat = align256(off_smat + L.sph_mat.size() * 4);
     const size_t off_light = align256(off_mat + L.mat.size() * 4);
@@ -138,9 +145,9 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     w.n_sph = (uint32_t)num_spheres;
     w.n_mat = (uint32_t)num_materials;
     w.n_light = (uint32_t)num_lights;
-    if (T.n_nodes > 0)
-        w.bvh = bvh_dev_from(T, {nullptr, nullptr, nullptr, base + off_big, base + off_tiles, base + off_boxes,
-                                 base + off_tsph, base + off_tidx});
+    if (T.n_tiles > 0)
+        w.bvh = bvh_dev_from(T, {base + off_big, base + off_tiles, base + off_boxes, base + off_tsph, base + off_tidx});
+    if (accel != ATX_ACCEL_BVH) w.bvh.n_nodes = 0;
     const bool kahan = accumulator == ATX_ACCUM_KAHAN;
     // one launch for all frames; with accumulation off a launch per frame, the
     // index back at 1 after the first (Renderer.cu:245-248).  The entries stay

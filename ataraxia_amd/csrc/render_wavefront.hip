@@ -48,7 +48,6 @@
 // each of 5 to 8 resident waves per SIMD (amdgpu_waves_per_eu; 7 by default),
 // launches with trees one for 5 (kWfWavesTree).
 #include "device_types.h"
-#include "trace_bvh.h"
 #include "trace_device.h"
 #include "trace_tiles.h"
 #include "wavefront.h"

@@ -19,9 +19,14 @@
 // hi + lo; hi takes the upper 11 bits of x, so x - hi is exact.
 //
 // Error bound, with n = |o|, D = n + 8 and u = 2^-24:
-//  * the flat loop's own rounding: a hit it reports satisfies
-//    disc >= -(93 u |o - c|^2 + 36 u r^2) (derived in trace_bvh.h), and o
-//    itself is rounded in tile units (3.4 u D^2): within 2^-17 D^2;
+//  * the flat loop's own rounding: oc, b, c, disc, sqrt, numerator and quotient
+//    are each rounded once.  With F(t) = |o + t d - c|^2 - r^2 and d_c = |o - c|,
+//    b is off by at most 4.01 u d_c, c by 6.02 u d_c^2 + u r^2, the rounding of
+//    disc moves c by at most 2.02 u (2 d_c^2 + r^2); the root of that quadratic
+//    has |F| <= 48.2 u d_c^2 + 16.1 u r^2, and the last three roundings move t by
+//    at most u (5.03 d_c + 3.02 r) on a slope of at most 6 d_c + 2 r.  So a hit
+//    it reports has |F(t)| <= 93 u d_c^2 + 36 u r^2, and its line disc >= minus
+//    that.  o itself is rounded in tile units (3.4 u D^2): within 2^-17 D^2;
 //  * hi + lo: ray side within 2^-20 |x| (lo is truncated), sphere side within
 //    2^-22 |x|, lo * lo left out (2^-21): 1.75 2^-20 of the terms' absolute sum,
 //    which is at most 1.5 (|f| + 8)^2.  E - |f|^2 is truncated towards zero,
@@ -35,11 +40,18 @@
 //
 // Boxes.  A tile's box holds its spheres; per ray it is inflated by M, a
 // bound of the excess sqrt(r^2 + q) - r, q = 2^-17 (D^2 + r^2), that the first
-// error above allows (it is at most q / (2 r) and at most sqrt(q); r <= 8
-// here, and t_lin = 2^-18 / smallest radius, rounded up), and by 2^-18 (n + 16)
-// for the slab test's own rounding.  Tiles of more than kTileFlat tiles come in groups of eight with
-// a box of their own.  Distances are culled as in the tree.  Without boxes
-// (tboxes null: ATX_ACCEL_NONE) the product tests every sphere.
+// error above allows (at most q / (2 r), t_lin = 2^-18 / smallest radius, and
+// at most sqrt(q) <= 2^-8.5 (D + 4); r <= 8 <= D), and by 2^-18 (n + 16) for the
+// slab test's own rounding (a few u of the coordinates' magnitudes).  Scenes
+// of more than kTileFlat tiles also have a box for every eight.  A box is
+// skipped when its inflated entry lies beyond an upper bound of the best
+// sphere's exact t (best_hi / a, rounded up by 2^-20): everything in it then
+// has a strictly larger t, which the reference rejects whatever its index.
+// Shadow queries (dist2 >= 0: only the reference's decision t > 0 && t*t < dist2
+// on the closest hit matters) also skip boxes beyond sqrt(dist2) and stop at
+// the first sphere whose exact t is proven below it; the sphere they return is
+// then some occluder, not necessarily the closest.  Without boxes (n_nodes 0:
+// ATX_ACCEL_NONE) the product tests every sphere.
 //
 // What bounds it: VALU issue (0.31 instructions per cycle and SIMD in the path
 // kernel; minima, compares and shifts run at half the rate of multiply-adds),
@@ -58,10 +70,42 @@
 #pragma once
 
 #include "bvh.h"
-#include "trace_bvh.h"
 #include "trace_device.h"
 
 namespace atx {
+
+#if defined(__HIP_DEVICE_COMPILE__)
+#define ATX_GLOBAL __attribute__((address_space(1)))
+#else
+#define ATX_GLOBAL
+#endif
+
+// Spheres found in tiles are named by their slot (tagged) while the query runs
+// and mapped to their scene index once at its end; scenes with tiles have at
+// most kTileMaxSpheres + kBvhMaxBig spheres, so scene indices never carry the
+// tag.
+constexpr int32_t kLeafSlot = 0x40000000;
+
+struct BvhQuery {
+    uint32_t tests = 0;   // sphere tests
+    uint32_t boxes = 0;   // box tests
+    uint32_t exact = 0;   // orders settled by exact distances, exact loops
+};
+
+// min(a, b) as one v_min_f32.  fminf on a value carried around a loop costs a
+// canonicalising v_max_f32 besides the min; neither operand can be a
+// signalling NaN here (both come out of arithmetic), for which that
+// canonicalisation exists.
+__device__ __forceinline__ float bvh_min_raw(float a, float b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return __builtin_fminf(a, b);
+#endif
+}
 
 #if defined(__HIP_DEVICE_COMPILE__)
 #define TILE_CONST __attribute__((address_space(4)))
@@ -174,7 +218,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
         const int32_t id = B.big[j];
         tile_candidate(B, flat, flat((uint32_t)id), id, o, d, a, f, q);
     }
-    q.tests += B.tboxes ? B.n_big : n_all;   // without boxes every sphere is tested
+    q.tests += B.n_nodes ? B.n_big : n_all;   // without boxes every sphere is tested
 
     // the ray in tile units and its line's closest point to their origin
     const float ox = (o.x - B.cx) * B.ts, oy = (o.y - B.cy) * B.ts, oz = (o.z - B.cz) * B.ts;
@@ -246,7 +290,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
     const ATX_GLOBAL uint4* tiles = (const ATX_GLOBAL uint4*)(uintptr_t)B.tiles + lane;
     const ATX_GLOBAL float4* tsph = (const ATX_GLOBAL float4*)(uintptr_t)B.tsph;
     const uint32_t n_tiles = B.n_tiles;
-    const bool boxed = B.tboxes != nullptr, groups = n_tiles > kTileFlat;
+    const bool boxed = B.n_nodes != 0u, groups = n_tiles > kTileFlat;
     for (uint32_t t = 0; t < n_tiles;) {
         // candidates of up to kTileChunk touched tiles
         uint32_t nm = 0u, some = 0u;

@@ -107,7 +107,7 @@ struct WfScene {
     // least the list's (empty chunks past the list end the hand-out).
     const uint32_t* hit_px;
     uint32_t n_hit;
-    BvhDev bvh;            // n_nodes = 0: flat loop over all spheres
+    BvhDev bvh;            // n_tiles = 0: flat loop over all spheres
     UDiv div_group;        // by kJobGroupPx * frames (set by layout_launch)
     UDiv div_light;        // by max(n_light, 1) (set by layout_launch)
 };

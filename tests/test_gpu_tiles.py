@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kernel", [ATX_KERNEL_PLAIN, ATX_KERNEL_WAVEFRONT], ids=["plain", "wavefront"])
 @pytest.mark.parametrize("spheres,ground", [(16, False), (31, True), (32, True), (33, False), (65, True), (255, False),
-                                            (257, True), (512, True), (513, False), (545, True), (2049, True)])
+                                            (257, True), (512, True), (513, False), (545, True), (2049, True), (17000, True)])
 def test_tile_sizes_match_oracle(spheres, ground, kernel):
     ext = 20.0 * (spheres / 256.0) ** 0.5
     sph, mat, lig = random_scene(SplitMix64(spheres), spheres, 3, ext, (0.0, 6.0), (10.0, 20.0), ground=ground)
