@@ -99,7 +99,8 @@ struct Server {
     bool have_prev = false;         // the previous launch ran without an idle period since
     DevBuf table, queue_ctr, counters;
     DevBuf samples;                 // the tick's sample buffer (shared by the active requests)
-    size_t samples_excess = 0;      // its capacity beyond the active requests' shares, charged to hbm_in_use
+    size_t samples_shares = 0;      // the charged requests' shares of it
+    size_t samples_excess = 0;      // its capacity beyond those, charged to hbm_in_use
     double rendered = 0.0, busy_s = 0.0;   // samples rendered and GPU seconds so far (worker)
     // persistent grids: ticks with trees, flat-loop-only ticks
     uint32_t grid = 0, grid_flat = 0;
@@ -194,6 +195,17 @@ static bool admit(Server* s, Request& r)
     return true;
 }
 
+// Charges the budget with what the sample buffer holds beyond the shares of
+// the requests charged (admitted and not yet released, whether or not they
+// take part in the next launch).  Under s->mu, by the worker.
+static void charge_excess(Server* s)
+{
+    const size_t held = s->samples.bytes();
+    const size_t excess = held > s->samples_shares ? held - s->samples_shares : 0;
+    s->stats.hbm_in_use = s->stats.hbm_in_use - s->samples_excess + excess;
+    s->samples_excess = excess;
+}
+
 // Releases a request's device buffers.  A release waits for the device to
 // be idle, so only the worker calls it, between launches.
 static void release_device(Server* s, Request& r)
@@ -205,13 +217,11 @@ static void release_device(Server* s, Request& r)
     r.dirs.release();
     r.first.release();
     std::lock_guard<std::mutex> lk(s->mu);
-    // its share of the tick's sample buffer stays allocated: it becomes excess,
-    // so that nothing is admitted on bytes the buffer still holds
-    const size_t excess =
-        std::max(s->samples_excess,
-                 std::min(s->samples_excess + sample_share(r, s->cfg.frames_per_tick), s->samples.bytes()));
-    s->stats.hbm_in_use = s->stats.hbm_in_use - r.device_bytes + (excess - s->samples_excess);
-    s->samples_excess = excess;
+    // what the sample buffer still holds of its share becomes excess, so that
+    // nothing is admitted on it
+    s->stats.hbm_in_use -= r.device_bytes;
+    s->samples_shares -= sample_share(r, s->cfg.frames_per_tick);
+    charge_excess(s);
 }
 
 // Releases the device buffers of requests the retire thread has finished
@@ -298,8 +308,9 @@ static void admit_queued(Server* s)
             const size_t from_excess = std::min(s->samples_excess, sample_share(*r, F));
             if (s->stats.hbm_in_use + r->device_bytes - from_excess > s->cfg.hbm_budget_bytes) break;
             if (tick_paths + tick_paths_of(*r, F) >= kMaxTickPaths) break;   // 32-bit job indices
-            s->stats.hbm_in_use += r->device_bytes - from_excess;
-            s->samples_excess -= from_excess;
+            s->stats.hbm_in_use += r->device_bytes;
+            s->samples_shares += sample_share(*r, F);
+            charge_excess(s);
             s->stats.hbm_high_water = std::max(s->stats.hbm_high_water, s->stats.hbm_in_use);
             tick_paths += tick_paths_of(*r, F);
             newly.push_back(r);
@@ -376,20 +387,15 @@ static bool launch_tick(Server* s, std::vector<WfScene>& table, std::vector<std:
     WfPass wp{};
     // The buffer grows to the largest tick since the server last idled (a
     // hipFree and hipMalloc per shrink would stall the device between
-    // ticks).  Its capacity beyond the shares the active requests are
-    // charged (kSampleBytes per pixel and frame of a tick) is charged to the budget
+    // ticks).  Its capacity beyond the shares that requests are charged
+    // (kSampleBytes per pixel and frame of a tick) is charged to the budget
     // as well, so hbm_in_use counts every byte the server holds.
     const size_t need = std::max<size_t>(1, launch_samples(table.data(), table.size())) * kSampleBytes;
     bool ok = s->samples.reserve(need) == hipSuccess;
     {
-        size_t shares = 0;
-        for (auto& r : in_tick)
-            shares += (size_t)r->cam.width * r->cam.height * std::min<size_t>(F, r->spp) * kSampleBytes;
-        const size_t excess = s->samples.bytes() > shares ? s->samples.bytes() - shares : 0;
         std::lock_guard<std::mutex> lk(s->mu);
-        s->stats.hbm_in_use = s->stats.hbm_in_use - s->samples_excess + excess;
+        charge_excess(s);
         s->stats.hbm_high_water = std::max(s->stats.hbm_high_water, s->stats.hbm_in_use);
-        s->samples_excess = excess;
     }
     const bool flat = wf_flat_only(table.data(), table.size());
     const WfLaunch shape{flat ? s->grid_flat : s->grid, flat};
@@ -524,8 +530,7 @@ static void worker_main(Server* s)
             s->samples.release();  // and the tick's sample buffer, sized for ticks that have ended
             {
                 std::lock_guard<std::mutex> lk(s->mu);
-                s->stats.hbm_in_use -= s->samples_excess;
-                s->samples_excess = 0;
+                charge_excess(s);
             }
             admit_queued(s);
             s->have_prev = false;  // the device idled for want of work: no gap to count
