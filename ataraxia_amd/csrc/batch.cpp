@@ -77,7 +77,7 @@ static void drop_graph(Batch* b)
 
 static int enqueue_launches(Batch* b)
 {
-    ATX_HIP(launch_zero_u32(b->d_queue.as<unsigned int>(), b->launches, b->stream));
+    ATX_HIP(launch_zero_u32(b->d_queue.as<unsigned int>(), b->launches * kQueueWords, b->stream));
     for (uint32_t l = 0; l < b->launches; ++l) {
         WfPass wp{};
         wp.scenes = b->d_table.as<WfScene>() + b->launch_off[l];
@@ -85,7 +85,7 @@ static int enqueue_launches(Batch* b)
         wp.total_chunks = b->launch_chunks[l];
         wp.chunk_px = b->launch_chunk_px[l];
         wp.total_px = b->launch_px[l];
-        wp.queue = b->d_queue.as<unsigned int>() + l;
+        wp.queue = b->d_queue.as<unsigned int>() + l * kQueueWords;
         wp.counters = b->counters.as<unsigned long long>();
         ATX_HIP(launch_wavefront(wp, WfLaunch{b->grid, b->flat_only, b->tuning.waves_per_simd}, b->stream));
     }
@@ -106,7 +106,7 @@ static int batch_prepare(Batch* b, uint32_t max_frames)
     const size_t n = b->order.size();
     std::stable_sort(b->order.begin(), b->order.end(),
                      [b](uint32_t x, uint32_t y) { return b->scenes[x]->spp > b->scenes[y]->spp; });
-    b->chunk_px = b->tuning.chunk_px;   // 0: auto_chunk_px per launch
+    b->chunk_px = b->tuning.chunk_px;   // 0: launch_chunk_px per launch
     b->frames_per_launch = b->tuning.frames_per_launch ? b->tuning.frames_per_launch : kDefaultFramesPerLaunch;
     b->kahan = b->accumulator == ATX_ACCUM_KAHAN;
     b->flat_only = batch_flat_only(b);
@@ -177,7 +177,8 @@ static int batch_prepare(Batch* b, uint32_t max_frames)
     ATX_HIP(b->d_samples.reserve(std::max<size_t>(1, most) * kSampleBytes));
     for (size_t l = 0; l < b->launch_off.size(); ++l) {
         const WfScene* lt = table.data() + b->launch_off[l];
-        const uint32_t P = b->chunk_px ? b->chunk_px : auto_chunk_px(launch_jobs(lt, b->launch_scenes[l]), b->grid);
+        const uint32_t P = b->chunk_px ? b->chunk_px
+                                       : launch_chunk_px(launch_jobs(lt, b->launch_scenes[l]), b->grid, b->flat_only);
         WfPass lp{};
         if (!layout_launch(table.data() + b->launch_off[l], b->launch_scenes[l], P,
                            b->d_samples.as<float3>(), &lp)) {
@@ -193,7 +194,7 @@ static int batch_prepare(Batch* b, uint32_t max_frames)
     ATX_HIP(b->d_table.reserve(std::max<size_t>(1, table.size()) * sizeof(WfScene)));
     if (!table.empty())
         ATX_HIP(hipMemcpy(b->d_table.get(), table.data(), table.size() * sizeof(WfScene), hipMemcpyHostToDevice));
-    ATX_HIP(b->d_queue.reserve(std::max<uint32_t>(1, b->launches) * sizeof(unsigned int)));
+    ATX_HIP(b->d_queue.reserve(std::max<size_t>(1, b->launches) * kQueueWords * sizeof(unsigned int)));
     if (b->tuning.use_graph && b->launches) {
         ATX_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int rc = enqueue_launches(b);
@@ -222,7 +223,7 @@ int batch_run(Batch* b, uint32_t max_frames, double* ms_out)
         int rc = batch_prepare(b, max_frames);
         if (rc != ATX_OK) return rc;
     }
-    ATX_HIP(hipMemsetAsync(b->counters.get(), 0, kCtrCount * sizeof(unsigned long long), b->stream));
+    ATX_HIP(hipMemsetAsync(b->counters.get(), 0, kCounterBytes, b->stream));
     ATX_HIP(hipEventRecord(b->ev0, b->stream));
     if (b->exec) {
         ATX_HIP(hipGraphLaunch(b->exec, b->stream));
@@ -231,7 +232,7 @@ int batch_run(Batch* b, uint32_t max_frames, double* ms_out)
         if (rc != ATX_OK) return rc;
     }
     ATX_HIP(hipEventRecord(b->ev1, b->stream));
-    unsigned long long ctr[kCtrCount];
+    unsigned long long ctr[kCounterWords];
     ATX_HIP(hipMemcpyAsync(ctr, b->counters.get(), sizeof(ctr), hipMemcpyDeviceToHost, b->stream));
     ATX_HIP(hipStreamSynchronize(b->stream));
     float ms = 0.0f;
@@ -243,11 +244,11 @@ int batch_run(Batch* b, uint32_t max_frames, double* ms_out)
         samples += (uint64_t)e.cam.width * e.cam.height * frames;
     }
     b->stats.samples = samples;
-    b->stats.rays = ctr[kCtrRays] + ctr[kCtrReused] + b->skipped;
-    b->stats.reused_rays = ctr[kCtrReused] + b->skipped;
-    b->stats.sphere_tests = ctr[kCtrTests];
-    b->stats.exact_retraces = ctr[kCtrExact];
-    b->stats.box_tests = ctr[kCtrBoxes];
+    b->stats.reused_rays = counter_sum(ctr, kCtrReused) + b->skipped;
+    b->stats.rays = counter_sum(ctr, kCtrRays) + b->stats.reused_rays;
+    b->stats.sphere_tests = counter_sum(ctr, kCtrTests);
+    b->stats.exact_retraces = counter_sum(ctr, kCtrExact);
+    b->stats.box_tests = counter_sum(ctr, kCtrBoxes);
     b->stats.gpu_ms = ms;
     b->stats.launches = b->launches;
     b->stats.path_ms = 0.0;
@@ -325,7 +326,7 @@ int atx_batch_create(atx_batch** out)
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
-    if (e == hipSuccess) e = b->counters.reserve(kCtrCount * sizeof(unsigned long long));
+    if (e == hipSuccess) e = b->counters.reserve(kCounterBytes);
     if (e != hipSuccess) {
         set_error("batch create: %s", hipGetErrorString(e));
         atx_batch_destroy(reinterpret_cast<atx_batch*>(b));

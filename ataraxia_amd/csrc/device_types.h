@@ -19,7 +19,8 @@
 
 namespace atx {
 
-// Counters written by the kernels (device memory, u64 each).
+// Counters written by the kernels (device memory, u64 each, on kCounterLines
+// lines whose sums are the counts).
 enum CounterSlot : uint32_t {
     kCtrRays = 0,          // rays traced (continuation/primary + shadow)
     kCtrExact = 1,         // traces resolved by the exact fallback loop
@@ -28,5 +29,21 @@ enum CounterSlot : uint32_t {
     kCtrReused = 4,        // rays answered from the per-pixel first-bounce cache
     kCtrCount = 5,
 };
+// A wave adds to one line, with one request for all of its sums: every wave
+// adding each sum to a single line took 11.6 ns apiece, 4 x 7168 of them at
+// the end of a launch (1080p, one frame: path kernel 0.39 -> 0.27 ms;
+// 640x360, 4 spheres, 64 frames: 0.57 -> 0.44 ms).
+constexpr uint32_t kCounterLines = 16;
+constexpr uint32_t kCounterStride = 16;   // 128 bytes
+constexpr uint32_t kCounterWords = kCounterLines * kCounterStride;
+constexpr size_t kCounterBytes = kCounterWords * sizeof(unsigned long long);
+
+inline unsigned long long counter_sum(const unsigned long long* lines, CounterSlot k)
+{
+    unsigned long long s = 0;
+    for (uint32_t i = 0; i < kCounterLines; ++i)
+        s += lines[i * kCounterStride + k];
+    return s;
+}
 
 }  // namespace atx

@@ -30,7 +30,7 @@ namespace atx {
 namespace {
 
 constexpr size_t kScratchBytes = 8u << 20;   // per device: 8 MiB for the scene
-constexpr size_t kControlBytes = 4096;       // and a page for counters, queue and table entry
+constexpr size_t kControlBytes = 8192;       // and two pages for counters, queue and table entry
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes + kControlBytes];
@@ -94,9 +94,10 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     // scratch layout: spheres | material ids | materials | lights | tiles, then
     // past kScratchBytes counters | queue | table entry
     const size_t off_ctr = kScratchBytes;
-    const size_t off_queue = align256(off_ctr + kCtrCount * sizeof(unsigned long long));
-    const size_t off_table = align256(off_queue + sizeof(unsigned int));
-    static_assert(sizeof(WfScene) + 3 * 256 <= kControlBytes, "control page");
+    const size_t off_queue = align256(off_ctr + kCounterBytes);
+    const size_t off_table = align256(off_queue + kQueueWords * sizeof(unsigned int));
+    static_assert(kCounterBytes + kQueueWords * sizeof(unsigned int) + sizeof(WfScene) + 3 * 256 <= kControlBytes,
+                  "control pages");
     const size_t off_sph = 0;
     const size_t off_smat = align256(off_sph + L.sph.size() * 4);
     const size_t off_mat = align256(off_smat + L.sph_mat.size() * 4);
@@ -135,7 +136,7 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     ATX_HIP(put(off_tidx, T.tidx.data(), T.tidx.size() * 4));
     // the counters start at zero in every call (a fill kernel, not a memset node)
     ATX_HIP(launch_zero_u32(reinterpret_cast<unsigned int*>(base + off_ctr),
-                            (uint32_t)(kCtrCount * sizeof(unsigned long long) / 4), stream));
+                            (uint32_t)(kCounterBytes / 4), stream));
 
     WfScene w{};
     w.sph = reinterpret_cast<const float4*>(base + off_sph);
@@ -166,7 +167,7 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
         p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
         p.counters = reinterpret_cast<unsigned long long*>(base + off_ctr);
         ATX_HIP(put(off_table, &w, sizeof(w)));
-        ATX_HIP(launch_zero_u32(p.queue, 1, stream));
+        ATX_HIP(launch_zero_u32(p.queue, kQueueWords, stream));
         ATX_HIP(launch_in_place(p, w.bvh.n_tiles == 0, stream));
     }
     // the host copies above read L and T, which end with this call

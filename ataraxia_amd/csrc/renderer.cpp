@@ -45,7 +45,7 @@ struct Renderer {
     uint32_t n_hit = 0;
     bool n_hit_exact = false;
     DevBuf dbg_rad, dbg_hit, dbg_sh;   // debug capture buffers, reused across calls
-    uint32_t wf_chunk = 0;   // jobs per chunk; 0: auto_chunk_px per launch
+    uint32_t wf_chunk = 0;   // jobs per chunk; 0: launch_chunk_px per launch
     uint32_t wf_frames = kRendererFramesPerLaunch;
     uint32_t wf_waves = 0;   // path-kernel instance (resident waves per SIMD); 0: default
     DevBuf accum, comp, image, counters;
@@ -159,7 +159,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             if (use_first) use_hit_list(e, r->wf_first.get(), r->n_hit_exact ? r->n_hit : (uint32_t)npx);
             const uint64_t est =
                 e.hit_px && !r->n_hit_exact && r->n_hit ? (uint64_t)r->n_hit * e.frames : scene_jobs(e);
-            const uint32_t P = r->wf_chunk ? r->wf_chunk : auto_chunk_px(est, shape.workgroups);
+            const uint32_t P = r->wf_chunk ? r->wf_chunk : launch_chunk_px(est, shape.workgroups, shape.flat_only);
             launch_chunk.push_back(P);
             WfPass lp{};
             if (!layout_launch(&e, 1, P, r->wf_samples.as<float3>(), &lp)) {
@@ -194,12 +194,12 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     const uint32_t n_launch = (uint32_t)table.size();
     if (n_launch) {
         ATX_HIP(r->wf_table.reserve(n_launch * sizeof(WfScene)));
-        ATX_HIP(r->wf_queue.reserve(n_launch * sizeof(unsigned int)));
+        ATX_HIP(r->wf_queue.reserve(n_launch * kQueueWords * sizeof(unsigned int)));
         ATX_HIP(hipMemcpyAsync(r->wf_table.get(), table.data(), n_launch * sizeof(WfScene), hipMemcpyHostToDevice,
                                r->stream));
-        ATX_HIP(launch_zero_u32(r->wf_queue.as<unsigned int>(), n_launch, r->stream));
+        ATX_HIP(launch_zero_u32(r->wf_queue.as<unsigned int>(), n_launch * kQueueWords, r->stream));
     }
-    ATX_HIP(hipMemsetAsync(r->counters.get(), 0, kCtrCount * sizeof(unsigned long long), r->stream));
+    ATX_HIP(hipMemsetAsync(r->counters.get(), 0, kCounterBytes, r->stream));
     ATX_HIP(hipEventRecord(r->ev0, r->stream));
     if (wf) {
         for (size_t l = 0; l < table.size(); ++l) {
@@ -209,7 +209,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             wp.total_chunks = table[l].n_chunks;
             wp.chunk_px = launch_chunk[l];
             wp.total_px = table[l].width * table[l].height;
-            wp.queue = r->wf_queue.as<unsigned int>() + l;
+            wp.queue = r->wf_queue.as<unsigned int>() + l * kQueueWords;
             wp.counters = r->counters.as<unsigned long long>();
             ATX_HIP(hipEventRecord(r->wf_ev[2 * l], r->stream));
             ATX_HIP(launch_wavefront(wp, shape, r->stream, r->wf_ev[2 * l + 1]));
@@ -224,7 +224,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         for (uint32_t f = 0; f < frames; ++f) {
             WfPass wp = passes[f];
             wp.scenes = r->wf_table.as<WfScene>() + f;
-            wp.queue = r->wf_queue.as<unsigned int>() + f;
+            wp.queue = r->wf_queue.as<unsigned int>() + f * kQueueWords;
             wp.counters = r->counters.as<unsigned long long>();
             ATX_HIP(launch_in_place(wp, flat_only, r->stream));
             // Renderer.cu:245-248
@@ -234,10 +234,9 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     }
     ATX_HIP(hipEventRecord(r->ev1, r->stream));
     unsigned long long* ctr = r->readback;
-    ATX_HIP(hipMemcpyAsync(ctr, r->counters.get(), kCtrCount * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                           r->stream));
+    ATX_HIP(hipMemcpyAsync(ctr, r->counters.get(), kCounterBytes, hipMemcpyDeviceToHost, r->stream));
     const bool read_hits = use_first && !r->n_hit_exact;
-    uint32_t* n_hit_read = reinterpret_cast<uint32_t*>(r->readback + kCtrCount);
+    uint32_t* n_hit_read = reinterpret_cast<uint32_t*>(r->readback + kCounterWords);
     if (read_hits)
         ATX_HIP(hipMemcpyAsync(n_hit_read, first_cache_view(r->wf_first.get(), npx, r->geo.n_light).n_hits,
                                sizeof(uint32_t), hipMemcpyDeviceToHost, r->stream));
@@ -264,11 +263,11 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         if (e.hit_px) e.n_hit = r->n_hit;
     r->stats.samples = (uint64_t)npx * frames;
     const uint64_t skipped = wf ? skipped_primaries(table.data(), table.size()) : 0;
-    r->stats.rays = ctr[kCtrRays] + ctr[kCtrReused] + skipped;
-    r->stats.reused_rays = ctr[kCtrReused] + skipped;
-    r->stats.sphere_tests = ctr[kCtrTests];
-    r->stats.exact_retraces = ctr[kCtrExact];
-    r->stats.box_tests = ctr[kCtrBoxes];
+    r->stats.reused_rays = counter_sum(ctr, kCtrReused) + skipped;
+    r->stats.rays = counter_sum(ctr, kCtrRays) + r->stats.reused_rays;
+    r->stats.sphere_tests = counter_sum(ctr, kCtrTests);
+    r->stats.exact_retraces = counter_sum(ctr, kCtrExact);
+    r->stats.box_tests = counter_sum(ctr, kCtrBoxes);
     r->stats.gpu_ms = ms;
     r->stats.launches = wf ? table.size() : frames;
     r->stats.path_ms = path_ms;
@@ -295,9 +294,9 @@ int atx_renderer_create(atx_renderer** out)
     hipError_t e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&r->ev0);
     if (e == hipSuccess) e = hipEventCreate(&r->ev1);
-    if (e == hipSuccess) e = r->counters.reserve(kCtrCount * sizeof(unsigned long long));
+    if (e == hipSuccess) e = r->counters.reserve(kCounterBytes);
     if (e == hipSuccess)
-        e = hipHostMalloc((void**)&r->readback, (kCtrCount + 1) * sizeof(unsigned long long), hipHostMallocDefault);
+        e = hipHostMalloc((void**)&r->readback, (kCounterWords + 1) * sizeof(unsigned long long), hipHostMallocDefault);
     if (e != hipSuccess) {
         set_error("renderer create: %s", hipGetErrorString(e));
         atx_renderer_destroy(reinterpret_cast<atx_renderer*>(r));

@@ -400,12 +400,13 @@ static bool launch_tick(Server* s, std::vector<WfScene>& table, std::vector<std:
     const bool flat = wf_flat_only(table.data(), table.size());
     const WfLaunch shape{flat ? s->grid_flat : s->grid, flat};
     const uint32_t P =
-        s->cfg.chunk_px ? s->cfg.chunk_px : auto_chunk_px(launch_jobs(table.data(), table.size()), shape.workgroups);
+        s->cfg.chunk_px ? s->cfg.chunk_px
+                        : launch_chunk_px(launch_jobs(table.data(), table.size()), shape.workgroups, flat);
     if (ok) ok = layout_launch(table.data(), table.size(), P, s->samples.as<float3>(), &wp);
     ok = ok && s->table.reserve(table.size() * sizeof(WfScene)) == hipSuccess &&
          hipMemcpyAsync(s->table.get(), table.data(), table.size() * sizeof(WfScene), hipMemcpyHostToDevice,
                         s->stream) == hipSuccess &&
-         launch_zero_u32(s->queue_ctr.as<unsigned int>(), 1, s->stream) == hipSuccess &&
+         launch_zero_u32(s->queue_ctr.as<unsigned int>(), kQueueWords, s->stream) == hipSuccess &&
          hipEventRecord(s->ev0, s->stream) == hipSuccess;
     if (ok) {
         wp.scenes = s->table.as<WfScene>();
@@ -598,9 +599,9 @@ int atx_server_create(atx_server** out, const atx_server_config* cfg)
     ATX_HIP(hipEventCreate(&s->ev0));
     ATX_HIP(hipEventCreate(&s->ev1));
     ATX_HIP(hipEventCreate(&s->ev_prev));
-    ATX_HIP(s->queue_ctr.reserve(256));
-    ATX_HIP(s->counters.reserve(kCtrCount * sizeof(unsigned long long)));
-    ATX_HIP(hipMemset(s->counters.get(), 0, kCtrCount * sizeof(unsigned long long)));
+    ATX_HIP(s->queue_ctr.reserve(kQueueWords * sizeof(unsigned int)));
+    ATX_HIP(s->counters.reserve(kCounterBytes));
+    ATX_HIP(hipMemset(s->counters.get(), 0, kCounterBytes));
     s->grid = wavefront_full_grid(false);
     s->grid_flat = wavefront_full_grid(true);
     s->epoch = std::chrono::steady_clock::now();

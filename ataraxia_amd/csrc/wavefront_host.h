@@ -181,18 +181,33 @@ inline bool wf_flat_only(const WfScene* tab, size_t n)
     return true;
 }
 
-// Jobs per chunk for a launch of `jobs` jobs on a persistent grid of
-// `workgroups` (4 waves each) when the caller gives none.  Small chunks share
-// the launch out evenly to the end; large ones keep a wave on neighbouring
-// pixels (and in a many-frame launch on the same pixel) and fetch fewer
-// blocks.  Measured on the 1080p workload (1 to 64 frames per launch, chunks
-// of 64 to 1024 jobs, both kernel instances): 512 jobs from about 5000 jobs
-// per wave on (16 frames and more), 256 below; within 6 % of the best chunk
-// at every frame count.
+// Jobs per chunk of a long launch: 512 from about 5000 jobs per wave on (4
+// waves per workgroup), 256 below.
 inline uint32_t auto_chunk_px(uint64_t jobs, uint32_t workgroups)
 {
     const uint64_t per_wave = jobs / (4ull * (workgroups ? workgroups : 1u));
     return per_wave >= 5000u ? 512u : 256u;
+}
+
+// Jobs per chunk for a launch of `jobs` jobs on a persistent grid of
+// `workgroups` when the caller gives none.  Small chunks share a launch out
+// evenly to the end and give more waves work at its start; large ones keep a
+// wave on neighbouring pixels (and in a many-frame launch on the same pixel).
+// The steps follow the jobs per wave; path kernel ms at 64, 128, 256 and 512
+// jobs per chunk:
+//   tiles, 300 spheres: 320x180 (11 per wave) .085 .130 .189 .335; 1920x1080
+//     (405) .324 .339 .355 .445; 640x360, 16 frames (720) .359 .347 .358
+//     .415; 64 frames (2880) .831 .812 .837 .888; 1280x720, 64 frames (11520)
+//     2.70 2.57 2.50 2.53; 1920x1080, 256 frames (104000) - 21.9 21.1 20.7
+//   flat, 4 spheres: 320x180 (8) .035 .057 .079 .129; 640x360 (32) .068 .064
+//     .081 .125; 1280x720 (129) .153 .144 .114 .141; 1920x1080 (289) .202
+//     .202 .192 .170; 640x360, 64 frames (2057) .495 .483 .452 .429
+inline uint32_t launch_chunk_px(uint64_t jobs, uint32_t workgroups, bool flat_only)
+{
+    const uint64_t per_wave = jobs / (4ull * (workgroups ? workgroups : 1u));
+    if (per_wave < (flat_only ? 16u : 512u)) return 64u;
+    if (per_wave < (flat_only ? 64u : 4000u)) return 128u;
+    return flat_only && per_wave >= 256u ? 512u : auto_chunk_px(jobs, workgroups);
 }
 
 // Frames per launch of batches and serving ticks (each scene or request
