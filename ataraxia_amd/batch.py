@@ -107,13 +107,13 @@ class Batch:
 
     def get_image(self, scene_id: int) -> np.ndarray:
         sc = self.scenes[scene_id]
-        img = np.zeros(sc.camera.width * sc.camera.height, np.uint32)
+        img = np.empty(sc.camera.width * sc.camera.height, np.uint32)
         check(lib.atx_batch_get_image(self._h, scene_id, ptr(img), img.size))
         return img.reshape(sc.camera.height, sc.camera.width)
 
     def get_accumulation(self, scene_id: int) -> np.ndarray:
         sc = self.scenes[scene_id]
-        acc = np.zeros(sc.camera.width * sc.camera.height * 4, np.float32)
+        acc = np.empty(sc.camera.width * sc.camera.height * 4, np.float32)
         check(lib.atx_batch_get_accumulation(self._h, scene_id, ptr(acc), acc.size))
         return acc.reshape(sc.camera.height, sc.camera.width, 4)
 

@@ -48,6 +48,7 @@ struct Batch {
     int accel = ATX_ACCEL_BVH;
     atx_batch_tuning tuning{0, 0, 1, 0, 0};
     DevBuf d_table, d_queue, counters;
+    HostStage results;
     std::vector<uint32_t> order;          // table position -> scene id
     std::vector<uint32_t> launch_off;     // first table entry of launch l
     std::vector<uint32_t> launch_scenes;  // scenes taking part in launch l
@@ -475,7 +476,7 @@ int atx_batch_get_image(atx_batch* h, uint32_t scene_id, uint32_t* rgba, uint64_
     if (!e) return ATX_ERR_NOTFOUND;
     const uint64_t npx = (uint64_t)e->cam.width * e->cam.height;
     ATX_CHECK_ARG(rgba && n >= npx, "buffer too small (%llu < %llu)", (unsigned long long)n, (unsigned long long)npx);
-    ATX_HIP(hipMemcpy(rgba, e->image.get(), npx * 4, hipMemcpyDeviceToHost));
+    ATX_HIP(b->results.copy_out(rgba, e->image.get(), npx * 4, b->stream));
     return ATX_OK;
 }
 
@@ -486,7 +487,7 @@ int atx_batch_get_accumulation(atx_batch* h, uint32_t scene_id, float* rgba, uin
     if (!e) return ATX_ERR_NOTFOUND;
     const uint64_t nf = 4ull * e->cam.width * e->cam.height;
     ATX_CHECK_ARG(rgba && n >= nf, "buffer too small (%llu < %llu)", (unsigned long long)n, (unsigned long long)nf);
-    ATX_HIP(hipMemcpy(rgba, e->accum.get(), nf * 4, hipMemcpyDeviceToHost));
+    ATX_HIP(b->results.copy_out(rgba, e->accum.get(), nf * 4, b->stream));
     return ATX_OK;
 }
 

@@ -73,59 +73,47 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l)
 {
-    return (16 * n + 16) + (4 * n + 16) + (48 * m + 16) + (16 * m + 16) + (32 * l + 16) + bvh_device_bytes(n);
+    return 16 * n + 4 * n + 48 * m + 16 * m + 32 * l + bvh_device_bytes(n) + (ScenePack::kArrays + 1) * 256;
 }
 
-int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
-                 const atx_light* lights, uint64_t l, DevScene* out)
+ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T)
 {
-    HostSceneLayout L;
-    int rc = build_scene_layout(spheres, n, materials, m, lights, l, &L);
-    if (rc != ATX_OK) return rc;
-    ATX_HIP(out->sph.reserve(L.sph.size() * 4 + 16));
-    ATX_HIP(out->sph_mat.reserve(L.sph_mat.size() * 4 + 16));
-    ATX_HIP(out->mat.reserve(L.mat.size() * 4 + 16));
-    ATX_HIP(out->mat_rr.reserve(L.mat_rr.size() * 4 + 16));
-    ATX_HIP(out->light.reserve(L.light.size() * 4 + 16));
-    if (!L.sph.empty()) ATX_HIP(hipMemcpy(out->sph.get(), L.sph.data(), L.sph.size() * 4, hipMemcpyHostToDevice));
-    if (!L.sph_mat.empty())
-        ATX_HIP(hipMemcpy(out->sph_mat.get(), L.sph_mat.data(), L.sph_mat.size() * 4, hipMemcpyHostToDevice));
-    if (!L.mat.empty()) ATX_HIP(hipMemcpy(out->mat.get(), L.mat.data(), L.mat.size() * 4, hipMemcpyHostToDevice));
-    if (!L.mat_rr.empty())
-        ATX_HIP(hipMemcpy(out->mat_rr.get(), L.mat_rr.data(), L.mat_rr.size() * 4, hipMemcpyHostToDevice));
-    if (!L.light.empty())
-        ATX_HIP(hipMemcpy(out->light.get(), L.light.data(), L.light.size() * 4, hipMemcpyHostToDevice));
-    out->n_sph = (uint32_t)n;
-    out->n_mat = (uint32_t)m;
-    out->n_light = (uint32_t)l;
-
-    HostBvh T;
-    build_bvh(L.sph.data(), (uint32_t)n, 0, &T);
-    out->bvh = BvhDev{};
-    if (T.n_tiles > 0) {
-        const auto put = [](DevBuf& b, const void* src, size_t bytes) -> hipError_t {
-            const hipError_t e = b.reserve(bytes + 16);
-            return e != hipSuccess || bytes == 0 ? e : hipMemcpy(b.get(), src, bytes, hipMemcpyHostToDevice);
-        };
-        ATX_HIP(put(out->big, T.big.data(), T.big.size() * 4));
-        ATX_HIP(put(out->tiles, T.tiles.data(), T.tiles.size() * 4));
-        ATX_HIP(put(out->tile_boxes, T.tboxes.data(), T.tboxes.size() * 4));
-        ATX_HIP(put(out->tile_sph, T.tsph.data(), T.tsph.size() * 4));
-        ATX_HIP(put(out->tile_idx, T.tidx.data(), T.tidx.size() * 4));
-        out->bvh = bvh_dev_from(T, {out->big.get(), out->tiles.get(), out->tile_boxes.get(), out->tile_sph.get(),
-                                    out->tile_idx.get()});
-    }
-    return ATX_OK;
+    const auto put = [this](Array a, const auto& v) {
+        off[a] = bytes;
+        src[a] = v.data();
+        src_bytes[a] = v.size() * 4;
+        bytes += (src_bytes[a] + 255) & ~size_t(255);
+    };
+    bytes = 0;
+    put(kSph, L.sph);
+    put(kSphMat, L.sph_mat);
+    put(kMat, L.mat);
+    put(kLight, L.light);
+    put(kBig, T.big);
+    put(kTiles, T.tiles);
+    put(kTileBoxes, T.tboxes);
+    put(kTileSph, T.tsph);
+    put(kTileIdx, T.tidx);
+    put(kMatRr, L.mat_rr);
 }
 
-BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at)
+std::vector<unsigned char> ScenePack::block() const
+{
+    std::vector<unsigned char> b(bytes);
+    for (int a = 0; a < kArrays; ++a)
+        if (src_bytes[a]) memcpy(b.data() + off[a], src[a], src_bytes[a]);
+    return b;
+}
+
+BvhDev ScenePack::bvh(const HostBvh& T, const void* base) const
 {
     BvhDev b{};
-    b.tiles = static_cast<const uint4*>(at.tiles);
-    b.tboxes = static_cast<const float4*>(at.tboxes);
-    b.tsph = static_cast<const float4*>(at.tsph);
-    b.tidx = static_cast<const int32_t*>(at.tidx);
-    b.big = static_cast<const int32_t*>(at.big);
+    if (T.n_tiles == 0) return b;
+    b.tiles = at<uint4>(base, kTiles);
+    b.tboxes = at<float4>(base, kTileBoxes);
+    b.tsph = at<float4>(base, kTileSph);
+    b.tidx = at<int32_t>(base, kTileIdx);
+    b.big = at<int32_t>(base, kBig);
     b.n_tiles = T.n_tiles;
     b.n_nodes = (uint32_t)(T.tboxes.size() / 8);
     b.n_big = (uint32_t)T.big.size();
@@ -135,6 +123,31 @@ BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at)
     b.ts = T.ts;
     b.t_lin = T.t_lin;
     return b;
+}
+
+int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
+                 const atx_light* lights, uint64_t l, DevScene* out)
+{
+    HostSceneLayout L;
+    int rc = build_scene_layout(spheres, n, materials, m, lights, l, &L);
+    if (rc != ATX_OK) return rc;
+    HostBvh T;
+    build_bvh(L.sph.data(), (uint32_t)n, 0, &T);
+    const ScenePack pack(L, T);
+    // never an empty block: the kernels' pointers stay valid without spheres
+    ATX_HIP(out->block.reserve(pack.bytes + 256));
+    if (pack.bytes) ATX_HIP(hipMemcpy(out->block.get(), pack.block().data(), pack.bytes, hipMemcpyHostToDevice));
+    const void* base = out->block.get();
+    out->sph = pack.at<float4>(base, ScenePack::kSph);
+    out->sph_mat = pack.at<int32_t>(base, ScenePack::kSphMat);
+    out->mat = pack.at<float4>(base, ScenePack::kMat);
+    out->mat_rr = pack.at<float4>(base, ScenePack::kMatRr);
+    out->light = pack.at<float4>(base, ScenePack::kLight);
+    out->n_sph = (uint32_t)n;
+    out->n_mat = (uint32_t)m;
+    out->n_light = (uint32_t)l;
+    out->bvh = pack.bvh(T, base);
+    return ATX_OK;
 }
 
 }  // namespace atx

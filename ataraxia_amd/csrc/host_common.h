@@ -15,6 +15,8 @@
 
 #include "../../include/atx.h"
 #include "bvh.h"
+#include "bvh_build.h"
+#include "host_transfer.h"
 
 namespace atx {
 
@@ -172,23 +174,35 @@ struct HostSceneLayout {
 int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material* materials,
                        uint64_t m, const atx_light* lights, uint64_t l, HostSceneLayout* out);
 
+// The arrays of a scene and its tiles laid out in one block, each from a
+// multiple of 256 bytes on, so that they go to the device in one copy (ten
+// copies, each waited for, took about 110 us).
+struct ScenePack {
+    enum Array { kSph, kSphMat, kMat, kLight, kBig, kTiles, kTileBoxes, kTileSph, kTileIdx, kMatRr, kArrays };
+    size_t off[kArrays];
+    size_t bytes;   // a multiple of 256
+    const void* src[kArrays];
+    size_t src_bytes[kArrays];
+    ScenePack(const HostSceneLayout& L, const HostBvh& T);
+    std::vector<unsigned char> block() const;
+    // the kernel's view of T, whose arrays are in the block at `base`
+    BvhDev bvh(const HostBvh& T, const void* base) const;
+    template <class X> const X* at(const void* base, Array a) const
+    {
+        return reinterpret_cast<const X*>(static_cast<const unsigned char*>(base) + off[a]);
+    }
+};
+
 // One scene's geometry in HBM (device layout of device_types.h), with its
 // tiles (bvh.h; bvh.n_tiles = 0 when the scene has none).
 struct DevScene {
-    DevBuf sph, sph_mat, mat, mat_rr, light;
-    DevBuf big, tiles, tile_boxes, tile_sph, tile_idx;
+    DevBuf block;   // ScenePack
+    const float4 *sph = nullptr, *mat = nullptr, *mat_rr = nullptr, *light = nullptr;
+    const int32_t* sph_mat = nullptr;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
     BvhDev bvh{};
-    void use_pool(DevPool* pool)
-    {
-        for (DevBuf* b : {&sph, &sph_mat, &mat, &mat_rr, &light, &big, &tiles, &tile_boxes, &tile_sph, &tile_idx})
-            b->use_pool(pool);
-    }
-    size_t bytes() const
-    {
-        return sph.bytes() + sph_mat.bytes() + mat.bytes() + mat_rr.bytes() + light.bytes() + big.bytes() +
-               tiles.bytes() + tile_boxes.bytes() + tile_sph.bytes() + tile_idx.bytes();
-    }
+    void use_pool(DevPool* pool) { block.use_pool(pool); }
+    size_t bytes() const { return block.bytes(); }
     // The tiles to hand to a kernel; for ATX_ACCEL_NONE without their boxes, so
     // that every ray tests every sphere.
     BvhDev accel(int mode) const
@@ -202,13 +216,6 @@ struct DevScene {
 // Validates, converts and uploads (synchronously) a flattened scene.
 int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
                  const atx_light* lights, uint64_t l, DevScene* out);
-
-// Kernel view of host-built tiles whose arrays were copied to the given
-// device addresses.
-struct BvhArrays {
-    const void *big, *tiles, *tboxes, *tsph, *tidx;
-};
-BvhDev bvh_dev_from(const HostBvh& T, const BvhArrays& at);
 
 // Device bytes a scene of this size occupies (geometry and tree).
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l);

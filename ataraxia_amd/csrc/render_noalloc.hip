@@ -98,16 +98,9 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     const size_t off_table = align256(off_queue + kQueueWords * sizeof(unsigned int));
     static_assert(kCounterBytes + kQueueWords * sizeof(unsigned int) + sizeof(WfScene) + 3 * 256 <= kControlBytes,
                   "control pages");
-    const size_t off_sph = 0;
-    const size_t off_smat = align256(off_sph + L.sph.size() * 4);
-    const size_t off_mat = align256(off_smat + L.sph_mat.size() * 4);
-    const size_t off_light = align256(off_mat + L.mat.size() * 4);
-    const size_t off_big = align256(off_light + L.light.size() * 4);
-    const size_t off_tiles = align256(off_big + T.big.size() * 4);
-    const size_t off_boxes = align256(off_tiles + T.tiles.size() * 4);
-    const size_t off_tsph = align256(off_boxes + T.tboxes.size() * 4);
-    const size_t off_tidx = align256(off_tsph + T.tsph.size() * 4);
-    const size_t total = align256(off_tidx + T.tidx.size() * 4);
+    L.mat_rr.clear();   // the in-place kernel takes no first-hit roulette from it
+    const ScenePack pack(L, T);
+    const size_t total = pack.bytes;
     if (total > kScratchBytes) {
         set_error("scene needs %zu bytes of device scratch; atx_render_frames_noalloc holds at most %zu "
                   "(use atx_renderer_* for larger scenes)",
@@ -125,29 +118,21 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     auto put = [&](size_t off, const void* src, size_t bytes) -> hipError_t {
         return bytes ? hipMemcpyAsync(base + off, src, bytes, hipMemcpyHostToDevice, stream) : hipSuccess;
     };
-    ATX_HIP(put(off_sph, L.sph.data(), L.sph.size() * 4));
-    ATX_HIP(put(off_smat, L.sph_mat.data(), L.sph_mat.size() * 4));
-    ATX_HIP(put(off_mat, L.mat.data(), L.mat.size() * 4));
-    ATX_HIP(put(off_light, L.light.data(), L.light.size() * 4));
-    ATX_HIP(put(off_big, T.big.data(), T.big.size() * 4));
-    ATX_HIP(put(off_tiles, T.tiles.data(), T.tiles.size() * 4));
-    ATX_HIP(put(off_boxes, T.tboxes.data(), T.tboxes.size() * 4));
-    ATX_HIP(put(off_tsph, T.tsph.data(), T.tsph.size() * 4));
-    ATX_HIP(put(off_tidx, T.tidx.data(), T.tidx.size() * 4));
+    const std::vector<unsigned char> block = pack.block();
+    ATX_HIP(put(0, block.data(), block.size()));
     // the counters start at zero in every call (a fill kernel, not a memset node)
     ATX_HIP(launch_zero_u32(reinterpret_cast<unsigned int*>(base + off_ctr),
                             (uint32_t)(kCounterBytes / 4), stream));
 
     WfScene w{};
-    w.sph = reinterpret_cast<const float4*>(base + off_sph);
-    w.sph_mat = reinterpret_cast<const int32_t*>(base + off_smat);
-    w.mat = reinterpret_cast<const float4*>(base + off_mat);
-    w.light = reinterpret_cast<const float4*>(base + off_light);
+    w.sph = pack.at<float4>(base, ScenePack::kSph);
+    w.sph_mat = pack.at<int32_t>(base, ScenePack::kSphMat);
+    w.mat = pack.at<float4>(base, ScenePack::kMat);
+    w.light = pack.at<float4>(base, ScenePack::kLight);
     w.n_sph = (uint32_t)num_spheres;
     w.n_mat = (uint32_t)num_materials;
     w.n_light = (uint32_t)num_lights;
-    if (T.n_tiles > 0)
-        w.bvh = bvh_dev_from(T, {base + off_big, base + off_tiles, base + off_boxes, base + off_tsph, base + off_tidx});
+    w.bvh = pack.bvh(T, base);
     if (accel != ATX_ACCEL_BVH) w.bvh.n_nodes = 0;
     const bool kahan = accumulator == ATX_ACCUM_KAHAN;
     // one launch for all frames; with accumulation off a launch per frame, the

@@ -49,6 +49,7 @@ struct Renderer {
     uint32_t wf_frames = kRendererFramesPerLaunch;
     uint32_t wf_waves = 0;   // path-kernel instance (resident waves per SIMD); 0: default
     DevBuf accum, comp, image, counters;
+    HostStage results;
     // pinned host memory the call's statistics are copied into (counters,
     // then the hit list's length): copies into pageable memory block the
     // host until the stream is idle, one after the other
@@ -481,8 +482,7 @@ int atx_renderer_get_image(atx_renderer* h, uint32_t* rgba, uint64_t n)
     ATX_CHECK_ARG(n >= npx, "buffer holds %llu pixels, image has %llu", (unsigned long long)n,
                   (unsigned long long)npx);
     if (npx == 0) return ATX_OK;
-    ATX_HIP(hipMemcpyAsync(rgba, r->image.get(), npx * 4, hipMemcpyDeviceToHost, r->stream));
-    ATX_HIP(hipStreamSynchronize(r->stream));
+    ATX_HIP(r->results.copy_out(rgba, r->image.get(), npx * 4, r->stream));
     return ATX_OK;
 }
 
@@ -493,8 +493,7 @@ int atx_renderer_get_accumulation(atx_renderer* h, float* rgba, uint64_t n)
     const uint64_t nf = 4ull * r->width * r->height;
     ATX_CHECK_ARG(n >= nf, "buffer holds %llu floats, need %llu", (unsigned long long)n, (unsigned long long)nf);
     if (nf == 0) return ATX_OK;
-    ATX_HIP(hipMemcpyAsync(rgba, r->accum.get(), nf * 4, hipMemcpyDeviceToHost, r->stream));
-    ATX_HIP(hipStreamSynchronize(r->stream));
+    ATX_HIP(r->results.copy_out(rgba, r->accum.get(), nf * 4, r->stream));
     return ATX_OK;
 }
 

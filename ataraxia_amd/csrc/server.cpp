@@ -59,8 +59,7 @@ struct Request {
     uint32_t n_hit = 0;             // pixels of its hit list
     uint32_t frames_done = 0;
     // results
-    std::vector<uint32_t> rgba;
-    std::vector<float> acc_host;
+    HostMem rgba, acc_host;         // image, accumulation
     int state = ATX_REQ_QUEUED;
     double t_submit = 0, t_admit = 0, t_done = 0;
     std::string error;
@@ -95,6 +94,10 @@ struct Server {
     // stream, beside the running launch; the worker waits for them (not for
     // the launch) to read the caches' hit counts
     hipStream_t adm_stream = nullptr;
+    // the retire thread's: results leave beside the running launch (the launch
+    // that wrote them has been waited for); made with the first result
+    hipStream_t out_stream = nullptr;
+    HostStage results;
     bool no_hit_lists = false;      // a hit count could not be read: jobs cover every pixel
     bool have_prev = false;         // the previous launch ran without an idle period since
     DevBuf table, queue_ctr, counters;
@@ -250,10 +253,12 @@ static void finish(Server* s, const std::shared_ptr<Request>& rp, bool ok, bool 
     Request& r = *rp;
     const size_t npx = (size_t)r.cam.width * r.cam.height;
     if (ok) {
-        r.rgba.resize(npx);
-        r.acc_host.resize(4 * npx);
-        if (hipMemcpy(r.rgba.data(), r.image.get(), npx * 4, hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(r.acc_host.data(), r.accum.get(), npx * 16, hipMemcpyDeviceToHost) != hipSuccess) {
+        r.rgba = host_alloc(npx * 4);
+        r.acc_host = host_alloc(npx * 16);
+        if (!r.rgba || !r.acc_host ||
+            (!s->out_stream && hipStreamCreateWithFlags(&s->out_stream, hipStreamNonBlocking) != hipSuccess) ||
+            s->results.copy_out(r.rgba.get(), r.image.get(), npx * 4, s->out_stream) != hipSuccess ||
+            s->results.copy_out(r.acc_host.get(), r.accum.get(), npx * 16, s->out_stream) != hipSuccess) {
             ok = false;
             r.error = "result copy failed";
         }
@@ -656,6 +661,7 @@ int atx_server_destroy(atx_server* h)
     if (s->ev_prev) (void)hipEventDestroy(s->ev_prev);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     if (s->adm_stream) (void)hipStreamDestroy(s->adm_stream);
+    if (s->out_stream) (void)hipStreamDestroy(s->out_stream);
     delete s;
     return ATX_OK;
 }
@@ -752,26 +758,35 @@ int atx_server_get_result(atx_server* h, uint64_t id, uint32_t* rgba, uint64_t n
 {
     Server* s = cast(h);
     ATX_CHECK_ARG(s, "server is NULL");
-    std::lock_guard<std::mutex> lk(s->mu);
-    auto it = s->all.find(id);
-    if (it == s->all.end()) {
-        set_error("unknown request %llu", (unsigned long long)id);
-        return ATX_ERR_NOTFOUND;
+    std::shared_ptr<Request> r;
+    {
+        std::lock_guard<std::mutex> lk(s->mu);
+        auto it = s->all.find(id);
+        if (it == s->all.end()) {
+            set_error("unknown request %llu", (unsigned long long)id);
+            return ATX_ERR_NOTFOUND;
+        }
+        r = it->second;
+        if (r->state != ATX_REQ_DONE) {
+            set_error("request %llu is not done", (unsigned long long)id);
+            return ATX_ERR_STATE;
+        }
     }
-    Request& r = *it->second;
-    if (r.state != ATX_REQ_DONE) {
-        set_error("request %llu is not done", (unsigned long long)id);
-        return ATX_ERR_STATE;
-    }
+    // a finished request's results do not change: copied without the lock,
+    // which the worker needs to start its next launch
+    const size_t npx = (size_t)r->cam.width * r->cam.height;
     if (rgba) {
-        ATX_CHECK_ARG(num_pixels >= r.rgba.size(), "rgba buffer too small");
-        std::copy(r.rgba.begin(), r.rgba.end(), rgba);
+        ATX_CHECK_ARG(num_pixels >= npx, "rgba buffer too small");
+        copy_threaded(rgba, r->rgba.get(), npx * 4);
     }
     if (accum) {
-        ATX_CHECK_ARG(num_floats >= r.acc_host.size(), "accum buffer too small");
-        std::copy(r.acc_host.begin(), r.acc_host.end(), accum);
+        ATX_CHECK_ARG(num_floats >= 4 * npx, "accum buffer too small");
+        copy_threaded(accum, r->acc_host.get(), npx * 16);
     }
-    if (release) s->all.erase(it);
+    if (release) {
+        std::lock_guard<std::mutex> lk(s->mu);
+        s->all.erase(id);
+    }
     return ATX_OK;
 }
 

@@ -37,11 +37,11 @@ inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_c
                           int accel, WfScene* out)
 {
     memset(out, 0, sizeof(*out));
-    out->sph = g.sph.as<float4>();
-    out->sph_mat = g.sph_mat.as<int32_t>();
-    out->mat = g.mat.as<float4>();
-    out->mat_rr = g.mat_rr.as<float4>();
-    out->light = g.light.as<float4>();
+    out->sph = g.sph;
+    out->sph_mat = g.sph_mat;
+    out->mat = g.mat;
+    out->mat_rr = g.mat_rr;
+    out->light = g.light;
     out->n_sph = g.n_sph;
     out->n_mat = g.n_mat;
     out->n_light = g.n_light;

@@ -115,12 +115,12 @@ class Renderer:
 
     # -- outputs -------------------------------------------------------------------
     def get_image(self) -> np.ndarray:
-        img = np.zeros(self.width * self.height, dtype=np.uint32)
+        img = np.empty(self.width * self.height, dtype=np.uint32)
         check(lib.atx_renderer_get_image(self._h, ptr(img), img.size))
         return img.reshape(self.height, self.width)
 
     def get_accumulation(self) -> np.ndarray:
-        acc = np.zeros(self.width * self.height * 4, dtype=np.float32)
+        acc = np.empty(self.width * self.height * 4, dtype=np.float32)
         check(lib.atx_renderer_get_accumulation(self._h, ptr(acc), acc.size))
         return acc.reshape(self.height, self.width, 4)
 

@@ -77,8 +77,8 @@ class Server:
 
     def result(self, rid: int, release: bool = False):
         w, h = self.sizes[rid]
-        img = np.zeros(w * h, np.uint32)
-        acc = np.zeros(w * h * 4, np.float32)
+        img = np.empty(w * h, np.uint32)
+        acc = np.empty(w * h * 4, np.float32)
         check(lib.atx_server_get_result(self._h, rid, ptr(img), img.size, ptr(acc), acc.size, 1 if release else 0))
         return img.reshape(h, w), acc.reshape(h, w, 4)
 
