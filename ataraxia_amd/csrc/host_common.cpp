@@ -60,6 +60,12 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
         const f3 tp = divs(albedo, p);
         float* r = &out->mat_rr[4 * i];
         r[0] = tp.x; r[1] = tp.y; r[2] = tp.z; r[3] = p;
+        const float in_unit[] = {a.albedo[0], a.albedo[1], a.albedo[2], a.F0[0], a.F0[1], a.F0[2], a.metallic, a.roughness};
+        for (float v : in_unit)
+            if (!(v >= 0.0f && v <= 1.0f)) out->unit_materials = false;
+        if (a.roughness > 0.0f && a.roughness < 0x1p-10f) out->unit_materials = false;
+        for (int k = 0; k < 3; ++k)
+            if (a.albedo[k] > 0.0f && a.albedo[k] < out->least_albedo) out->least_albedo = a.albedo[k];
     }
     out->light.resize(8 * l);
     for (uint64_t i = 0; i < l; ++i) {
@@ -146,6 +152,8 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     out->n_sph = (uint32_t)n;
     out->n_mat = (uint32_t)m;
     out->n_light = (uint32_t)l;
+    out->least_albedo = L.least_albedo;
+    out->unit_materials = L.unit_materials;
     out->bvh = pack.bvh(T, base);
     return ATX_OK;
 }

@@ -166,6 +166,11 @@ struct HostSceneLayout {
     std::vector<float> mat;       // 12 per material
     std::vector<float> mat_rr;    // 4 per material: albedo / p, p (see WfScene::mat_rr)
     std::vector<float> light;     // 8 per light
+    // the materials' ranges (mild_materials): their least albedo component but
+    // 0 (1 when there is none), and whether albedo, F0, metallic and roughness lie
+    // in [0, 1], the roughness not between 0 and 2^-10
+    float least_albedo = 1.0f;
+    bool unit_materials = true;
 };
 
 // Builds the device layout; ids outside [0, num_materials) are clamped to 0
@@ -200,6 +205,8 @@ struct DevScene {
     const float4 *sph = nullptr, *mat = nullptr, *mat_rr = nullptr, *light = nullptr;
     const int32_t* sph_mat = nullptr;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
+    float least_albedo = 1.0f;      // of HostSceneLayout
+    bool unit_materials = false;
     BvhDev bvh{};
     void use_pool(DevPool* pool) { block.use_pool(pool); }
     size_t bytes() const { return block.bytes(); }

@@ -29,6 +29,8 @@
 
 namespace atx {
 
+constexpr float kPi = 3.14159274101257324219f;  // glm::pi<float>()
+
 struct f3 {
     float x, y, z;
 };
@@ -54,8 +56,70 @@ ATX_HD float rint_(float x) { return rintf(x); }
 ATX_HD float fabs_(float x) { return fabsf(x); }
 #endif
 
+// ---- square roots and quotients without the compiler's range handling -------
+// The compiler's correctly rounded square root takes 14 instructions and its
+// division 11, 7 and 5 of them on the slower of the two VALU pipes: scaling
+// into and out of range and special cases.  Where the operands are known (or
+// tested, one test for several) to lie far from both ends of the exponent
+// range, the steps below give the same bits for 8 and 8, and for 5 per further
+// quotient by the same divisor (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990).  Path kernel: 640x360,
+// 4 spheres, 64 frames 0.409 -> 0.383 ms (14.5 % fewer vector instructions),
+// 1080p, 129 spheres, 256 frames 20.6 -> 20.1 ms (5 % fewer).
+
+// sqrt(d) from y, 1 / sqrt(d) to one ulp; h: half its inverse, closer than y.
+ATX_HD float sqrt_from(float d, float y, float& h)
+{
+    float g = d * y;
+    h = 0.5f * y;
+    const float e = fma_(-h, g, 0.5f);
+    g = fma_(g, e, g);
+    h = fma_(h, e, h);
+    return fma_(fma_(-g, g, d), h, g);
+}
+ATX_HD uint32_t bits_of(float x) { return __builtin_bit_cast(uint32_t, x); }
+// 1 / s from that h.  The start is moved up one ulp: two steps then round
+// correctly for every s, also those just below a power of two.
+ATX_HD float inverse_from(float s, float h)
+{
+    float r = __builtin_bit_cast(float, bits_of(h + h) + 1u);
+    r = fma_(fma_(-s, r, 1.0f), r, r);
+    return fma_(fma_(-s, r, 1.0f), r, r);
+}
+// 1 / y from the device's approximation r0.
+ATX_HD float reciprocal_from(float y, float r0) { return fma_(fma_(-y, r0, 1.0f), r0, r0); }
+// x / y from r, the reciprocal of y.
+ATX_HD float quotient(float x, float y, float r)
+{
+    const float q0 = x * r;
+    const float q1 = fma_(fma_(-y, q0, x), r, q0);
+    return fma_(fma_(-y, q1, x), r, q1);
+}
+// x / kPi for |x| in {0} and [2^-90, 2^90] (but for the sign of a zero).
+ATX_HD float over_pi(float x)
+{
+    constexpr float kInv = 0x1.45f306p-2f;   // 1 / kPi
+    const float q = x * kInv;
+    return fma_(fma_(-kPi, q, x), kInv, q);
+}
+// 2^-96 <= x <= 2^96: square roots and quotients of such numbers stay normal.
+ATX_HD bool mid_range(float x) { return bits_of(x) - 0x0f800000u <= 0x6f800000u - 0x0f800000u; }
+
 ATX_HD float length(f3 a) { return sqrt_cr(dot(a, a)); }
-ATX_HD f3 normalize(f3 a) { float inv = 1.0f / sqrt_cr(dot(a, a)); return scale(a, inv); }
+ATX_HD f3 normalize(f3 a)
+{
+    const float d = dot(a, a);
+#if defined(__HIP_DEVICE_COMPILE__)
+    float h;
+    const float len = sqrt_from(d, __builtin_amdgcn_rsqf(d), h);
+    float inv = inverse_from(len, h);
+    if (__builtin_expect(!mid_range(d), 0))
+        inv = 1.0f / sqrt_cr(d);
+    return scale(a, inv);
+#else
+    return scale(a, 1.0f / sqrt_cr(d));
+#endif
+}
 ATX_HD f3 cross(f3 a, f3 b)
 {
     return mk(a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y);
@@ -64,7 +128,6 @@ ATX_HD float gmax(float a, float b) { return a < b ? b : a; }
 ATX_HD float gmin(float a, float b) { return b < a ? b : a; }
 ATX_HD float gclamp(float x, float lo, float hi) { return gmin(gmax(x, lo), hi); }
 
-constexpr float kPi = 3.14159274101257324219f;  // glm::pi<float>()
 
 // ---- PCG hash (Core/include/Random.h:59-70) --------------------------------
 ATX_HD uint32_t pcg_hash(uint32_t seed)
@@ -188,14 +251,71 @@ ATX_HD f3 cook_torrance(f3 albedo, f3 F0, float metallic, float roughness, f3 N,
     return scale(add(mul(kD, diffuse), specular), n_dot_l);
 }
 
+#if defined(__HIPCC__)
+// cook_torrance for a scene of mild materials (WfScene::mild): the same
+// expressions with the quotients above, valid where `ok` comes back true (a
+// rounded half-vector term or a specular term near zero leaves it false).
+__device__ __forceinline__ f3 cook_torrance_mild(f3 albedo, f3 F0, float metallic, float roughness, f3 N, f3 V, f3 L,
+                                                 bool& ok)
+{
+    const f3 H = normalize(add(V, L));
+    const float n_dot_l = gmax(dot(N, L), 0.0000001f);
+    const float n_dot_v = gmax(dot(N, V), 0.0000001f);
+    const float n_dot_h = gmax(dot(N, H), 0.0f);
+    const float v_dot_h = gmax(dot(V, H), 0.0f);
+    const float cos_theta = gclamp(v_dot_h, 0.0f, 1.0f);
+    const float p5 = pow5(1.0f - cos_theta);
+    const f3 one = mk(1.0f, 1.0f, 1.0f);
+    const f3 F = add(F0, scale(sub(one, F0), p5));
+    const auto over = [](float x, float y) { return quotient(x, y, reciprocal_from(y, __builtin_amdgcn_rcpf(y))); };
+    // distribution_ggx: a2 is 0 or at least 2^-40
+    const float a = roughness * roughness;
+    const float a2 = a * a;
+    const float n_dot_h2 = n_dot_h * n_dot_h;
+    float d = n_dot_h2 * (a2 - 1.0f) + 1.0f;
+    d = kPi * d * d;
+    const float D = over(a2, d);
+    // geometry_schlick_ggx: 1/8 <= k <= 1/2, so the divisors lie between k and 1
+    const float r = roughness + 1.0f;
+    const float k = (r * r) / 8.0f;
+    const float G = over(n_dot_v, n_dot_v * (1.0f - k) + k) * over(n_dot_l, n_dot_l * (1.0f - k) + k);
+    const f3 kD = scale(sub(one, F), 1.0f - metallic);
+    const f3 num = scale(F, D * G);
+    const float denom = 4.0f * n_dot_l * n_dot_v + 0.001f;
+    const float rd = reciprocal_from(denom, __builtin_amdgcn_rcpf(denom));
+    const f3 specular = mk(quotient(num.x, denom, rd), quotient(num.y, denom, rd), quotient(num.z, denom, rd));
+    // 1 - F is 0 or at least 2^-24 in magnitude, the albedo 0 or at least 2^-40
+    const f3 dn = mul(sub(one, F), albedo);
+    const f3 diffuse = mk(over_pi(dn.x), over_pi(dn.y), over_pi(dn.z));
+    // numerators of the specular term: 0 (wraps to the largest) or at least 2^-80
+    const uint32_t least = min(min(bits_of(num.x) - 1u, bits_of(num.y) - 1u), bits_of(num.z) - 1u);
+    ok = d >= 0x1p-40f && least >= 0x17800000u - 1u;
+    return scale(add(mul(kD, diffuse), specular), n_dot_l);
+}
+#endif
+
 // ---- samplers (Engine/src/BRDF.cu:72-116) ------------------------------------
 ATX_HD f3 to_world(f3 N, float hx, float hy, float hz)
 {
+    const bool xz = fabs_(N.x) > fabs_(N.y);
     f3 T;
-    if (fabs_(N.x) > fabs_(N.y))
-        T = divs(mk(-N.z, 0.0f, N.x), sqrt_cr(N.x * N.x + N.z * N.z));
-    else
-        T = divs(mk(0.0f, -N.z, N.y), sqrt_cr(N.y * N.y + N.z * N.z));
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float u = xz ? N.x : N.y;
+    const float d = u * u + N.z * N.z;   // about 1/2 to 1 for a unit normal
+    float h;
+    const float s = sqrt_from(d, __builtin_amdgcn_rsqf(d), h);
+    const float r = inverse_from(s, h);
+    const float tz = quotient(u, s, r), tn = quotient(-N.z, s, r);
+    T = xz ? mk(tn, 0.0f, tz) : mk(0.0f, tn, tz);
+    // components near zero (or -0) take the compiler's division
+    if (__builtin_expect(!(mid_range(d) && fabs_(N.z) >= 0x1p-60f && fabs_(u) >= 0x1p-60f), 0))
+#endif
+    {
+        if (xz)
+            T = divs(mk(-N.z, 0.0f, N.x), sqrt_cr(N.x * N.x + N.z * N.z));
+        else
+            T = divs(mk(0.0f, -N.z, N.y), sqrt_cr(N.y * N.y + N.z * N.z));
+    }
     const f3 B = cross(N, T);
     return add(add(scale(T, hx), scale(B, hy)), scale(N, hz));
 }
@@ -213,16 +333,38 @@ ATX_HD f3 sample_next(f3 N, bool ggx, float roughness, uint32_t& seed)
 {
     const float u1 = pcg_float(seed);
     const float u2 = pcg_float(seed);
-    float radius, height;
+    // height = sqrt(A), radius = sqrt(B): the same square roots whichever branch
+    float A = 1.0f - u1;
     if (ggx) {
         const float a = roughness * roughness;
-        const float cos_theta = sqrt_cr((1.0f - u1) / (1.0f + (a * a - 1.0f) * u1));
-        radius = sqrt_cr(1.0f - cos_theta * cos_theta);
-        height = cos_theta;
-    } else {
-        radius = sqrt_cr(u1);
-        height = sqrt_cr(1.0f - u1);
+        const float den = 1.0f + (a * a - 1.0f) * u1;
+#if defined(__HIP_DEVICE_COMPILE__)
+        A = quotient(A, den, reciprocal_from(den, __builtin_amdgcn_rcpf(den)));
+#else
+        A = A / den;
+#endif
     }
+#if defined(__HIP_DEVICE_COMPILE__)
+    float h;
+    float height = sqrt_from(A, __builtin_amdgcn_rsqf(A), h);
+    float B = ggx ? 1.0f - height * height : u1;
+    float radius = sqrt_from(B, __builtin_amdgcn_rsqf(B), h);
+    // A is u1's complement (a multiple of 2^-32) or that over a divisor that is
+    // a multiple of 2^-24 where it is small: in range unless 0, NaN or far off
+    if (__builtin_expect(!(A >= 0x1p-40f && B >= 0x1p-40f), 0)) {
+        A = 1.0f - u1;
+        if (ggx) {
+            const float a = roughness * roughness;
+            A = A / (1.0f + (a * a - 1.0f) * u1);
+        }
+        height = sqrt_cr(A);
+        B = ggx ? 1.0f - height * height : u1;
+        radius = sqrt_cr(B);
+    }
+#else
+    const float height = sqrt_cr(A);
+    const float radius = sqrt_cr(ggx ? 1.0f - height * height : u1);
+#endif
     const float phi = 2.0f * kPi * u2;
     float s, c;
     sincos_(phi, s, c);

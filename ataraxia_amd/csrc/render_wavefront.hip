@@ -165,14 +165,19 @@ __device__ __forceinline__ bool shade_hit(CScene* S, const Hit& h, f3 ro, f3 rd,
 // Cook-Torrance term of a light that reaches the hit, weighted by the path
 // throughput (Renderer.cu:351-360).
 __device__ __forceinline__ f3 light_term(const float4* mat, const float4* light, int32_t mid, uint32_t lidx, f3 nrm,
-                                         f3 rd, f3 L, f3 tp)
+                                         f3 rd, f3 L, f3 tp, bool mild)
 {
     const float4 m0 = mat[3 * mid + 0];
     const float4 m1 = mat[3 * mid + 1];
     const f3 albedo = xyz(m0);
     const float metallic = m1.w;
     const f3 base = add(scale(xyz(m1), 1.0f - metallic), scale(albedo, metallic));
-    const f3 f = cook_torrance(albedo, base, metallic, m0.w, nrm, neg(rd), L);
+    f3 f;
+    bool ok = false;
+    if (mild)
+        f = cook_torrance_mild(albedo, base, metallic, m0.w, nrm, neg(rd), L, ok);
+    if (__builtin_expect(!ok, 0))
+        f = cook_torrance(albedo, base, metallic, m0.w, nrm, neg(rd), L);
     const float4 l0 = light[2 * lidx + 0];
     const float4 l1 = light[2 * lidx + 1];
     return mul(mul(scale(xyz(l1), l0.w), f), tp);
@@ -181,7 +186,7 @@ __device__ __forceinline__ f3 light_term(const float4* mat, const float4* light,
 __device__ __forceinline__ void add_light(CScene* S, int32_t mid, uint32_t lidx, f3 nrm, f3 rd, f3 L, f3 tp,
                                           f3& col)
 {
-    col = add(col, light_term(S->mat, S->light, mid, lidx, nrm, rd, L, tp));
+    col = add(col, light_term(S->mat, S->light, mid, lidx, nrm, rd, L, tp, S->mild != 0u));
 }
 
 // Throughput and Russian roulette at the end of a bounce (Renderer.cu:362-379).
@@ -189,10 +194,23 @@ __device__ __forceinline__ void add_light(CScene* S, int32_t mid, uint32_t lidx,
 __device__ __forceinline__ bool roulette(CScene* S, int32_t mid, f3& tp, int32_t bounce, uint32_t& seed)
 {
     tp = mul(tp, xyz(S->mat[3 * mid]));
-    const float p = gmax(0.1f, gmin(1.0f, length(tp)));
+    float p;
+    if (S->mild) {
+        // p is 0.1 for every length below that, 1 for every one above it
+        float h;
+        const float d = __builtin_amdgcn_fmed3f(dot(tp, tp), 0x1p-20f, 4.0f);
+        p = gmax(0.1f, gmin(1.0f, sqrt_from(d, __builtin_amdgcn_rsqf(d), h)));
+    } else {
+        p = gmax(0.1f, gmin(1.0f, length(tp)));
+    }
     if (pcg_float(seed) > p)
         return true;
-    tp = divs(tp, p);
+    if (S->mild) {
+        const float r = reciprocal_from(p, __builtin_amdgcn_rcpf(p));
+        tp = mk(quotient(tp.x, p, r), quotient(tp.y, p, r), quotient(tp.z, p, r));
+    } else {
+        tp = divs(tp, p);
+    }
     return bounce + 1 >= S->max_bounces;
 }
 
@@ -916,7 +934,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
             f3 term = zero;
             if (hit && lit_by(h, dist2)) {
                 mask |= 1u << l;
-                term = light_term(s.mat, s.light, mid, l, nrm, rd, d, one);
+                term = light_term(s.mat, s.light, mid, l, nrm, rd, d, one, s.mild != 0u);
             }
             a.light[(size_t)l * npx + px] = make_float4(term.x, term.y, term.z, 0.0f);
         }

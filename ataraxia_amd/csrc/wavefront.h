@@ -65,6 +65,9 @@ struct WfScene {
     const float4* sph;
     const int32_t* sph_mat;
     const float4* mat;
+    // 1: the materials and max_bounces are such that no quotient of a light
+    // term or of a roulette can leave the normal range (mild_materials)
+    uint32_t mild;
     const float4* mat_rr;  // per material: albedo / p and p, the roulette at a path's first hit
     const float4* light;
     uint32_t n_sph;

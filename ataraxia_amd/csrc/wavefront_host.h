@@ -3,6 +3,7 @@
 // wavefront mode).
 #pragma once
 
+#include <math.h>
 #include <string.h>
 
 #include "camera_host.h"
@@ -10,6 +11,15 @@
 #include "wavefront.h"
 
 namespace atx {
+
+// Whether WfScene::mild holds for materials in the layout of HostSceneLayout:
+// albedo, F0, metallic and roughness within [0, 1], roughness 0 or at least
+// 2^-10, and albedos 0 or so large that a path's throughput, a product of at
+// most max_bounces of them over numbers up to 1, is 0 or at least 2^-80.
+inline bool mild_materials(float least_albedo, bool unit_range, int32_t max_bounces)
+{
+    return unit_range && least_albedo >= 0x1p-40f && max_bounces * -log2f(least_albedo) <= 80.0f;
+}
 
 // Everything of an entry but the scene's arrays.
 inline void fill_wf_view(const atx_settings& st, const atx_camera& cam, float4* accum, float4* comp, uint32_t* image,
@@ -42,6 +52,7 @@ inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_c
     out->mat = g.mat;
     out->mat_rr = g.mat_rr;
     out->light = g.light;
+    out->mild = mild_materials(g.least_albedo, g.unit_materials, st.max_bounces) ? 1u : 0u;
     out->n_sph = g.n_sph;
     out->n_mat = g.n_mat;
     out->n_light = g.n_light;
