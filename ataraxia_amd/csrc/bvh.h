@@ -12,11 +12,13 @@
 //   tiles  uint4[n_tiles][128]  matrix operands in half precision
 //   tboxes float4[n_nodes][2]   box (centre, half size; tile units) of every
 //                           tile, then of every eight consecutive tiles
-//   tsph   float4[n]        spheres in tile order (cx, cy, cz, r*r)
-//   tidx   int32[n]         their index in the scene
-//   big    int32[n_big]     spheres kept out of the tiles (radius larger than
-//                           the region of the others, e.g. a ground sphere,
-//                           or non-finite data); tested by a flat loop first
+//   tsph   float4[n]        spheres by slot (cx, cy, cz, r*r): those of the
+//                           tiles in tile order, then from slot big0 on the
+//                           n_big kept out of the tiles (radius larger than
+//                           the region of the others, e.g. a ground sphere, or
+//                           non-finite data), which a loop tests first
+//   tidx   int32[n]         each slot's sphere in the scene
+//   tmat   int32[n]         its material (nullptr: looked up by tidx)
 // Boxes are rounded outwards from double precision, so each contains its
 // spheres exactly.
 #pragma once
@@ -33,10 +35,10 @@ struct BvhDev {
     const float4* tboxes;
     const float4* tsph;
     const int32_t* tidx;
-    const int32_t* big;
+    const int32_t* tmat;
     uint32_t n_tiles;   // 0 = flat loop over all spheres
     uint32_t n_nodes;   // boxes; 0 = every ray tests every sphere
-    uint32_t n_big;
+    uint32_t n_big, big0;
     float cx, cy, cz;   // centre of the tiles' region
     float ts;           // tile units per world unit (a power of two)
     float t_lin;        // 2^-18 / smallest radius in tile units

@@ -79,11 +79,20 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l)
 {
-    return 16 * n + 4 * n + 48 * m + 16 * m + 32 * l + bvh_device_bytes(n) + (ScenePack::kArrays + 1) * 256;
+    return 16 * n + 4 * n + 4 * n + 48 * m + 16 * m + 32 * l + bvh_device_bytes(n) + (ScenePack::kArrays + 1) * 256;
 }
 
-ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T)
+ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups)
+    : tile_sph(T.tsph), tile_idx(T.tidx)
 {
+    if (T.n_tiles > 0) {
+        for (int32_t id : T.big) {
+            tile_sph.insert(tile_sph.end(), &L.sph[4 * (size_t)id], &L.sph[4 * (size_t)id] + 4);
+            tile_idx.push_back(id);
+        }
+        for (int32_t id : tile_idx)
+            if (lookups) tile_mat.push_back(L.sph_mat[id]);
+    }
     const auto put = [this](Array a, const auto& v) {
         off[a] = bytes;
         src[a] = v.data();
@@ -95,12 +104,14 @@ ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T)
     put(kSphMat, L.sph_mat);
     put(kMat, L.mat);
     put(kLight, L.light);
-    put(kBig, T.big);
     put(kTiles, T.tiles);
     put(kTileBoxes, T.tboxes);
-    put(kTileSph, T.tsph);
-    put(kTileIdx, T.tidx);
-    put(kMatRr, L.mat_rr);
+    put(kTileSph, tile_sph);
+    put(kTileIdx, tile_idx);
+    put(kTileMat, tile_mat);
+    const std::vector<float> none;
+    if (lookups) put(kMatRr, L.mat_rr);
+    else put(kMatRr, none);
 }
 
 std::vector<unsigned char> ScenePack::block() const
@@ -119,10 +130,11 @@ BvhDev ScenePack::bvh(const HostBvh& T, const void* base) const
     b.tboxes = at<float4>(base, kTileBoxes);
     b.tsph = at<float4>(base, kTileSph);
     b.tidx = at<int32_t>(base, kTileIdx);
-    b.big = at<int32_t>(base, kBig);
+    b.tmat = tile_mat.empty() ? nullptr : at<int32_t>(base, kTileMat);
     b.n_tiles = T.n_tiles;
     b.n_nodes = (uint32_t)(T.tboxes.size() / 8);
     b.n_big = (uint32_t)T.big.size();
+    b.big0 = (uint32_t)T.tidx.size();
     b.cx = T.cx;
     b.cy = T.cy;
     b.cz = T.cz;

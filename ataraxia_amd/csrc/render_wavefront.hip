@@ -138,27 +138,33 @@ __device__ __forceinline__ bool lit_by(const Hit& h, float dist2)
     return !(st > 0.0f && st * st < dist2);
 }
 
-// The hit material's emission, added to col (Renderer.cu:334-337).
-__device__ __forceinline__ void add_emission(const float4* mat, int32_t mid, f3 tp, f3& col)
+// The hit material's emission (m2: its last quarter), added to col
+// (Renderer.cu:334-337).
+__device__ __forceinline__ void add_emission(float4 m2, f3 tp, f3& col)
 {
-    const float4 m2 = mat[3 * mid + 2];
     if (m2.w > 0.0f)
         col = add(col, mul(scale(xyz(m2), m2.w), tp));
 }
 
-// Emission of a continuation hit and the light its shadow ray goes to.
-// Returns true when a shadow ray follows (the scene has lights).
-__device__ __forceinline__ bool shade_hit(CScene* S, const Hit& h, f3 ro, f3 rd, f3 tp, uint32_t seed, f3& col,
-                                          f3& nrm, f3& so, int32_t& mid, uint32_t& lidx, f3& L, float& dist2)
+// Emission of a continuation hit on `sphere` of material mid and the light its
+// shadow ray goes to.  Returns true when a shadow ray follows (the scene has
+// lights).
+__device__ __forceinline__ bool shade_hit(CScene* S, float4 sphere, int32_t mid, const Hit& h, f3 ro, f3 rd, f3 tp,
+                                          uint32_t seed, f3& col, f3& nrm, f3& so, uint32_t& lidx, f3& L, float& dist2)
 {
+    // both loads before the first use of either
+    float4 light = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (S->n_light != 0) {
+        lidx = umod(pcg_hash(seed), S->div_light);   // pcg_hash(seed) % n_light
+        light = S->light[2 * lidx];
+    }
+    const float4 m2 = S->mat[3 * mid + 2];
     f3 pos;
-    hit_frame(as_const(S->sph)[h.id], h, ro, rd, pos, nrm, so);
-    mid = S->sph_mat[h.id];
-    add_emission(S->mat, mid, tp, col);
+    hit_frame(sphere, h, ro, rd, pos, nrm, so);
+    add_emission(m2, tp, col);
     if (S->n_light == 0)
         return false;
-    lidx = umod(pcg_hash(seed), S->div_light);   // pcg_hash(seed) % n_light
-    light_ray(S->light[2 * lidx], pos, L, dist2);
+    light_ray(light, pos, L, dist2);
     return true;
 }
 
@@ -191,9 +197,13 @@ __device__ __forceinline__ void add_light(CScene* S, int32_t mid, uint32_t lidx,
 
 // Throughput and Russian roulette at the end of a bounce (Renderer.cu:362-379).
 // Returns true when the path ends here, by the draw or at its last bounce.
-__device__ __forceinline__ bool roulette(CScene* S, int32_t mid, f3& tp, int32_t bounce, uint32_t& seed)
+// surface: the material's roughness and metallic, for the next direction.
+__device__ __forceinline__ bool roulette(CScene* S, int32_t mid, f3& tp, int32_t bounce, uint32_t& seed, f3& surface)
 {
-    tp = mul(tp, xyz(S->mat[3 * mid]));
+    const float4 m0 = S->mat[3 * mid];
+    surface.x = m0.w;
+    surface.y = S->mat[3 * mid + 1].w;
+    tp = mul(tp, xyz(m0));
     float p;
     if (S->mild) {
         // p is 0.1 for every length below that, 1 for every one above it
@@ -217,18 +227,19 @@ __device__ __forceinline__ bool roulette(CScene* S, int32_t mid, f3& tp, int32_t
 // The same at bounce 0, where the throughput is 1: the scene holds p and
 // albedo / p per material (mat_rr), which saves a square root and three
 // divisions in every path.
-__device__ __forceinline__ bool roulette_first(CScene* S, int32_t mid, f3& tp, uint32_t& seed)
+__device__ __forceinline__ bool roulette_first(CScene* S, int32_t mid, f3& tp, uint32_t& seed, f3& surface)
 {
+    surface.x = S->mat[3 * mid].w;
+    surface.y = S->mat[3 * mid + 1].w;
     const float4 rr = S->mat_rr[mid];
     tp = xyz(rr);
     return pcg_float(seed) > rr.w || S->max_bounces <= 1;
 }
 
 // The next direction of a path that goes on (Renderer.cu:381-384).
-__device__ __forceinline__ void next_direction(CScene* S, int32_t mid, f3 nrm, f3& rd, int32_t& bounce,
-                                               uint32_t& seed)
+__device__ __forceinline__ void next_direction(f3 surface, f3 nrm, f3& rd, int32_t& bounce, uint32_t& seed)
 {
-    rd = sample_next(nrm, S->mat[3 * mid + 1].w > 0.0f, S->mat[3 * mid].w, seed);
+    rd = sample_next(nrm, surface.y > 0.0f, surface.x, seed);
     ++bounce;
     seed += (uint32_t)bounce;
 }
@@ -492,7 +503,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                             h.id = hid;
                             h.t = __uint_as_float(r0.y);
                             f3 so, L;
-                            shade_hit(S, h, ro, rd, tp, seed, col, nrm, so, mid, lidx, L, dist2);
+                            mid = (int32_t)r0.w;
+                            shade_hit(S, as_const(S->sph)[h.id], mid, h, ro, rd, tp, seed, col, nrm, so, lidx, L, dist2);
                             vd = rd;
                             ro = so;
                             rd = L;
@@ -509,7 +521,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                                 if ((r0.z >> lidx) & 1u)
                                     col = add(col, xyz(lt));
                             }
-                            done = roulette_first(S, mid, tp, seed);
+                            done = roulette_first(S, mid, tp, seed, vd);
                             state = kNew;
                         }
                         if (done) {
@@ -591,7 +603,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         // kernel issued 1890 VALU instructions per round instead of 1600
         // (1080p, 256 frames: 22.5 -> 20.0 ms).
         if (state == kNew) {
-            next_direction(S, mid, nrm, rd, bounce, seed);
+            next_direction(vd, nrm, rd, bounce, seed);
             state = kCont;
         }
 
@@ -603,6 +615,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         rays += (unsigned long long)__popcll(__ballot(traces));
         const bool shadow = state == kShadow;
         Hit h;
+        float4 hit_sphere;
+        int32_t hit_mat;
         const bool tree = kTree && S && S->bvh.n_tiles != 0u;
         const auto query = [&]() {
             if constexpr (kPark) {
@@ -622,14 +636,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             BvhQuery q;
             if (tree) {
                 const BvhDev B = S->bvh;
-                h = trace_tiles(B, flat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
+                h = trace_tiles(B, flat, S->sph_mat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
             } else {
                 if (kInPlace && S->exact)
                     h = trace_exact(flat, S->n_sph, ro, rd);
                 else
                     h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
                 q.tests = S->n_sph;
+                if (h.id >= 0) {
+                    q.sphere = flat((uint32_t)h.id);
+                    q.mat = S->sph_mat[h.id];
+                }
             }
+            hit_sphere = q.sphere;
+            hit_mat = q.mat;
             if constexpr (kPark) {
                 __asm__ volatile("" ::: "memory");
                 col = mk(__uint_as_float(parked[0][lane]), __uint_as_float(parked[1][lane]),
@@ -667,7 +687,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                     end_path = true;
                 } else {
                     f3 so, L;
-                    if (shade_hit(S, h, ro, rd, tp, seed, col, nrm, so, mid, lidx, L, dist2)) {
+                    mid = hit_mat;
+                    if (shade_hit(S, hit_sphere, mid, h, ro, rd, tp, seed, col, nrm, so, lidx, L, dist2)) {
                         vd = rd;
                         rd = L;
                         state = kShadow;
@@ -695,7 +716,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         }
         if (end_bounce) {
             // the next ray leaves from the hit's offset origin, which ro holds
-            if (roulette(S, mid, tp, bounce, seed))
+            if (roulette(S, mid, tp, bounce, seed, vd))
                 end_path = true;
             else
                 state = kNew;
@@ -874,6 +895,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
     first.id = -1;
     first.t = FLT_MAX;
     int32_t mid = 0;
+    float4 hit_sphere = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     uint32_t mask = 0u;
     uint32_t slot = 0u;   // index in the hit list
     // the primary ray, then a shadow ray towards each light (one query in the
@@ -895,10 +917,18 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
         if constexpr (kTree) {
             BvhQuery q;
             if (__any(act))   // a wave of missing pixels has no shadow rays
-                h = trace_tiles(B, flat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
+                h = trace_tiles(B, flat, s.sph_mat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
+            if (k == 0u) {
+                hit_sphere = q.sphere;
+                mid = q.mat;
+            }
         } else if (act) {
             uint32_t ex = 0;
             h = trace_filtered(flat, s.n_sph, o, d, ex);
+            if (k == 0u && h.id >= 0) {
+                hit_sphere = flat((uint32_t)h.id);
+                mid = s.sph_mat[h.id];
+            }
         }
         if (k == 0u) {
             first = h;
@@ -925,9 +955,8 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
                 const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
                 slot = base + (uint32_t)__popcll(hm & below);
                 a.hits[slot] = px;
-                hit_frame(as_const(s.sph)[first.id], first, ro, rd, pos, nrm, so);
-                mid = s.sph_mat[first.id];
-                add_emission(s.mat, mid, one, col);
+                hit_frame(hit_sphere, first, ro, rd, pos, nrm, so);
+                add_emission(s.mat[3 * mid + 2], one, col);
             }
         } else if (in) {
             const uint32_t l = k - 1u;
