@@ -447,9 +447,8 @@ void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out)
 size_t bvh_device_bytes(uint64_t n)
 {
     const uint64_t tiles = (n + kTileSpheres - 1) / kTileSpheres, boxes = tiles + (tiles + 7) / 8;
-    const size_t big = 4 * (kBvhMaxBig + 1) + 16;
-    if (n > kTileMaxSpheres + kBvhMaxBig) return big;
-    return (size_t)(tiles * kTileWords * 4 + boxes * 32 + 32) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16) + big;
+    if (n < kBvhMinSpheres || n > kTileMaxSpheres + kBvhMaxBig) return 0;   // no tiles
+    return (size_t)(tiles * kTileWords * 4 + boxes * 32 + 32) + (size_t)(16 * n + 16) + (size_t)(4 * n + 16);
 }
 
 }  // namespace atx

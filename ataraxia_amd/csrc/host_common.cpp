@@ -79,10 +79,10 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
 
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l)
 {
-    return 16 * n + 4 * n + 4 * n + 48 * m + 16 * m + 32 * l + bvh_device_bytes(n) + (ScenePack::kArrays + 1) * 256;
+    return 16 * n + 4 * n + 4 * n + 48 * m + 16 * m + 32 * l + bvh_device_bytes(n) + (ScenePack::kArrays + 1) * 16;
 }
 
-ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups)
+ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups, size_t align)
     : tile_sph(T.tsph), tile_idx(T.tidx)
 {
     if (T.n_tiles > 0) {
@@ -93,11 +93,11 @@ ScenePack::ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups)
         for (int32_t id : tile_idx)
             if (lookups) tile_mat.push_back(L.sph_mat[id]);
     }
-    const auto put = [this](Array a, const auto& v) {
+    const auto put = [this, align](Array a, const auto& v) {
         off[a] = bytes;
         src[a] = v.data();
         src_bytes[a] = v.size() * 4;
-        bytes += (src_bytes[a] + 255) & ~size_t(255);
+        bytes += (src_bytes[a] + align - 1) / align * align;
     };
     bytes = 0;
     put(kSph, L.sph);
@@ -153,7 +153,7 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     build_bvh(L.sph.data(), (uint32_t)n, 0, &T);
     const ScenePack pack(L, T);
     // never an empty block: the kernels' pointers stay valid without spheres
-    ATX_HIP(out->block.reserve(pack.bytes + 256));
+    ATX_HIP(out->block.reserve(pack.bytes + 16));
     if (pack.bytes) ATX_HIP(hipMemcpy(out->block.get(), pack.block().data(), pack.bytes, hipMemcpyHostToDevice));
     const void* base = out->block.get();
     out->sph = pack.at<float4>(base, ScenePack::kSph);

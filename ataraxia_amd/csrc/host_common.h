@@ -180,18 +180,18 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
                        uint64_t m, const atx_light* lights, uint64_t l, HostSceneLayout* out);
 
 // The arrays of a scene and its tiles laid out in one block, each from a
-// multiple of 256 bytes on, so that they go to the device in one copy (ten
+// multiple of `align` bytes on, so that they go to the device in one copy (ten
 // copies, each waited for, took about 110 us).
 struct ScenePack {
     enum Array { kSph, kSphMat, kMat, kLight, kTiles, kTileBoxes, kTileSph, kTileIdx, kTileMat, kMatRr, kArrays };
     size_t off[kArrays];
-    size_t bytes;   // a multiple of 256
+    size_t bytes;   // a multiple of align
     const void* src[kArrays];
     size_t src_bytes[kArrays];
     std::vector<float> tile_sph;                 // by slot (bvh.h)
     std::vector<int32_t> tile_idx, tile_mat;
     // lookups: also the arrays that save a dependent load (tmat, mat_rr)
-    ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups = true);
+    ScenePack(const HostSceneLayout& L, const HostBvh& T, bool lookups = true, size_t align = 16);
     std::vector<unsigned char> block() const;
     // the kernel's view of T, whose arrays are in the block at `base`
     BvhDev bvh(const HostBvh& T, const void* base) const;

@@ -98,7 +98,7 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     const size_t off_table = align256(off_queue + kQueueWords * sizeof(unsigned int));
     static_assert(kCounterBytes + kQueueWords * sizeof(unsigned int) + sizeof(WfScene) + 3 * 256 <= kControlBytes,
                   "control pages");
-    const ScenePack pack(L, T, false);   // as many spheres as fit
+    const ScenePack pack(L, T, false, 256);   // as many spheres as fit
     const size_t total = pack.bytes;
     if (total > kScratchBytes) {
         set_error("scene needs %zu bytes of device scratch; atx_render_frames_noalloc holds at most %zu "

@@ -765,13 +765,14 @@ __global__ __launch_bounds__(256) void k_accumulate(WfPass a)
     const bool first = S.frame0 == 1u;
     // a pixel left out of the jobs (its primary ray misses): every frame's
     // sample is the one such a path returns, the sky colour or black
-    const bool sky = S.hit_px && (int32_t)S.first[4 * (size_t)px].x < 0;
+    uint32_t slot = S.hit_px ? __float_as_uint(S.dirs[px].w) : px;
+    const bool sky = slot == kNoSlot;
+    slot = sky ? 0u : slot;
     const float4 sky_c = S.sky_light ? make_float4(0.6f, 0.7f, 0.9f, 1.0f) : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
     float4 acc = first ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : S.accum[px];
     // this pixel's samples: frame f at sp[f * step] (slots are hit-list
     // indices with a hit list, else pixels; a sky pixel has none)
     const uint32_t slots = job_slots(S.hit_px, npx);
-    const uint32_t slot = sky ? 0u : S.hit_px ? S.first[4 * (size_t)px + 3].y : px;
     const uint32_t left = slots - (slot & ~(kJobGroupPx - 1u));
     const uint32_t step = left < kJobGroupPx ? left : kJobGroupPx;
     const ATX_GLOBAL float3* sp = (const ATX_GLOBAL float3*)(uintptr_t)S.samples + job_of(slot, 0u, slots, S.frames);
@@ -852,6 +853,7 @@ struct FirstArgs {
     uint4* rec;        // 4 per pixel
     float4* light;     // [light][pixel], or nullptr
     uint32_t* hits;    // pixels whose primary ray hits, appended
+    float4* dirs;      // s.dirs, whose w takes each pixel's index among them
     uint32_t* n_hits;  // their count (zero before the launch)
 };
 
@@ -897,7 +899,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
     int32_t mid = 0;
     float4 hit_sphere = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     uint32_t mask = 0u;
-    uint32_t slot = 0u;   // index in the hit list
+    uint32_t slot = kNoSlot;   // index in the hit list
     // the primary ray, then a shadow ray towards each light (one query in the
     // code: a second copy of it would take the registers of both)
     const uint32_t n_rays = 1u + (a.light ? s.n_light : 0u);
@@ -970,11 +972,12 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
     }
     if (!in)
         return;
+    a.dirs[px].w = __uint_as_float(slot);
     uint4* r = a.rec + 4 * (size_t)px;
     r[0] = make_uint4((uint32_t)first.id, __float_as_uint(first.t), mask, (uint32_t)mid);
     r[1] = make_uint4(__float_as_uint(nrm.x), __float_as_uint(nrm.y), __float_as_uint(nrm.z), __float_as_uint(so.x));
     r[2] = make_uint4(__float_as_uint(so.y), __float_as_uint(so.z), __float_as_uint(col.x), __float_as_uint(col.y));
-    r[3] = make_uint4(__float_as_uint(col.z), slot, 0u, 0u);
+    r[3] = make_uint4(__float_as_uint(col.z), 0u, 0u, 0u);
 }
 
 __global__ void k_zero_u32(unsigned int* p, uint32_t n)
@@ -1076,6 +1079,7 @@ hipError_t launch_first_hits(const WfScene& s, hipStream_t stream)
     a.rec = v.rec;
     a.light = v.light;
     a.hits = v.hits;
+    a.dirs = const_cast<float4*>(s.dirs);
     a.n_hits = v.n_hits;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, v.n_hits, 1u);
     const uint32_t tiles = ((s.width + 7u) / 8u) * ((s.height + 7u) / 8u);

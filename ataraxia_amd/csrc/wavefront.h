@@ -96,7 +96,8 @@ struct WfScene {
     int32_t* dbg_shadow;
     float3* samples;       // this launch's samples (r, g, b), indexed by the scene's job
                            // (job_pixel_frame order); k_accumulate adds the alpha of 1 itself
-    const float4* dirs;    // primary ray direction per pixel (x, y, z, 0); nullptr: computed per path
+    const float4* dirs;    // primary ray direction per pixel (x, y, z), w: its index in the hit list once
+                           // k_first_hit has run (as bits); nullptr: computed per path
     const uint4* first;        // first-bounce records, 4 per pixel (launch_first_hits); nullptr: traced per path
     const float4* first_light; // first-bounce light terms, [light][pixel] (nullptr: none)
     // With a first-bounce cache, the pixels whose primary ray hits a sphere:
@@ -248,14 +249,18 @@ hipError_t launch_camera_dirs(const WfScene& s, float4* dirs, hipStream_t stream
 //          lights), the hit's material;
 //      [1] normal x, y, z, origin of the rays leaving the hit x;
 //      [2] origin y, z, radiance after the hit's emission r, g;
-//      [3] radiance b, the pixel's index in the hit list (hits only), 0, 0;
+//      [3] radiance b, 0, 0, 0;
 //  * then, for scenes of 1..kFirstMaxLights lights, per light and pixel
 //    ([light][pixel]) the light's Cook-Torrance term at the hit (float4,
 //    w = 0; zero when the light does not reach the hit);
 //  * then the list of pixels whose primary ray hits (uint32 each, in no
 //    particular order) and its length (uint32, 16-byte slot).
+// Each pixel's index in the list (kNoSlot: not in it), which k_accumulate
+// reads, goes to the fourth component of its primary direction (read from the
+// records, 64 bytes apart, it cost k_accumulate 16 us more at 1080p).
 // The path kernel then does bounce 0 from it where it hands out a job.
 constexpr uint32_t kFirstMaxLights = 32;
+constexpr uint32_t kNoSlot = ~0u;
 struct FirstCacheView {
     uint4* rec;
     float4* light;
