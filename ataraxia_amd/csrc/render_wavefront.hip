@@ -749,6 +749,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
 __global__ __launch_bounds__(256) void k_accumulate(WfPass a)
 {
     const uint32_t g = blockIdx.x * 256u + threadIdx.x;
+    if (a.totals && blockIdx.x == 0u && threadIdx.x <= kCtrCount) {
+        unsigned long long s = 0;
+        if (threadIdx.x == kCtrCount)
+            s = a.n_hits ? *a.n_hits : 0u;
+        else
+            for (uint32_t k = 0; k < kCounterLines; ++k)
+                s += a.counters[k * kCounterStride + threadIdx.x];
+        a.totals[threadIdx.x] = s;
+    }
     if (g >= a.total_px)
         return;
     uint32_t lo = 0, hi = a.n_scenes;          // last scene with px_begin <= g
@@ -1017,7 +1026,10 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
         return hipErrorInvalidValue;
     // no jobs (every pixel's primary ray misses): k_accumulate alone
     if (p.total_chunks > 0) {
-        hipLaunchKernelGGL(path_kernel(l.flat_only, l.waves), dim3(l.workgroups), dim3(256), 0, stream, p);
+        // no workgroup without a first chunk for a wave
+        const uint32_t most = (p.total_chunks + 3u) / 4u;
+        hipLaunchKernelGGL(path_kernel(l.flat_only, l.waves), dim3(l.workgroups < most ? l.workgroups : most),
+                           dim3(256), 0, stream, p);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && paths_done)

@@ -35,7 +35,8 @@ struct Renderer {
     bool has_scene = false;
     int kernel = ATX_KERNEL_WAVEFRONT;
     int accel = ATX_ACCEL_BVH;
-    DevBuf wf_table, wf_queue, wf_samples, wf_dirs, wf_first;
+    DevBuf launch_dev, wf_samples, wf_dirs, wf_first;
+    std::vector<unsigned char> launch_host;   // copied to launch_dev by every call
     // wf_dirs holds the primary rays of dirs_cam; wf_first the first-bounce
     // cache of that camera and the current scene (set_scene clears first_valid)
     atx_camera dirs_cam{}, prev_cam{};
@@ -48,11 +49,11 @@ struct Renderer {
     uint32_t wf_chunk = 0;   // jobs per chunk; 0: launch_chunk_px per launch
     uint32_t wf_frames = kRendererFramesPerLaunch;
     uint32_t wf_waves = 0;   // path-kernel instance (resident waves per SIMD); 0: default
-    DevBuf accum, comp, image, counters;
+    DevBuf accum, comp, image;
     HostStage results;
-    // pinned host memory the call's statistics are copied into (counters,
-    // then the hit list's length): copies into pageable memory block the
-    // host until the stream is idle, one after the other
+    // pinned host memory for the call's statistics: k_accumulate of the last
+    // launch writes the sums and the hit list's length there (a copy more on
+    // the stream took 10 us); plain calls copy the counter lines
     unsigned long long* readback = nullptr;
     uint32_t width = 0, height = 0;
     atx_settings settings{1, 0, {0, 0}, 15};  // Scene.h:49-56 defaults
@@ -193,26 +194,36 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         }
     }
     const uint32_t n_launch = (uint32_t)table.size();
-    if (n_launch) {
-        ATX_HIP(r->wf_table.reserve(n_launch * sizeof(WfScene)));
-        ATX_HIP(r->wf_queue.reserve(n_launch * kQueueWords * sizeof(unsigned int)));
-        ATX_HIP(hipMemcpyAsync(r->wf_table.get(), table.data(), n_launch * sizeof(WfScene), hipMemcpyHostToDevice,
-                               r->stream));
-        ATX_HIP(launch_zero_u32(r->wf_queue.as<unsigned int>(), n_launch * kQueueWords, r->stream));
-    }
-    ATX_HIP(hipMemsetAsync(r->counters.get(), 0, kCounterBytes, r->stream));
+    // The launches' table, their queues and the counters (both zero) are one
+    // block, sent in one copy; as a copy, a fill kernel and a memset they
+    // took 35 us of a 320x180 call's 124.
+    const size_t off_queue = (n_launch * sizeof(WfScene) + 255) & ~size_t(255);
+    const size_t off_ctr = off_queue + n_launch * kQueueWords * sizeof(unsigned int);
+    r->launch_host.assign(off_ctr + kCounterBytes, 0);
+    if (n_launch) memcpy(r->launch_host.data(), table.data(), n_launch * sizeof(WfScene));
+    ATX_HIP(r->launch_dev.reserve(r->launch_host.size()));
+    ATX_HIP(hipMemcpyAsync(r->launch_dev.get(), r->launch_host.data(), r->launch_host.size(), hipMemcpyHostToDevice,
+                           r->stream));
+    const WfScene* d_table = r->launch_dev.as<WfScene>();
+    unsigned int* d_queue = reinterpret_cast<unsigned int*>(r->launch_dev.as<unsigned char>() + off_queue);
+    unsigned long long* d_ctr = reinterpret_cast<unsigned long long*>(r->launch_dev.as<unsigned char>() + off_ctr);
+    const bool read_hits = use_first && !r->n_hit_exact;
     ATX_HIP(hipEventRecord(r->ev0, r->stream));
     if (wf) {
         for (size_t l = 0; l < table.size(); ++l) {
             WfPass wp{};
-            wp.scenes = r->wf_table.as<WfScene>() + l;
+            wp.scenes = d_table + l;
             wp.n_scenes = 1;
             wp.total_chunks = table[l].n_chunks;
             wp.chunk_px = launch_chunk[l];
             wp.total_px = table[l].width * table[l].height;
-            wp.queue = r->wf_queue.as<unsigned int>() + l * kQueueWords;
-            wp.counters = r->counters.as<unsigned long long>();
-            ATX_HIP(hipEventRecord(r->wf_ev[2 * l], r->stream));
+            wp.queue = d_queue + l * kQueueWords;
+            wp.counters = d_ctr;
+            if (l + 1 == table.size()) {
+                wp.totals = r->readback;
+                wp.n_hits = read_hits ? first_cache_view(r->wf_first.get(), npx, r->geo.n_light).n_hits : nullptr;
+            }
+            if (l > 0) ATX_HIP(hipEventRecord(r->wf_ev[2 * l], r->stream));   // the first starts at ev0
             ATX_HIP(launch_wavefront(wp, shape, r->stream, r->wf_ev[2 * l + 1]));
             // Renderer.cu:245-248, once per frame of the launch
             for (uint32_t f = 0; f < launch_frames[l]; ++f) {
@@ -224,9 +235,9 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         const bool flat_only = n_launch == 0 || wf_flat_only(table.data(), 1);
         for (uint32_t f = 0; f < frames; ++f) {
             WfPass wp = passes[f];
-            wp.scenes = r->wf_table.as<WfScene>() + f;
-            wp.queue = r->wf_queue.as<unsigned int>() + f * kQueueWords;
-            wp.counters = r->counters.as<unsigned long long>();
+            wp.scenes = d_table + f;
+            wp.queue = d_queue + f * kQueueWords;
+            wp.counters = d_ctr;
             ATX_HIP(launch_in_place(wp, flat_only, r->stream));
             // Renderer.cu:245-248
             if (r->settings.accumulation) r->frame_index++;
@@ -234,13 +245,8 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         }
     }
     ATX_HIP(hipEventRecord(r->ev1, r->stream));
-    unsigned long long* ctr = r->readback;
-    ATX_HIP(hipMemcpyAsync(ctr, r->counters.get(), kCounterBytes, hipMemcpyDeviceToHost, r->stream));
-    const bool read_hits = use_first && !r->n_hit_exact;
-    uint32_t* n_hit_read = reinterpret_cast<uint32_t*>(r->readback + kCounterWords);
-    if (read_hits)
-        ATX_HIP(hipMemcpyAsync(n_hit_read, first_cache_view(r->wf_first.get(), npx, r->geo.n_light).n_hits,
-                               sizeof(uint32_t), hipMemcpyDeviceToHost, r->stream));
+    if (!wf)
+        ATX_HIP(hipMemcpyAsync(r->readback, d_ctr, kCounterBytes, hipMemcpyDeviceToHost, r->stream));
     if (dbg_rad) ATX_HIP(hipMemcpyAsync(dbg_rad, d_rad.get(), npx * sizeof(float4), hipMemcpyDeviceToHost, r->stream));
     if (dbg_hit) ATX_HIP(hipMemcpyAsync(dbg_hit, d_hit.get(), npx * dbg_bounces * 4, hipMemcpyDeviceToHost, r->stream));
     if (dbg_shadow) ATX_HIP(hipMemcpyAsync(dbg_shadow, d_sh.get(), npx * dbg_bounces * 4, hipMemcpyDeviceToHost, r->stream));
@@ -252,23 +258,28 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         path_ms = 0.0;
         for (size_t l = 0; l < table.size(); ++l) {
             float t = 0.0f;
-            ATX_HIP(hipEventElapsedTime(&t, r->wf_ev[2 * l], r->wf_ev[2 * l + 1]));
+            ATX_HIP(hipEventElapsedTime(&t, l > 0 ? r->wf_ev[2 * l] : r->ev0, r->wf_ev[2 * l + 1]));
             path_ms += t;
         }
     }
+    // the call's counts: left in the pinned block by the last launch, else
+    // summed from the lines
+    unsigned long long ctr[kCtrCount];
+    for (uint32_t k = 0; k < kCtrCount; ++k)
+        ctr[k] = wf ? r->readback[k] : counter_sum(r->readback, (CounterSlot)k);
     if (read_hits) {
-        r->n_hit = *n_hit_read;
+        r->n_hit = (uint32_t)r->readback[kCtrCount];
         r->n_hit_exact = true;
     }
     for (WfScene& e : table)
         if (e.hit_px) e.n_hit = r->n_hit;
     r->stats.samples = (uint64_t)npx * frames;
     const uint64_t skipped = wf ? skipped_primaries(table.data(), table.size()) : 0;
-    r->stats.reused_rays = counter_sum(ctr, kCtrReused) + skipped;
-    r->stats.rays = counter_sum(ctr, kCtrRays) + r->stats.reused_rays;
-    r->stats.sphere_tests = counter_sum(ctr, kCtrTests);
-    r->stats.exact_retraces = counter_sum(ctr, kCtrExact);
-    r->stats.box_tests = counter_sum(ctr, kCtrBoxes);
+    r->stats.reused_rays = ctr[kCtrReused] + skipped;
+    r->stats.rays = ctr[kCtrRays] + r->stats.reused_rays;
+    r->stats.sphere_tests = ctr[kCtrTests];
+    r->stats.exact_retraces = ctr[kCtrExact];
+    r->stats.box_tests = ctr[kCtrBoxes];
     r->stats.gpu_ms = ms;
     r->stats.launches = wf ? table.size() : frames;
     r->stats.path_ms = path_ms;
@@ -295,9 +306,8 @@ int atx_renderer_create(atx_renderer** out)
     hipError_t e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&r->ev0);
     if (e == hipSuccess) e = hipEventCreate(&r->ev1);
-    if (e == hipSuccess) e = r->counters.reserve(kCounterBytes);
     if (e == hipSuccess)
-        e = hipHostMalloc((void**)&r->readback, (kCounterWords + 1) * sizeof(unsigned long long), hipHostMallocDefault);
+        e = hipHostMalloc((void**)&r->readback, kCounterBytes, hipHostMallocDefault);
     if (e != hipSuccess) {
         set_error("renderer create: %s", hipGetErrorString(e));
         atx_renderer_destroy(reinterpret_cast<atx_renderer*>(r));

@@ -124,6 +124,10 @@ struct WfPass {
     uint32_t total_px;     // pixels of all scenes of the launch
     unsigned int* queue;   // this launch's chunk counters (kQueueWords, zero before launch)
     unsigned long long* counters;
+    // k_accumulate then leaves the counters' sums and, if given, *n_hits here
+    // (pinned host memory; nullptr: not)
+    unsigned long long* totals;
+    const uint32_t* n_hits;
     uint32_t refill_min;   // idle lanes a wave waits for before it hands out jobs (set by launch_wavefront)
     uint32_t pad_;
 };
