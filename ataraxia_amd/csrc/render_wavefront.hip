@@ -350,12 +350,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     // the trace runs: the state then needs no VGPRs there, and the trace fits
     // its register budget without spilling (17 KB of LDS per 256-lane
     // workgroup, 136 KB per CU at 8 waves per SIMD; a tile query's candidate
-    // masks take another 9 KB).
+    // masks take another 14 KB).
     constexpr bool kPark = kWaves >= 7 || kTree;
     constexpr uint32_t kParked = 17;
     __shared__ uint32_t parked_all[4][kPark ? kParked : 1][64];
     uint32_t(*parked)[64] = parked_all[threadIdx.x >> 6];
-    __shared__ uint32_t tile_masks[4][kTree ? kTileRows : 1][64];
+    constexpr uint32_t kChunk = kInPlace ? kTileChunkInPlace : kTileChunk;
+    __shared__ uint32_t tile_masks[4][kTree ? kChunk + 1 : 1][64];
     // in place: the pixel's primary direction and the frame its path is in
     __shared__ uint32_t own_all[4][kInPlace ? 4 : 1][64];
     uint32_t(*own)[64] = own_all[threadIdx.x >> 6];
@@ -636,7 +637,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             BvhQuery q;
             if (tree) {
                 const BvhDev B = S->bvh;
-                h = trace_tiles(B, flat, S->sph_mat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
+                h = trace_tiles<kChunk>(B, flat, S->sph_mat, S->n_sph, ro, rd, qd2, traces, tile_masks[threadIdx.x >> 6], q);
             } else {
                 if (kInPlace && S->exact)
                     h = trace_exact(flat, S->n_sph, ro, rd);
@@ -896,7 +897,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
     const float4 dv = s.dirs[px];
     const f3 rd = mk(dv.x, dv.y, dv.z);
     const SphSrc flat{as_const(s.sph)};
-    __shared__ uint32_t tile_masks[kFirstWaves][kTree ? kTileRows : 1][64];
+    __shared__ uint32_t tile_masks[kFirstWaves][kTree ? kTileChunk + 1 : 1][64];
     __shared__ uint32_t wave_hits[kFirstWaves], list_base;
     const BvhDev B = s.bvh;
     const f3 one = mk(1.0f, 1.0f, 1.0f);
@@ -928,7 +929,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
         if constexpr (kTree) {
             BvhQuery q;
             if (__any(act))   // a wave of missing pixels has no shadow rays
-                h = trace_tiles(B, flat, s.sph_mat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
+                h = trace_tiles<kTileChunk>(B, flat, s.sph_mat, s.n_sph, o, d, dist2, act, tile_masks[threadIdx.x >> 6], q);
             if (k == 0u) {
                 hit_sphere = q.sphere;
                 mid = q.mat;

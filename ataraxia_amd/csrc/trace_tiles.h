@@ -195,9 +195,9 @@ __device__ __forceinline__ bool tile_candidate(const BvhDev& B, float4 s, int32_
 
 // Closest hit (dist2 < 0) or shadow query (dist2 >= 0) of ray (o, d) of the
 // lanes with `act`; every lane of the wave must call it (the matrix products
-// and lane exchanges take all 64 lanes).  masks: kTileRows rows of this
+// and lane exchanges take all 64 lanes).  masks: kChunk + 1 rows of this
 // wave in LDS.  The result of the other lanes is a miss.
-template <class FlatSrc>
+template <uint32_t kChunk, class FlatSrc>
 __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat, const int32_t* sph_mat,
                                            uint32_t n_all, f3 o, f3 d, float dist2, bool act, uint32_t (*masks)[64], BvhQuery& q)
 {
@@ -287,7 +287,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
     const uint32_t n_tiles = B.n_tiles;
     const bool boxed = B.n_nodes != 0u, groups = n_tiles > kTileFlat;
     for (uint32_t t = 0; t < n_tiles;) {
-        // candidates of up to kTileChunk touched tiles
+        // candidates of up to kChunk touched tiles
         uint32_t nm = 0u, some = 0u;
         const float lim = act ? tlim * B.ts : -1.0f;   // a lane that does not act touches nothing
         for (;;) {
@@ -314,7 +314,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
                 touched = act ? (1u << nt) - 1u : 0u;
                 need = __any(act) ? (1u << nt) - 1u : 0u;
             }
-            if (nm + (uint32_t)__popc(need) > kTileChunk)
+            if (nm + (uint32_t)__popc(need) > kChunk)
                 break;   // no room: test the candidates so far, then come back
             while (need != 0u) {
                 const uint32_t k = (uint32_t)__builtin_ctz(need);
@@ -331,7 +331,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
                 tile_swap(m0, m1);   // both halves of this lane's own ray
                 const uint32_t keep = touch ? ~((m0 & 0xffffu) | (m1 << 16)) : 0u;
                 masks[nm][lane] = keep;
-                masks[kTileChunk][nm] = (t + k) * 32u;
+                masks[kChunk][nm] = (t + k) * 32u;
                 some |= keep != 0u ? 1u << nm : 0u;
                 ++nm;
             }
@@ -345,7 +345,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
                 const uint32_t k = (uint32_t)__builtin_ctz(some);
                 some &= some - 1u;
                 m = masks[k][lane];
-                base = masks[kTileChunk][k];
+                base = masks[kChunk][k];
             }
             const uint32_t k = base + (uint32_t)__builtin_ctz(m);
             m &= m - 1u;
