@@ -343,7 +343,6 @@ template <uint32_t kWaves, bool kTree, bool kInPlace = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const unsigned long long lanes_below = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
     const uint32_t P = a.chunk_px;
     // The instances for trees and for 7 and 8 resident waves per SIMD park the
     // path state that a trace does not read (17 values per lane) in LDS while
@@ -395,7 +394,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     // overflow); exact retraces (rare) straight to their counter
     unsigned long long rays = 0, reused = 0;
     uint32_t tests = 0, boxes = 0;
-    unsigned long long* const counters = a.counters + (wave_id % kCounterLines) * kCounterStride;
+    // not kept: computed where it is used
+    const auto counters = [&]() { return a.counters + (wave_id % kCounterLines) * kCounterStride; };
 
     // in place: starts pixel `job`'s path of the launch's frame f
     const auto start_in_place = [&](uint32_t f, f3 dir) {
@@ -431,7 +431,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 break;
             if (blk_next < blk_end) {
                 const uint32_t avail = blk_end - blk_next;
-                const uint32_t rank = (uint32_t)__popcll(idle & lanes_below);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
                 const uint32_t nidle = (uint32_t)__popcll(idle);
                 uint32_t cached_rays = 0;   // this lane's rays taken from the first-bounce cache
                 if constexpr (kInPlace) {
@@ -670,7 +671,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             }
             if (traces) {
                 if (q.exact)
-                    atomicAdd(counters + kCtrExact, (unsigned long long)q.exact);
+                    atomicAdd(counters() + kCtrExact, (unsigned long long)q.exact);
                 tests += q.tests;
                 boxes += q.boxes;
             }
@@ -723,7 +724,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 state = kNew;
         }
         if (__any(tests >= 0x80000000u || boxes >= 0x80000000u))
-            flush_counters(counters, lane, tests, boxes, 0ull, 0ull);
+            flush_counters(counters(), lane, tests, boxes, 0ull, 0ull);
         if (end_path) {
             state = kIdle;
             if constexpr (kInPlace) {
@@ -738,7 +739,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         }
     }
 
-    flush_counters(counters, lane, tests, boxes, rays, reused);
+    flush_counters(counters(), lane, tests, boxes, rays, reused);
 }
 
 // Adds every pixel's samples of the launch to its accumulation in frame order
@@ -875,19 +876,21 @@ struct FirstArgs {
 // A wave takes an 8 x 8 tile of pixels: its rays stay closer together than
 // along a 64-pixel row (1080p: 0.586 -> 0.556 ms), and the hit list then
 // runs tile by tile.
-// A workgroup of 8 waves appends its hits to the list with one atomic (one
-// per 11.6 ns on the device, whoever asks): one per wave bounded the kernel,
-// 1080p with 129 spheres 0.376 -> 0.308 ms, 640x360 with 4 0.042 -> 0.016 ms
-// (4 waves 0.319 and 0.020, 16 waves 0.343 and 0.015).
-constexpr uint32_t kFirstWaves = 8;
+// A workgroup appends its hits to the list with one atomic (one per 11.6 ns on
+// the device, whoever asks): one per wave bounded the kernel, 1080p with 129
+// spheres 0.376 -> 0.295 ms, 640x360 with 4 0.042 -> 0.016 ms.  With tiles 4 waves,
+// which wait less for each other (8: 0.311 ms; 1600x900, 8000 spheres 1.12 and
+// 1.19), else 8 (4: 0.020 ms, 16: 0.015).
 template <bool kTree>
-__global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
+constexpr uint32_t kFirstWaves = kTree ? 4 : 8;
+template <bool kTree>
+__global__ __launch_bounds__(kFirstWaves<kTree> * 64) void k_first_hit(FirstArgs a)
 {
     const WfScene& s = a.s;
     const uint32_t npx = s.width * s.height;
     // one 8 x 8 tile of pixels per wave
     const uint32_t tiles_x = (s.width + 7u) / 8u;
-    const uint32_t wave = blockIdx.x * kFirstWaves + (threadIdx.x >> 6);
+    const uint32_t wave = blockIdx.x * kFirstWaves<kTree> + (threadIdx.x >> 6);
     const uint32_t ty = wave / tiles_x, tx = wave - ty * tiles_x;
     const uint32_t x = tx * 8u + (threadIdx.x & 7u), y = ty * 8u + ((threadIdx.x >> 3) & 7u);
     // lanes past the image's edge stay for the wave's tile queries
@@ -897,8 +900,8 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
     const float4 dv = s.dirs[px];
     const f3 rd = mk(dv.x, dv.y, dv.z);
     const SphSrc flat{as_const(s.sph)};
-    __shared__ uint32_t tile_masks[kFirstWaves][kTree ? kTileChunk + 1 : 1][64];
-    __shared__ uint32_t wave_hits[kFirstWaves], list_base;
+    __shared__ uint32_t tile_masks[kFirstWaves<kTree>][kTree ? kTileChunk + 1 : 1][64];
+    __shared__ uint32_t wave_hits[kFirstWaves<kTree>], list_base;
     const BvhDev B = s.bvh;
     const f3 one = mk(1.0f, 1.0f, 1.0f);
     const f3 zero = mk(0.0f, 0.0f, 0.0f);
@@ -954,7 +957,7 @@ __global__ __launch_bounds__(kFirstWaves * 64) void k_first_hit(FirstArgs a)
                 wave_hits[w] = (uint32_t)__popcll(hm);
             __syncthreads();
             uint32_t base = 0, all = 0;
-            for (uint32_t i = 0; i < kFirstWaves; ++i) {
+            for (uint32_t i = 0; i < kFirstWaves<kTree>; ++i) {
                 const uint32_t n = wave_hits[i];
                 base += i < w ? n : 0u;
                 all += n;
@@ -1097,7 +1100,8 @@ hipError_t launch_first_hits(const WfScene& s, hipStream_t stream)
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, v.n_hits, 1u);
     const uint32_t tiles = ((s.width + 7u) / 8u) * ((s.height + 7u) / 8u);
     const auto kernel = s.bvh.n_tiles ? k_first_hit<true> : k_first_hit<false>;
-    hipLaunchKernelGGL(kernel, dim3((tiles + kFirstWaves - 1u) / kFirstWaves), dim3(kFirstWaves * 64u), 0, stream, a);
+    const uint32_t waves = s.bvh.n_tiles ? kFirstWaves<true> : kFirstWaves<false>;
+    hipLaunchKernelGGL(kernel, dim3((tiles + waves - 1u) / waves), dim3(waves * 64u), 0, stream, a);
     return hipGetLastError();
 }
 
