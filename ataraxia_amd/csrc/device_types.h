@@ -7,7 +7,7 @@
 //   sph_mat  int32[N]    material index (clamped to [0, M) on the host)
 //   mat      float4[3M]  (albedo, roughness) (F0, metallic)
 //                        (emission colour, emission intensity)
-//   light    float4[2L]  (position, intensity) (colour, 0)
+//   light    float4[2L]  (position, intensity) (colour * intensity, 0)
 // r*r is precomputed once; the reference evaluates radius*radius inside its
 // loop (Renderer.cu:264), which rounds to the same value.
 #pragma once

@@ -64,6 +64,7 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
         for (float v : in_unit)
             if (!(v >= 0.0f && v <= 1.0f)) out->unit_materials = false;
         if (a.roughness > 0.0f && a.roughness < 0x1p-10f) out->unit_materials = false;
+        if (a.emission_intensity > 0.0f) out->emits = true;
         for (int k = 0; k < 3; ++k)
             if (a.albedo[k] > 0.0f && a.albedo[k] < out->least_albedo) out->least_albedo = a.albedo[k];
     }
@@ -72,7 +73,9 @@ int build_scene_layout(const atx_sphere* spheres, uint64_t n, const atx_material
         const atx_light& a = lights[i];
         float* o = &out->light[8 * i];
         o[0] = a.position[0]; o[1] = a.position[1]; o[2] = a.position[2]; o[3] = a.intensity;
-        o[4] = a.color[0]; o[5] = a.color[1]; o[6] = a.color[2]; o[7] = 0.0f;
+        for (int k = 0; k < 3; ++k)
+            o[4 + k] = a.color[k] * a.intensity;
+        o[7] = 0.0f;
     }
     return ATX_OK;
 }
@@ -166,6 +169,7 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     out->n_light = (uint32_t)l;
     out->least_albedo = L.least_albedo;
     out->unit_materials = L.unit_materials;
+    out->emits = L.emits;
     out->bvh = pack.bvh(T, base);
     return ATX_OK;
 }

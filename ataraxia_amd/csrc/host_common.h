@@ -171,6 +171,7 @@ struct HostSceneLayout {
     // in [0, 1], the roughness not between 0 and 2^-10
     float least_albedo = 1.0f;
     bool unit_materials = true;
+    bool emits = false;   // some emission intensity is above zero
 };
 
 // Builds the device layout; ids outside [0, num_materials) are clamped to 0
@@ -209,7 +210,7 @@ struct DevScene {
     const int32_t* sph_mat = nullptr;
     uint32_t n_sph = 0, n_mat = 0, n_light = 0;
     float least_albedo = 1.0f;      // of HostSceneLayout
-    bool unit_materials = false;
+    bool unit_materials = false, emits = false;
     BvhDev bvh{};
     void use_pool(DevPool* pool) { block.use_pool(pool); }
     size_t bytes() const { return block.bytes(); }

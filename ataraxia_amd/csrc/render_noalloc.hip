@@ -132,6 +132,7 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     w.n_mat = (uint32_t)num_materials;
     w.n_light = (uint32_t)num_lights;
     w.mild = mild_materials(L.least_albedo, L.unit_materials, settings->max_bounces) ? 1u : 0u;
+    w.emits = L.emits ? 1u : 0u;
     w.bvh = pack.bvh(T, base);
     if (accel != ATX_ACCEL_BVH) w.bvh.n_nodes = 0;
     const bool kahan = accumulator == ATX_ACCUM_KAHAN;

@@ -84,7 +84,7 @@ struct BvhQuery {
     uint32_t tests = 0;   // sphere tests
     uint32_t boxes = 0;   // box tests
     uint32_t exact = 0;   // orders settled by exact distances, exact loops
-    // of the closest hit's sphere (tile queries that found one)
+    // of the closest hit's sphere (queries but shadow ones that found one)
     float4 sphere = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     int32_t mat = 0;
 };
@@ -195,11 +195,13 @@ __device__ __forceinline__ bool tile_candidate(const BvhDev& B, float4 s, int32_
 
 // Closest hit (dist2 < 0) or shadow query (dist2 >= 0) of ray (o, d) of the
 // lanes with `act`; every lane of the wave must call it (the matrix products
-// and lane exchanges take all 64 lanes).  masks: kChunk + 1 rows of this
-// wave in LDS.  The result of the other lanes is a miss.
+// and lane exchanges take all 64 lanes).  index: the id of a hit is to be the
+// sphere's index in the scene (else it is only not negative).  masks: kChunk + 1
+// rows of this wave in LDS.  The result of the other lanes is a miss.
 template <uint32_t kChunk, class FlatSrc>
 __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat, const int32_t* sph_mat,
-                                           uint32_t n_all, f3 o, f3 d, float dist2, bool act, uint32_t (*masks)[64], BvhQuery& q)
+                                           uint32_t n_all, f3 o, f3 d, float dist2, bool act, bool index,
+                                           uint32_t (*masks)[64], BvhQuery& q)
 {
     Hit h;
     h.id = -1;
@@ -340,7 +342,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
                 break;
         }
         // The next candidate's sphere is on its way while one is tested: whole
-        // calls 1080p, 129 spheres, 256 frames 19.41 -> 19.30 ms, 1600x900, 8000
+        // calls 1080p, 257 spheres, 256 frames 19.41 -> 19.30 ms, 1600x900, 8000
         // spheres 9.81 -> 9.74, 1280x720 in place 0.705 -> 0.697, batch of 12
         // scenes 48.9 -> 48.5.
         uint32_t m = 0u, base = 0u;
@@ -394,10 +396,19 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
         // one load less to wait for here, two in the shading and one before
         // the next direction, the path kernel went from 20.0 to 19.2 ms (1080p,
         // 129 spheres, 256 frames) and a batch of 12 scenes from 49.2 to 46.7.
-        q.sphere = tsph[f.best];
-        h.id = B.tidx[f.best];
-        q.mat = B.tmat ? B.tmat[f.best] : sph_mat[h.id];
-        h.t = exact_t(q.sphere, o, d, a);
+        // A shadow query needs nothing but t, and not its exact value where a
+        // bound above it already lies before the light.
+        const float above = f.best_hi * inv_a_up;
+        h.id = f.best;
+        h.t = above;
+        if (index || (!shadow && !B.tmat))
+            h.id = B.tidx[f.best];
+        if (!shadow)
+            q.mat = B.tmat ? B.tmat[f.best] : sph_mat[h.id];
+        if (!(shadow && above * above < dist2)) {
+            q.sphere = tsph[f.best];
+            h.t = exact_t(q.sphere, o, d, a);
+        }
     }
 #endif
     return h;

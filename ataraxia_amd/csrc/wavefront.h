@@ -68,6 +68,7 @@ struct WfScene {
     // 1: the materials and max_bounces are such that no quotient of a light
     // term or of a roulette can leave the normal range (mild_materials)
     uint32_t mild;
+    uint32_t emits;        // some material's emission intensity is above zero
     const float4* mat_rr;  // per material: albedo / p and p, the roulette at a path's first hit
     const float4* light;
     uint32_t n_sph;
@@ -253,7 +254,7 @@ hipError_t launch_camera_dirs(const WfScene& s, float4* dirs, hipStream_t stream
 //          lights), the hit's material;
 //      [1] normal x, y, z, origin of the rays leaving the hit x;
 //      [2] origin y, z, radiance after the hit's emission r, g;
-//      [3] radiance b, 0, 0, 0;
+//      [3] radiance b, the hit material's roughness and metallic, 0;
 //  * then, for scenes of 1..kFirstMaxLights lights, per light and pixel
 //    ([light][pixel]) the light's Cook-Torrance term at the hit (float4,
 //    w = 0; zero when the light does not reach the hit);

@@ -53,6 +53,7 @@ inline void fill_wf_scene(const DevScene& g, const atx_settings& st, const atx_c
     out->mat_rr = g.mat_rr;
     out->light = g.light;
     out->mild = mild_materials(g.least_albedo, g.unit_materials, st.max_bounces) ? 1u : 0u;
+    out->emits = g.emits ? 1u : 0u;
     out->n_sph = g.n_sph;
     out->n_mat = g.n_mat;
     out->n_light = g.n_light;
