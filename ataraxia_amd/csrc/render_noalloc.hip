@@ -140,21 +140,24 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     // index back at 1 after the first (Renderer.cu:245-248).  The entries stay
     // in place until their copies have run.
     const uint32_t launches = settings->accumulation ? 1u : frames;
-    std::vector<WfScene> entries(launches, w);
+    constexpr uint32_t kEntries = 64;
+    WfScene entries[kEntries];
     for (uint32_t l = 0; l < launches; ++l) {
-        WfScene& w = entries[l];
+        if (l != 0 && l % kEntries == 0) ATX_HIP(hipStreamSynchronize(stream));
+        WfScene& e = entries[l % kEntries];
+        e = w;
         const uint32_t n = settings->accumulation ? frames : 1u;
         const uint32_t fi = l == 0 ? first_frame : 1u;
         fill_wf_view(*settings, *cam, reinterpret_cast<float4*>(accum), kahan ? reinterpret_cast<float4*>(comp) : nullptr,
-                     image, kahan, fi, n, &w);
+                     image, kahan, fi, n, &e);
         WfPass p{};
-        ATX_CHECK_ARG(layout_in_place(w, &p), "viewport too large");
+        ATX_CHECK_ARG(layout_in_place(e, &p), "viewport too large");
         p.scenes = reinterpret_cast<const WfScene*>(base + off_table);
         p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
         p.counters = reinterpret_cast<unsigned long long*>(base + off_ctr);
-        ATX_HIP(put(off_table, &w, sizeof(w)));
+        ATX_HIP(put(off_table, &e, sizeof(e)));
         ATX_HIP(launch_zero_u32(p.queue, kQueueWords, stream));
-        ATX_HIP(launch_in_place(p, w.bvh.n_tiles == 0, stream));
+        ATX_HIP(launch_in_place(p, e.bvh.n_tiles == 0, stream));
     }
     // the host copies above read L and T, which end with this call
     ATX_HIP(hipStreamSynchronize(stream));

@@ -63,6 +63,9 @@ struct Renderer {
     atx_render_stats stats{};
 };
 
+// Queues of one call (16 lines each).
+constexpr uint32_t kRendererQueues = 1024;
+
 static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t frames, float* dbg_rad,
                                   int32_t* dbg_hit, int32_t* dbg_shadow, uint32_t dbg_bounces)
 {
@@ -196,9 +199,11 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     const uint32_t n_launch = (uint32_t)table.size();
     // The launches' table, their queues and the counters (both zero) are one
     // block, sent in one copy; as a copy, a fill kernel and a memset they
-    // took 35 us of a 320x180 call's 124.
+    // took 35 us of a 320x180 call's 124.  Past kRendererQueues launches (one
+    // frame each) a queue is cleared and used again.
+    const uint32_t n_queue = std::min(n_launch, kRendererQueues);
     const size_t off_queue = (n_launch * sizeof(WfScene) + 255) & ~size_t(255);
-    const size_t off_ctr = off_queue + n_launch * kQueueWords * sizeof(unsigned int);
+    const size_t off_ctr = off_queue + n_queue * kQueueWords * sizeof(unsigned int);
     r->launch_host.assign(off_ctr + kCounterBytes, 0);
     if (n_launch) memcpy(r->launch_host.data(), table.data(), n_launch * sizeof(WfScene));
     ATX_HIP(r->launch_dev.reserve(r->launch_host.size()));
@@ -207,6 +212,10 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     const WfScene* d_table = r->launch_dev.as<WfScene>();
     unsigned int* d_queue = reinterpret_cast<unsigned int*>(r->launch_dev.as<unsigned char>() + off_queue);
     unsigned long long* d_ctr = reinterpret_cast<unsigned long long*>(r->launch_dev.as<unsigned char>() + off_ctr);
+    const auto queue_of = [&](uint32_t l, unsigned int** q) {
+        *q = d_queue + (l % n_queue) * kQueueWords;
+        return l < n_queue ? hipSuccess : launch_zero_u32(*q, kQueueWords, r->stream);
+    };
     const bool read_hits = use_first && !r->n_hit_exact;
     ATX_HIP(hipEventRecord(r->ev0, r->stream));
     if (wf) {
@@ -217,7 +226,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             wp.total_chunks = table[l].n_chunks;
             wp.chunk_px = launch_chunk[l];
             wp.total_px = table[l].width * table[l].height;
-            wp.queue = d_queue + l * kQueueWords;
+            ATX_HIP(queue_of((uint32_t)l, &wp.queue));
             wp.counters = d_ctr;
             if (l + 1 == table.size()) {
                 wp.totals = r->readback;
@@ -236,7 +245,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         for (uint32_t f = 0; f < frames; ++f) {
             WfPass wp = passes[f];
             wp.scenes = d_table + f;
-            wp.queue = d_queue + f * kQueueWords;
+            ATX_HIP(queue_of(f, &wp.queue));
             wp.counters = d_ctr;
             ATX_HIP(launch_in_place(wp, flat_only, r->stream));
             // Renderer.cu:245-248
