@@ -132,7 +132,7 @@ extern "C" int atx_batch_autotune(atx_batch* h, const char* cache_path, atx_batc
         }
     }
     for (uint32_t w = kWfWavesMin; w <= kWfWavesMax; ++w) {
-        if (w == w0 || !flat) continue;   // launches with trees have one instance
+        if (w == w0 || !flat) continue;   // launches with tiles have one instance
         rc = try_one(atx_batch_tuning{best.chunk_px, wavefront_full_grid(flat, w), 1, best.frames_per_launch, w});
         if (rc != ATX_OK) {
             batch_set_subset(b, {});

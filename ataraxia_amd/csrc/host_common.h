@@ -228,7 +228,7 @@ struct DevScene {
 int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
                  const atx_light* lights, uint64_t l, DevScene* out);
 
-// Device bytes a scene of this size occupies (geometry and tree).
+// Device bytes a scene of this size occupies (geometry and tiles).
 size_t scene_device_bytes(uint64_t n, uint64_t m, uint64_t l);
 
 }  // namespace atx

@@ -65,7 +65,7 @@ ATX_HD float fabs_(float x) { return fabsf(x); }
 // quotient by the same divisor (Markstein, "Computation of elementary
 // functions on the IBM RISC System/6000 processor", 1990).  Path kernel: 640x360,
 // 4 spheres, 64 frames 0.409 -> 0.383 ms (14.5 % fewer vector instructions),
-// 1080p, 129 spheres, 256 frames 20.6 -> 20.1 ms (5 % fewer).
+// 1080p, 257 spheres, 256 frames 20.6 -> 20.1 ms (5 % fewer).
 
 // sqrt(d) from y, 1 / sqrt(d) to one ulp; h: half its inverse, closer than y.
 ATX_HD float sqrt_from(float d, float y, float& h)

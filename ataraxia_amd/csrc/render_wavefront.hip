@@ -23,7 +23,7 @@
 // times the launch's frames, frame after frame inside a group
 // (job_pixel_frame), so a wave traces 8 neighbouring pixels in many frames
 // at once: their rays start from the same few hits, which keeps the lanes of
-// a wave on nearby tree nodes and makes whole waves miss the same spheres in
+// a wave near the same spheres and makes whole waves miss the same spheres in
 // the flat loop.  Samples are stored in job order: a wave's block of jobs
 // fills whole 128-byte lines of the sample buffer, which no other wave
 // touches, and k_accumulate reads a pixel's frames 8 samples apart.
@@ -37,7 +37,7 @@
 // path at once.  With the cache's hit list, jobs cover only the pixels
 // whose primary ray hits; k_accumulate adds the others' constant sample.
 //
-// Rays of scenes with a tree are traced by whole waves (trace_tiles.h): all 64
+// Rays of scenes with tiles are traced by whole waves (trace_tiles.h): all 64
 // lanes go through a query together, those without a ray as well.  In scenes
 // without one every ray tests every sphere.  Spheres, boxes and the scene
 // table are read with wave-uniform addresses through the constant address
@@ -46,7 +46,7 @@
 //
 // Registers: launches whose scenes all use the flat loop have an instance for
 // each of 5 to 8 resident waves per SIMD (amdgpu_waves_per_eu; 7 by default),
-// launches with trees one for 5 (kWfWavesTree).
+// launches with tiles one for 5 (kWfWavesTree).
 #include "device_types.h"
 #include "trace_device.h"
 #include "trace_tiles.h"
@@ -328,14 +328,14 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
 // kernel with one lane per pixel and frame, 64 pixels to a wave until its
 // longest path ended, took 0.62 ms per frame at 1280x720 with 129 spheres;
 // here lanes go on with their next frame or another pixel: a call of 4 frames
-// 2.68 -> 0.81 ms.  The tree instance is bound like
+// 2.68 -> 0.81 ms, 0.65 with the steps since.  The tile instance is bound like
 // the sampling one, by VALU issue.
 template <uint32_t kWaves, bool kTree, bool kInPlace = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t P = a.chunk_px;
-    // The instances for trees and for 7 and 8 resident waves per SIMD park the
+    // The instances for tiles and for 7 and 8 resident waves per SIMD park the
     // path state that a trace does not read (17 values per lane) in LDS while
     // the trace runs: the state then needs no VGPRs there, and the trace fits
     // its register budget without spilling (17 KB of LDS per 256-lane
@@ -880,7 +880,7 @@ struct FirstArgs {
 // along a 64-pixel row (1080p: 0.586 -> 0.556 ms), and the hit list then
 // runs tile by tile.
 // A workgroup appends its hits to the list with one atomic (one per 11.6 ns on
-// the device, whoever asks): one per wave bounded the kernel, 1080p with 129
+// the device, whoever asks): one per wave bounded the kernel, 1080p with 257
 // spheres 0.376 -> 0.295 ms, 640x360 with 4 0.042 -> 0.016 ms.  With tiles 4 waves,
 // which wait less for each other (8: 0.311 ms; 1600x900, 8000 spheres 1.12 and
 // 1.19), else 8 (4: 0.020 ms, 16: 0.015).

@@ -105,7 +105,7 @@ struct Server {
     size_t samples_shares = 0;      // the charged requests' shares of it
     size_t samples_excess = 0;      // its capacity beyond those, charged to hbm_in_use
     double rendered = 0.0, busy_s = 0.0;   // samples rendered and GPU seconds so far (worker)
-    // persistent grids: ticks with trees, flat-loop-only ticks
+    // persistent grids: ticks with tiles, flat-loop-only ticks
     uint32_t grid = 0, grid_flat = 0;
     int device = 0;
 };
@@ -120,7 +120,7 @@ static double now_s(const Server* s)
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - s->epoch).count();
 }
 
-// Device bytes a request holds while admitted: scene, tree, accumulation,
+// Device bytes a request holds while admitted: scene, tiles, accumulation,
 // compensation, image, primary ray directions, first-bounce cache, and its
 // share of the tick's sample buffer.
 static size_t sample_share(const Request& r, uint32_t frames_per_tick)

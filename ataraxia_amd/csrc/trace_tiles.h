@@ -13,7 +13,7 @@
 // and a negative value rules the pair out.  The few spheres that are kept go
 // through filter_sphere like the flat loop's.
 //
-// Units.  Coordinates are relative to the centre of the tree's spheres and
+// Units.  Coordinates are relative to the centre of the tiles' spheres and
 // scaled by ts, a power of two, so that every sphere lies within 8 of the
 // origin.  A number x enters the product as two half-precision numbers
 // hi + lo; hi takes the upper 11 bits of x, so x - hi is exact.
@@ -53,10 +53,14 @@
 // then some occluder, not necessarily the closest.  Without boxes (n_nodes 0:
 // ATX_ACCEL_NONE) the product tests every sphere.
 //
-// What bounds it: VALU issue (0.31 instructions per cycle and SIMD in the path
+// What bounds it: VALU issue (0.30 instructions per cycle and SIMD in the path
 // kernel; minima, compares and shifts run at half the rate of multiply-adds),
-// at 5 waves per SIMD.  A 32x32x32 product takes about 66 cycles of a SIMD, and
-// the 16 shifts that collect its signs run beside it; with the two-product
+// at 5 waves per SIMD, which spend 39 % of their time issuing, 30 % waiting to
+// issue and 31 % waiting for data; loading the next tile's operands early
+// changed nothing (19.25 ms per 256 frames of 1080p both ways).  A 32x32x32 product takes about 66 cycles of a SIMD, and
+// the 16 shifts that collect its signs run beside it (one conversion of both
+// products to 6-bit floats instead of 32 shifts is a third shorter by itself,
+// but needs both at once: 18.0 -> 22.1 ms); with the two-product
 // form (b and |o - c|^2 - r^2, 2 VALU instructions per pair) it was 125.  All
 // control flow is wave-uniform but the candidates' loop (0.3 to 1.4 per ray, 4
 // to 5 in the slowest of 64 lanes at 64 to 512 spheres).  Against the per-lane
@@ -395,7 +399,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
         // material's index, the material and the light one after another.  With
         // one load less to wait for here, two in the shading and one before
         // the next direction, the path kernel went from 20.0 to 19.2 ms (1080p,
-        // 129 spheres, 256 frames) and a batch of 12 scenes from 49.2 to 46.7.
+        // 257 spheres, 256 frames) and a batch of 12 scenes from 49.2 to 46.7.
         // A shadow query needs nothing but t, and not its exact value where a
         // bound above it already lies before the light.
         const float above = f.best_hi * inv_a_up;

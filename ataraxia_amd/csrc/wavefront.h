@@ -84,7 +84,7 @@ struct WfScene {
     uint32_t n_chunks;     // ceil(width * height * frames / chunk_px)
     uint32_t kahan;        // 1: compensated accumulation (comp must be valid)
     uint32_t dbg_bounces;  // stride of the debug arrays
-    uint32_t exact;        // in-place launches without a tree: exact closest-hit loop
+    uint32_t exact;        // in-place launches without tiles: exact closest-hit loop
     uint32_t px_begin;     // first pixel of this scene in the launch's pixel range
     float inv_proj[16];
     float inv_view[16];
@@ -208,10 +208,11 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
 
 // Resident waves per SIMD the path kernel's registers are budgeted for.
 // Launches whose scenes all use the flat loop have an instance for each of 5
-// to 8 (the batch autotuner tries them all).  Launches with trees have one,
+// to 8 (the batch autotuner tries them all).  Launches with tiles have one,
 // for 5: a tile query holds 16 sums, 24 operands and its ray, which takes 96
-// VGPRs; the same kernel budgeted for 6 waves (80 VGPRs) spills 19 of them
-// (1080p, 256 frames: 20.0 ms of path kernel with 5, 23.2 with 6).
+// VGPRs; the same kernel budgeted for 6 waves (80 VGPRs) spills 33 of them
+// (1080p, 256 frames: 18.96 ms of path kernel with 5, 21.54 with 6, 20.81 with
+// 4).
 constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
@@ -226,7 +227,7 @@ __host__ __device__ __forceinline__ uint32_t wf_waves(uint32_t waves, bool flat_
 
 struct WfLaunch {
     uint32_t workgroups;     // persistent grid size (256-lane workgroups)
-    bool flat_only = false;  // no scene of the launch has a tree
+    bool flat_only = false;  // no scene of the launch has tiles
     uint32_t waves = 0;      // kernel instance (resident waves per SIMD); 0 = default
 };
 

@@ -184,7 +184,7 @@ inline uint32_t wavefront_full_grid(bool flat_only, uint32_t waves = 0)
     return device_cus() * (uint32_t)wavefront_max_blocks_per_cu(flat_only, waves);
 }
 
-// True when no scene of the table has a tree or tiles (the flat-loop instances)
+// True when no scene of the table has tiles (the flat-loop instances)
 inline bool wf_flat_only(const WfScene* tab, size_t n)
 {
     for (size_t k = 0; k < n; ++k)
@@ -226,8 +226,8 @@ inline uint32_t launch_chunk_px(uint64_t jobs, uint32_t workgroups, bool flat_on
 // advances this many frames per launch).
 constexpr uint32_t kDefaultFramesPerLaunch = 64;
 // Frames per launch of the single-scene renderer.  Every launch of the
-// persistent kernel costs about 0.7 ms beyond its paths (ramp-up and
-// drain; 1080p: 10.75 ms for 64 frames, 5.73 ms for 32), so a render call
+// persistent kernel costs its ramp-up and drain beyond its paths (an earlier
+// path kernel at 1080p: 10.75 ms for 64 frames, 5.73 ms for 32), so a render call
 // takes as few launches as its sample buffer allows: 1080p, 256 frames per
 // launch, 0.172 -> 0.160 ms per frame against 64.
 constexpr uint32_t kRendererFramesPerLaunch = 256;

@@ -6,7 +6,7 @@ Default workload (the metric's configuration), ``--workload plain_1080p``:
 scene from the seeded generator.  One "step" is one frame (one path sample
 for every pixel).  `value` is the single-scene renderer's production path:
 the persistent wavefront kernel (several frames per launch) with the sphere
-BVH.  The plain one-lane-per-pixel kernel and the flat loop over all spheres
+tiles.  The plain one-lane-per-pixel kernel and the flat loop over all spheres
 (the reference's algorithm) are timed on the same frames and reported in
 `variants`.  All four produce bit-identical images.
 
@@ -29,7 +29,7 @@ Other workloads (one JSON line each):
                          WRITE_SIZE counters
 
 The roofline entry is the VALU bound of the dominant kernel: 17 algorithmic
-FLOP per ray-sphere test and 12 per BVH node box test (6 FMA; FMA = 2), both
+FLOP per ray-sphere test and 12 per box test (6 FMA; FMA = 2), both
 counted exactly by the kernels, divided by that kernel's average launch
 duration from HIP events recorded on the renderer's stream around the path
 kernel alone (the persistent kernel's launches are each followed by a short
@@ -66,7 +66,7 @@ def parse():
     ap.add_argument("--exact-loop", action="store_true", help="use the exact (slow) closest-hit loop")
     ap.add_argument("--kernel", choices=["plain", "wavefront", "both"], default="both")
     ap.add_argument("--accel", choices=["bvh", "none", "both"], default="both",
-                    help="sphere BVH, flat loop over all spheres, or both")
+                    help="sphere tiles, every sphere for every ray, or both")
     ap.add_argument("--scenes", type=int, default=64, help="batch_mix: number of scenes")
     ap.add_argument("--tuning", default=None,
                     help="batch_mix: fixed chunk_px,workgroups,frames_per_launch instead of the autotuner")
@@ -220,7 +220,7 @@ def bench_plain_1080p(args):
         for a in accels:
             wall, st = time_single_scene(sc, kid[k], aid[a], args.steps, args.warmup)
             frames_per_launch = args.steps / max(1, st["launches"])
-            traffic, basis = traffic_from_profile(f"plain_1080p_k_render_{k}_{a}", f"k_render_{k}",
+            traffic, basis = traffic_from_profile(f"plain_1080p_k_render_{k}_{a}", "k_render_wavefront",
                                                   int(round(frames_per_launch)))
             variants[f"{k}/{a}"] = {"value": samples / wall, "ms_per_step": wall * 1e3 / args.steps,
                                     "gpu_ms_per_step": st["gpu_ms"] / args.steps,

@@ -323,7 +323,7 @@ public:
     // off).  Here the scene is flattened at those points as in the reference,
     // and uploaded only when the flattened spheres, materials or lights differ
     // from what the device holds: the device then holds exactly what the
-    // reference's upload would give, without rebuilding the sphere tree and
+    // reference's upload would give, without rebuilding the sphere tiles and
     // the first-bounce cache every frame.
     void Render(Camera& camera, const Scene& scene)
     {
@@ -346,7 +346,7 @@ public:
         const atx_camera c = camera.desc();
         check(atx_renderer_render(m_r, &c));
     }
-    // Scene uploads so far (each one rebuilds the device scene and its tree).
+    // Scene uploads so far (each one rebuilds the device scene and its tiles).
     uint64_t sceneUploads() const { return m_uploads; }
     // The RGBA8 pixels the reference uploads to its Vulkan Image.
     std::vector<uint32_t> getImage() const

@@ -100,7 +100,7 @@ ATX_STATIC_ASSERT(sizeof(atx_camera) == 44 && offsetof(atx_camera, fov_deg) == 2
 #define ATX_ACCUM_KAHAN 1
 
 /* Which spheres a ray tests (Renderer.cu:251-285 tests all of them).  BVH
- * (the default) walks a bounding-volume hierarchy built at scene upload and
+ * (the default) skips groups of spheres by boxes built at scene upload and
  * gives the same closest hit, bit for bit, including the lowest index among
  * equal distances; NONE tests every sphere.  Scenes with fewer than 16
  * spheres always use the flat loop.                                         */
@@ -114,7 +114,7 @@ typedef struct atx_render_stats {
                                 + shadow (as the reference traces them)         */
     uint64_t sphere_tests;   /* ray-sphere tests performed                      */
     uint64_t exact_retraces; /* traces resolved by the exact fallback loop      */
-    uint64_t box_tests;      /* ray-box tests of BVH nodes                      */
+    uint64_t box_tests;      /* ray-box tests                                   */
     double gpu_ms;           /* HIP-event time of the render kernels            */
     uint64_t launches;       /* path-kernel launches                            */
     double path_ms;          /* HIP-event time of the path kernel alone, summed
@@ -194,7 +194,7 @@ int atx_renderer_reserve(atx_renderer* r, uint32_t frames);
  * accumulation from zero).  The caller passes device buffers of width*height
  * entries: accum (4 floats per pixel), comp (4 floats per pixel, Kahan only,
  * else may be NULL) and image (RGBA8).  The scene (copied from host memory),
- * its sphere tree and the kernel's counters go into a fixed 8 MiB device
+ * its tiles and the kernel's counters go into a fixed 8 MiB device
  * array that the library holds per device for the life of the process; a
  * scene that needs more returns ATX_ERR_INVALID.  No device or pinned host
  * memory is allocated.  Work is queued on `stream` (a hipStream_t, NULL =
@@ -231,8 +231,8 @@ typedef struct atx_batch_tuning {
     uint32_t use_graph;         /* capture all launches in a HIP graph and replay it       */
     uint32_t frames_per_launch; /* frames each launch renders per scene (0 = 64)           */
     uint32_t waves_per_simd;    /* the path kernel's register budget: resident waves per
-                                   SIMD it is compiled for, 5..8 (0 = 6 with trees, 7 for
-                                   flat loops only); the launch bounds the autotuner picks */
+                                   SIMD it is compiled for, 5..8 (0 = the default, 7);
+                                   launches with tiles have one instance, for 5        */
 } atx_batch_tuning;
 
 typedef struct atx_batch atx_batch;
