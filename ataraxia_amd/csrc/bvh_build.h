@@ -21,8 +21,9 @@ constexpr uint32_t kTileWords = 512;     // 32-bit words of one tile
 // each (and one row for their first spheres): as many as leave room for five
 // workgroups on a CU.  1600x900, 8000 spheres: path kernel 9.13 -> 8.88 ms with
 // 13 instead of 8; 1024x1024, 512 spheres 3.00 -> 2.91; 1080p, 257 spheres, one
-// visit to four tiles, the same.  In-place launches hold 4 KB more themselves.
-constexpr uint32_t kTileChunk = 13, kTileChunkInPlace = 9;
+// visit to four tiles, the same.  In-place launches hold 4 KB more themselves, 6
+// with kept hits; a round of eight tiles has to fit.
+constexpr uint32_t kTileChunk = 13, kTileChunkInPlace = 9, kTileChunkKeep = 8;
 constexpr uint32_t kTileFlat = 16;       // with more tiles, every eight have a box of their own
 constexpr uint32_t kBvhGrid = 65535;     // node boxes are 16-bit cells of the tree's box
 

@@ -158,7 +158,7 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
             ATX_HIP(hipMemcpyAsync(base + off_table, &e, sizeof(e), hipMemcpyHostToDevice, stream));
             ATX_HIP(launch_zero_u32(p.queue, kQueueWords, stream));
         }
-        ATX_HIP(launch_in_place(p, e.bvh.n_tiles == 0, stream));
+        ATX_HIP(launch_in_place(p, e.bvh.n_tiles == 0, n, stream));
     }
     // the host copies above read L and T, which end with this call
     ATX_HIP(hipStreamSynchronize(stream));

@@ -57,7 +57,7 @@
 namespace atx {
 namespace {
 
-constexpr uint32_t kIdle = 0, kCont = 1, kShadow = 2, kNew = 3;
+constexpr uint32_t kIdle = 0, kCont = 1, kShadow = 2, kNew = 3, kAgain = 4;
 
 // The scene table and the sphere arrays do not change during a launch; read
 // through the constant address space, wave-uniform loads from them become
@@ -287,24 +287,26 @@ __device__ __forceinline__ uint32_t display(float4 acc, uint32_t frame)
                  gclamp(acc.w / fi, 0.0f, 1.0f));
 }
 
-// In-place launches: the sample of pixel px in frame f of the launch goes to
-// the accumulation; the last frame's also to the image.
-__device__ __forceinline__ void add_sample(CScene* S, uint32_t px, uint32_t f, f3 col)
+// In-place launches: the sample of pixel px, the same in n frames of the
+// launch from f on, goes to the accumulation; the last frame's also to the image.
+__device__ __forceinline__ void add_sample(CScene* S, uint32_t px, uint32_t f, uint32_t n, f3 col)
 {
     const uint32_t frame = S->frame0 + f;
     const bool kahan = S->kahan != 0u;
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float4 acc = frame == 1u ? zero : S->accum[px];
     float4 c = kahan && frame != 1u ? S->comp[px] : zero;
-    accumulate(kahan, col.x, acc.x, c.x);
-    accumulate(kahan, col.y, acc.y, c.y);
-    accumulate(kahan, col.z, acc.z, c.z);
-    accumulate(kahan, 1.0f, acc.w, c.w);
+    for (uint32_t k = 0; k < n; ++k) {
+        accumulate(kahan, col.x, acc.x, c.x);
+        accumulate(kahan, col.y, acc.y, c.y);
+        accumulate(kahan, col.z, acc.z, c.z);
+        accumulate(kahan, 1.0f, acc.w, c.w);
+    }
     S->accum[px] = acc;
     if (kahan)
         S->comp[px] = c;
-    if (f + 1u == S->frames) {
-        S->image[px] = display(acc, frame);
+    if (f + n == S->frames) {
+        S->image[px] = display(acc, frame + n - 1u);
         if (S->dbg_radiance)
             S->dbg_radiance[px] = make_float4(col.x, col.y, col.z, 1.0f);
     }
@@ -328,27 +330,33 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
 // kernel with one lane per pixel and frame, 64 pixels to a wave until its
 // longest path ended, took 0.62 ms per frame at 1280x720 with 129 spheres;
 // here lanes go on with their next frame or another pixel: a call of 4 frames
-// 2.68 -> 0.81 ms, 0.65 with the steps since.  The tile instance is bound like
+// 2.68 -> 0.81 ms, 0.63 with the steps since.  The tile instance is bound like
 // the sampling one, by VALU issue.
-template <uint32_t kWaves, bool kTree, bool kInPlace = false>
+// kKeep: a pixel's primary hit is the same in every frame, so its lane keeps it
+// and the frames after the first start at its shadow ray.  From three frames on
+// with tiles (1280x720, 129 spheres: 1 frame 266 us without and 281 with it, 2
+// frames 393 and 400, 4 frames 635 and 602, 8 frames 1175 and 965), always
+// without (8 spheres: 1 frame 199 and 179, 4 frames 393 and 339).
+template <uint32_t kWaves, bool kTree, bool kInPlace = false, bool kKeep = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t P = a.chunk_px;
-    // The instances for tiles and for 7 and 8 resident waves per SIMD park the
+    // The instances for tiles, in place and for 7 and 8 resident waves per SIMD park the
     // path state that a trace does not read (17 values per lane) in LDS while
     // the trace runs: the state then needs no VGPRs there, and the trace fits
     // its register budget without spilling (17 KB of LDS per 256-lane
     // workgroup, 136 KB per CU at 8 waves per SIMD; a tile query's candidate
     // masks take another 14 KB).
-    constexpr bool kPark = kWaves >= 7 || kTree;
+    constexpr bool kPark = kWaves >= 7 || kTree || kInPlace;
     constexpr uint32_t kParked = 17;
     __shared__ uint32_t parked_all[4][kPark ? kParked : 1][64];
     uint32_t(*parked)[64] = parked_all[threadIdx.x >> 6];
-    constexpr uint32_t kChunk = kInPlace ? kTileChunkInPlace : kTileChunk;
+    constexpr uint32_t kChunk = kKeep ? kTileChunkKeep : kInPlace ? kTileChunkInPlace : kTileChunk;
     __shared__ uint32_t tile_masks[4][kTree ? kChunk + 1 : 1][64];
-    // in place: the pixel's primary direction and the frame its path is in
-    __shared__ uint32_t own_all[4][kInPlace ? 4 : 1][64];
+    // in place: the pixel's primary direction, the frame its path is in, and the
+    // primary ray's hit (sphere, t) if kept
+    __shared__ uint32_t own_all[4][kKeep ? 6 : kInPlace ? 4 : 1][64];
     uint32_t(*own)[64] = own_all[threadIdx.x >> 6];
 
     // ---- wave-uniform scheduling state ----
@@ -406,6 +414,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     };
 
     for (;;) {
+        if constexpr (kKeep) {
+            // Frames that start at a known primary hit: once a quarter of the
+            // lanes that have a path wait for it, so that its shading runs for
+            // several at a time but the last few do not wait for each other.
+            const uint32_t again = (uint32_t)__popcll(__ballot(state == kAgain));
+            if (again != 0u && 4u * again >= (uint32_t)__popcll(__ballot(state != kIdle)) && state == kAgain) {
+                start_in_place(own[3][lane], mk(__uint_as_float(own[0][lane]), __uint_as_float(own[1][lane]),
+                                                __uint_as_float(own[2][lane])));
+                Hit h;
+                h.id = (int32_t)own[4][lane];
+                h.t = __uint_as_float(own[5][lane]);
+                f3 so, L;
+                mid = S->sph_mat[h.id];
+                shade_hit(S, as_const(S->sph)[h.id], mid, h, ro, rd, tp, seed, col, nrm, so, lidx, L, dist2);
+                vd = rd;
+                ro = so;
+                rd = L;
+                state = kShadow;
+            }
+        }
         // ---------------- hand jobs to idle lanes (uniform control flow) ----------------
         for (;;) {
             const unsigned long long idle = __ballot(state == kIdle);
@@ -631,7 +659,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             BvhQuery q;
             if (tree) {
                 const BvhDev B = S->bvh;
-                h = trace_tiles<kChunk>(B, flat, S->sph_mat, S->n_sph, ro, rd, qd2, traces, capture,
+                h = trace_tiles<kChunk>(B, flat, S->sph_mat, S->n_sph, ro, rd, qd2, traces,
+                                        capture || (kKeep && bounce == 0),
                                         tile_masks[threadIdx.x >> 6], q);
             } else {
                 if (kInPlace && S->exact)
@@ -677,6 +706,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             if (!shadow) {
                 if (capture && S->dbg_hit && (uint32_t)bounce < S->dbg_bounces)
                     S->dbg_hit[(size_t)pixel() * S->dbg_bounces + bounce] = h.id;
+                if (kKeep && bounce == 0) {
+                    own[4][lane] = (uint32_t)h.id;
+                    own[5][lane] = __float_as_uint(h.t);
+                }
                 if (h.id < 0) {
                     if (S->sky_light)
                         col = add(col, mul(mk(0.6f, 0.7f, 0.9f), tp));
@@ -732,10 +765,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
             state = kIdle;
             if constexpr (kInPlace) {
                 const uint32_t f = own[3][lane];
-                add_sample(S, job, f, col);
-                if (f + 1u < S->frames)
-                    start_in_place(f + 1u, mk(__uint_as_float(own[0][lane]), __uint_as_float(own[1][lane]),
-                                              __uint_as_float(own[2][lane])));
+                // the debug captures trace every ray; without lights the hit's
+                // bounce ends where it is shaded
+                const bool known = kKeep && S->n_light != 0 && S->max_bounces > 0 && !S->dbg_hit && !S->dbg_shadow;
+                const bool miss = known && (int32_t)own[4][lane] < 0;
+                const uint32_t n = miss ? S->frames - f : 1u;
+                add_sample(S, job, f, n, col);
+                if (f + n < S->frames) {
+                    own[3][lane] = f + n;
+                    if (known)
+                        state = kAgain;
+                    else
+                        start_in_place(f + n, mk(__uint_as_float(own[0][lane]), __uint_as_float(own[1][lane]),
+                                                 __uint_as_float(own[2][lane])));
+                }
             } else {
                 store_sample(S, slots, job, col);
             }
@@ -1053,14 +1096,15 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_in_place(const WfPass& pass, bool flat_only, hipStream_t stream)
+hipError_t launch_in_place(const WfPass& pass, bool flat_only, uint32_t frames, hipStream_t stream)
 {
     WfPass p = pass;
     p.refill_min = kRefillMin;
     if (p.total_chunks == 0 || p.n_scenes != 1)
         return hipErrorInvalidValue;
-    const PathKernel kernel = flat_only ? k_render_wavefront<kWfWavesFlat, false, true>
-                                        : k_render_wavefront<kWfWavesTree, true, true>;
+    const PathKernel kernel = flat_only ? k_render_wavefront<kWfWavesInPlace, false, true, true>
+                              : frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
+                                                      : k_render_wavefront<kWfWavesTree, true, true>;
     int dev = 0, cus = 0, blocks = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);

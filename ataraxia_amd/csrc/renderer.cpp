@@ -247,7 +247,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             wp.scenes = d_table + f;
             ATX_HIP(queue_of(f, &wp.queue));
             wp.counters = d_ctr;
-            ATX_HIP(launch_in_place(wp, flat_only, r->stream));
+            ATX_HIP(launch_in_place(wp, flat_only, 1, r->stream));
             // Renderer.cu:245-248
             if (r->settings.accumulation) r->frame_index++;
             else r->frame_index = 1;

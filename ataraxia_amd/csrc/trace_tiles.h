@@ -207,6 +207,7 @@ __device__ __forceinline__ Hit trace_tiles(const BvhDev& B, const FlatSrc& flat,
                                            uint32_t n_all, f3 o, f3 d, float dist2, bool act, bool index,
                                            uint32_t (*masks)[64], BvhQuery& q)
 {
+    static_assert(kChunk >= 8u, "a round's eight tiles have to fit");
     Hit h;
     h.id = -1;
     h.t = FLT_MAX;

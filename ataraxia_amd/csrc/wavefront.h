@@ -215,6 +215,8 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
 // 4).
 constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
+constexpr uint32_t kWfWavesInPlace = 6;   // flat scenes in place (79 VGPRs)
+constexpr uint32_t kKeepFrames = 3;       // in place with tiles: primary hits are kept from here on
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
 // The instance a launch uses: `waves` when it names a compiled instance,
 // else the default for its scenes.
@@ -239,7 +241,7 @@ hipError_t launch_wavefront(const WfPass& p, const WfLaunch& l, hipStream_t stre
 // laid out by layout_in_place): every pixel's frames one after another in one
 // lane, added to the accumulation as they end.  It needs neither samples nor
 // a first-bounce cache, so no memory beyond the scene's and the image's.
-hipError_t launch_in_place(const WfPass& p, bool flat_only, hipStream_t stream);
+hipError_t launch_in_place(const WfPass& p, bool flat_only, uint32_t frames, hipStream_t stream);
 hipError_t launch_zero_u32(unsigned int* p, uint32_t n, hipStream_t stream);
 // Writes the primary ray direction of every pixel of s's camera to dirs
 // (width * height float4, w = 0): camera_ray, computed once instead of per path.
