@@ -5,9 +5,9 @@
 // launch for all frames of the call), with the results of
 // atx_renderer_render_frames, but allocates no device memory: the caller
 // passes the accumulation, compensation and image buffers, and everything else
-// the kernel reads (the scene in its device layout, its tiles, the table entry,
-// the queue and the statistics counters) lives in one file-scope device array,
-// `scratch`, of kScratchBytes.  It is for callers that cannot call hipMalloc
+// the kernel reads besides its arguments (the scene in its device layout, its
+// tiles, the queue and the statistics counters) lives in one file-scope device
+// array, `scratch`, of kScratchBytes.  It is for callers that cannot call hipMalloc
 // (serving loops, harnesses that forbid allocation).
 //
 // Each device holds its own copy of `scratch` for the life of the process,
@@ -30,7 +30,7 @@ namespace atx {
 namespace {
 
 constexpr size_t kScratchBytes = 8u << 20;   // per device: 8 MiB for the scene
-constexpr size_t kControlBytes = 8192;       // and two pages for counters, queue and table entry, before it
+constexpr size_t kControlBytes = 4096;       // and a page for counters and queue, before it
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes + kControlBytes];
@@ -53,8 +53,6 @@ int scratch_address(int dev, unsigned char** out)
     *out = static_cast<unsigned char*>(g_scratch_ptr[dev]);
     return ATX_OK;
 }
-
-size_t align256(size_t v) { return (v + 255u) & ~(size_t)255u; }
 
 }  // namespace
 }  // namespace atx
@@ -91,12 +89,11 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
         kScratchBytes)
         T = HostBvh();
 
-    // scratch layout: counters | queue | table entry, then from kControlBytes on
+    // scratch layout: counters | queue, then from kControlBytes on
     // spheres | material ids | materials | lights | tiles
-    const size_t off_queue = align256(kCounterBytes);
-    const size_t off_table = align256(off_queue + kQueueWords * sizeof(unsigned int));
-    static_assert(kCounterBytes + kQueueWords * sizeof(unsigned int) + sizeof(WfScene) + 3 * 256 <= kControlBytes,
-                  "control pages");
+    const size_t off_queue = kCounterBytes;
+    static_assert(kCounterBytes % 256 == 0 && kCounterBytes + kQueueWords * sizeof(unsigned int) <= kControlBytes,
+                  "control page");
     const ScenePack pack(L, T, false, 256);   // as many spheres as fit
     const size_t total = pack.bytes;
     if (total > kScratchBytes) {
@@ -127,40 +124,29 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     w.bvh = pack.bvh(T, scene);
     if (accel != ATX_ACCEL_BVH) w.bvh.n_nodes = 0;
     const bool kahan = accumulator == ATX_ACCUM_KAHAN;
+    fill_wf_view(*settings, *cam, reinterpret_cast<float4*>(accum), kahan ? reinterpret_cast<float4*>(comp) : nullptr,
+                 image, kahan, first_frame, settings->accumulation ? frames : 1u, &w);
+    WfPass p{};
+    ATX_CHECK_ARG(layout_in_place(w, &p), "viewport too large");
+    p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
+    p.counters = reinterpret_cast<unsigned long long*>(base);
     // One launch for all frames; with accumulation off a launch per frame, the
-    // index back at 1 after the first (Renderer.cu:245-248).  The first launch's
-    // entry, its queue and the counters (both zero) go up with the scene, in one
-    // copy (two copies and two fill kernels less: 1280x720, 129 spheres, 4 frames
-    // 635 -> 629 us); the entries stay in place until their copies have run.
+    // index back at 1 after the first (Renderer.cu:245-248).  The queue and the
+    // counters (both zero) go up with the scene, in one copy.
     std::vector<unsigned char> block(kControlBytes, 0);
     const std::vector<unsigned char> packed = pack.block();
     block.insert(block.end(), packed.begin(), packed.end());
+    hipError_t e = hipMemcpyAsync(base, block.data(), block.size(), hipMemcpyHostToDevice, stream);
     const uint32_t launches = settings->accumulation ? 1u : frames;
-    constexpr uint32_t kEntries = 64;
-    WfScene entries[kEntries];
-    for (uint32_t l = 0; l < launches; ++l) {
-        if (l != 0 && l % kEntries == 0) ATX_HIP(hipStreamSynchronize(stream));
-        WfScene& e = entries[l % kEntries];
-        e = w;
-        const uint32_t n = settings->accumulation ? frames : 1u;
-        const uint32_t fi = l == 0 ? first_frame : 1u;
-        fill_wf_view(*settings, *cam, reinterpret_cast<float4*>(accum), kahan ? reinterpret_cast<float4*>(comp) : nullptr,
-                     image, kahan, fi, n, &e);
-        WfPass p{};
-        ATX_CHECK_ARG(layout_in_place(e, &p), "viewport too large");
-        p.scenes = reinterpret_cast<const WfScene*>(base + off_table);
-        p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
-        p.counters = reinterpret_cast<unsigned long long*>(base);
-        if (l == 0) {
-            memcpy(block.data() + off_table, &e, sizeof(e));
-            ATX_HIP(hipMemcpyAsync(base, block.data(), block.size(), hipMemcpyHostToDevice, stream));
-        } else {
-            ATX_HIP(hipMemcpyAsync(base + off_table, &e, sizeof(e), hipMemcpyHostToDevice, stream));
-            ATX_HIP(launch_zero_u32(p.queue, kQueueWords, stream));
+    for (uint32_t l = 0; l < launches && e == hipSuccess; ++l) {
+        if (l != 0) {
+            w.frame0 = 1u;
+            e = launch_zero_u32(p.queue, kQueueWords, stream);
         }
-        ATX_HIP(launch_in_place(p, e.bvh.n_tiles == 0, n, stream));
+        if (e == hipSuccess) e = launch_in_place(w, p, stream);
     }
-    // the host copies above read L and T, which end with this call
-    ATX_HIP(hipStreamSynchronize(stream));
+    // the copy reads `block`, which ends with this call
+    const hipError_t done = hipStreamSynchronize(stream);
+    ATX_HIP(e != hipSuccess ? e : done);
     return ATX_OK;
 }

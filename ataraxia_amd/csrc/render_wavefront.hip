@@ -78,6 +78,28 @@ __device__ __forceinline__ const ATX_CONST T* as_const(const T* p)
     return (const ATX_CONST T*)(uintptr_t)p;
 }
 
+// The path kernel's arguments.  An in-place launch has one scene, which comes
+// with them, so that a call of many launches needs no table.
+template <bool kInPlace>
+struct PathArgs {
+    WfPass p;
+    __device__ __forceinline__ CScene* scenes() const { return as_const(p.scenes); }
+};
+template <>
+struct PathArgs<true> {
+    WfPass p;
+    WfScene s;
+    __device__ __forceinline__ CScene* scenes() const
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return (CScene*)((const ATX_CONST char*)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(WfPass));
+#else
+        return nullptr;
+#endif
+    }
+};
+static_assert(sizeof(PathArgs<true>) == sizeof(WfPass) + sizeof(WfScene), "the scene follows the pass");
+
 struct SphSrc {
     CF4* p;
     __device__ __forceinline__ float4 operator()(uint32_t i) const { return p[i]; }
@@ -338,8 +360,10 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
 // frames 393 and 400, 4 frames 635 and 602, 8 frames 1175 and 965), always
 // without (8 spheres: 1 frame 199 and 179, 4 frames 393 and 339).
 template <uint32_t kWaves, bool kTree, bool kInPlace = false, bool kKeep = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(
+    PathArgs<kInPlace> args)
 {
+    const WfPass& a = args.p;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t P = a.chunk_px;
     // The instances for tiles, in place and for 7 and 8 resident waves per SIMD park the
@@ -360,7 +384,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     uint32_t(*own)[64] = own_all[threadIdx.x >> 6];
 
     // ---- wave-uniform scheduling state ----
-    CScene* scenes = as_const(a.scenes);
+    CScene* scenes = args.scenes();
     int32_t sid = -1;
     CScene* S = nullptr;
     int32_t pend = -1;              // a block of another scene, waiting for the lanes to drain
@@ -1052,7 +1076,7 @@ __global__ void k_zero_u32(unsigned int* p, uint32_t n)
 }
 
 // The path kernel's instance for a launch (wf_waves).
-using PathKernel = void (*)(WfPass);
+using PathKernel = void (*)(PathArgs<false>);
 PathKernel path_kernel(bool flat_only, uint32_t waves)
 {
     if (!flat_only)
@@ -1085,7 +1109,7 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
         // no workgroup without a first chunk for a wave
         const uint32_t most = (p.total_chunks + 3u) / 4u;
         hipLaunchKernelGGL(path_kernel(l.flat_only, l.waves), dim3(l.workgroups < most ? l.workgroups : most),
-                           dim3(256), 0, stream, p);
+                           dim3(256), 0, stream, PathArgs<false>{p});
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && paths_done)
@@ -1096,15 +1120,17 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_in_place(const WfPass& pass, bool flat_only, uint32_t frames, hipStream_t stream)
+hipError_t launch_in_place(const WfScene& s, const WfPass& pass, hipStream_t stream)
 {
-    WfPass p = pass;
+    PathArgs<true> args{pass, s};
+    WfPass& p = args.p;
     p.refill_min = kRefillMin;
     if (p.total_chunks == 0 || p.n_scenes != 1)
         return hipErrorInvalidValue;
-    const PathKernel kernel = flat_only ? k_render_wavefront<kWfWavesInPlace, false, true, true>
-                              : frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
-                                                      : k_render_wavefront<kWfWavesTree, true, true>;
+    void (*const kernel)(PathArgs<true>) =
+        s.bvh.n_tiles == 0u         ? k_render_wavefront<kWfWavesInPlace, false, true, true>
+        : s.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
+                                  : k_render_wavefront<kWfWavesTree, true, true>;
     int dev = 0, cus = 0, blocks = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1113,7 +1139,7 @@ hipError_t launch_in_place(const WfPass& pass, bool flat_only, uint32_t frames, 
         return e;
     const uint32_t full = (uint32_t)(cus > 0 ? cus : 1) * (uint32_t)(blocks > 0 ? blocks : 1);
     const uint32_t most = (p.total_chunks + 3u) / 4u;   // a first chunk for each wave
-    hipLaunchKernelGGL(kernel, dim3(full < most ? full : most), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(full < most ? full : most), dim3(256), 0, stream, args);
     return hipGetLastError();
 }
 

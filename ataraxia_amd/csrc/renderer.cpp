@@ -179,33 +179,29 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
         }
     }
 
-    // the plain kernel: an in-place launch per frame
-    std::vector<WfPass> passes;
+    // the plain kernel: an in-place launch per frame, its scene among the launch's
+    // arguments
+    const uint32_t n_launch = wf ? (uint32_t)table.size() : frames;
+    WfScene plain{};
+    WfPass plain_pass{};
     if (!wf) {
-        for (uint32_t f = 0, fi = r->frame_index; f < frames; ++f) {
-            WfScene e = entry(fi, 1);
-            e.exact = r->exact_loop ? 1u : 0u;
-            if (r->exact_loop) e.bvh.n_tiles = 0;
-            WfPass p{};
-            if (!layout_in_place(e, &p)) {
-                set_error("render: %u x %u pixels exceed one launch", e.width, e.height);
-                return ATX_ERR_INVALID;
-            }
-            table.push_back(e);
-            passes.push_back(p);
-            if (r->settings.accumulation) ++fi;
+        plain = entry(r->frame_index, 1);
+        plain.exact = r->exact_loop ? 1u : 0u;
+        if (r->exact_loop) plain.bvh.n_tiles = 0;
+        if (!layout_in_place(plain, &plain_pass)) {
+            set_error("render: %u x %u pixels exceed one launch", plain.width, plain.height);
+            return ATX_ERR_INVALID;
         }
     }
-    const uint32_t n_launch = (uint32_t)table.size();
     // The launches' table, their queues and the counters (both zero) are one
     // block, sent in one copy; as a copy, a fill kernel and a memset they
     // took 35 us of a 320x180 call's 124.  Past kRendererQueues launches (one
     // frame each) a queue is cleared and used again.
     const uint32_t n_queue = std::min(n_launch, kRendererQueues);
-    const size_t off_queue = (n_launch * sizeof(WfScene) + 255) & ~size_t(255);
+    const size_t off_queue = (table.size() * sizeof(WfScene) + 255) & ~size_t(255);
     const size_t off_ctr = off_queue + n_queue * kQueueWords * sizeof(unsigned int);
     r->launch_host.assign(off_ctr + kCounterBytes, 0);
-    if (n_launch) memcpy(r->launch_host.data(), table.data(), n_launch * sizeof(WfScene));
+    if (!table.empty()) memcpy(r->launch_host.data(), table.data(), table.size() * sizeof(WfScene));
     ATX_HIP(r->launch_dev.reserve(r->launch_host.size()));
     ATX_HIP(hipMemcpyAsync(r->launch_dev.get(), r->launch_host.data(), r->launch_host.size(), hipMemcpyHostToDevice,
                            r->stream));
@@ -241,13 +237,11 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
             }
         }
     } else {
-        const bool flat_only = n_launch == 0 || wf_flat_only(table.data(), 1);
         for (uint32_t f = 0; f < frames; ++f) {
-            WfPass wp = passes[f];
-            wp.scenes = d_table + f;
-            ATX_HIP(queue_of(f, &wp.queue));
-            wp.counters = d_ctr;
-            ATX_HIP(launch_in_place(wp, flat_only, 1, r->stream));
+            plain.frame0 = r->frame_index;
+            ATX_HIP(queue_of(f, &plain_pass.queue));
+            plain_pass.counters = d_ctr;
+            ATX_HIP(launch_in_place(plain, plain_pass, r->stream));
             // Renderer.cu:245-248
             if (r->settings.accumulation) r->frame_index++;
             else r->frame_index = 1;

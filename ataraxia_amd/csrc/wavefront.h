@@ -237,11 +237,11 @@ struct WfLaunch {
 // given, is recorded on the stream between the two.
 hipError_t launch_wavefront(const WfPass& p, const WfLaunch& l, hipStream_t stream,
                             hipEvent_t paths_done = nullptr);
-// In-place rendering of one scene (p.n_scenes 1, chunks of kInPlaceChunk jobs
-// laid out by layout_in_place): every pixel's frames one after another in one
-// lane, added to the accumulation as they end.  It needs neither samples nor
-// a first-bounce cache, so no memory beyond the scene's and the image's.
-hipError_t launch_in_place(const WfPass& p, bool flat_only, uint32_t frames, hipStream_t stream);
+// In-place rendering of the scene s (p laid out by layout_in_place): every
+// pixel's frames one after another in one lane, added to the accumulation as
+// they end.  It needs neither samples nor a first-bounce cache, so no memory
+// beyond the scene's and the image's.
+hipError_t launch_in_place(const WfScene& s, const WfPass& p, hipStream_t stream);
 hipError_t launch_zero_u32(unsigned int* p, uint32_t n, hipStream_t stream);
 // Writes the primary ray direction of every pixel of s's camera to dirs
 // (width * height float4, w = 0): camera_ray, computed once instead of per path.
