@@ -347,18 +347,17 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
     }
 }
 
-// kInPlace: a job is a pixel, and its lane renders the launch's frames one
-// after another into the accumulation; no samples, no first-bounce cache.  A
-// kernel with one lane per pixel and frame, 64 pixels to a wave until its
-// longest path ended, took 0.62 ms per frame at 1280x720 with 129 spheres;
-// here lanes go on with their next frame or another pixel: a call of 4 frames
-// 2.68 -> 0.81 ms, 0.63 with the steps since.  The tile instance is bound like
-// the sampling one, by VALU issue.
+// kInPlace (scenes with tiles; k_render_flat does the others): a job is a
+// pixel, and its lane renders the launch's frames one after another into the
+// accumulation; no samples, no first-bounce cache.  A kernel with one lane per
+// pixel and frame, 64 pixels to a wave until its longest path ended, took 0.62 ms
+// per frame at 1280x720 with 129 spheres; here lanes go on with their next frame
+// or another pixel: a call of 4 frames 2.68 -> 0.81 ms, 0.63 with the steps since.
+// It is bound like the sampling one, by VALU issue.
 // kKeep: a pixel's primary hit is the same in every frame, so its lane keeps it
-// and the frames after the first start at its shadow ray.  From three frames on
-// with tiles (1280x720, 129 spheres: 1 frame 266 us without and 281 with it, 2
-// frames 393 and 400, 4 frames 635 and 602, 8 frames 1175 and 965), always
-// without (8 spheres: 1 frame 199 and 179, 4 frames 393 and 339).
+// and the frames after the first start at its shadow ray, from three frames on
+// (1280x720, 129 spheres: 1 frame 266 us without and 281 with it, 2 frames 393 and
+// 400, 4 frames 635 and 602, 8 frames 1175 and 965).
 template <uint32_t kWaves, bool kTree, bool kInPlace = false, bool kKeep = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(
     PathArgs<kInPlace> args)
@@ -366,13 +365,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     const WfPass& a = args.p;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t P = a.chunk_px;
-    // The instances for tiles, in place and for 7 and 8 resident waves per SIMD park the
+    // The instances for tiles and for 7 and 8 resident waves per SIMD park the
     // path state that a trace does not read (17 values per lane) in LDS while
     // the trace runs: the state then needs no VGPRs there, and the trace fits
     // its register budget without spilling (17 KB of LDS per 256-lane
     // workgroup, 136 KB per CU at 8 waves per SIMD; a tile query's candidate
     // masks take another 14 KB).
-    constexpr bool kPark = kWaves >= 7 || kTree || kInPlace;
+    constexpr bool kPark = kWaves >= 7 || kTree;
     constexpr uint32_t kParked = 17;
     __shared__ uint32_t parked_all[4][kPark ? kParked : 1][64];
     uint32_t(*parked)[64] = parked_all[threadIdx.x >> 6];
@@ -687,10 +686,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                                         capture || (kKeep && bounce == 0),
                                         tile_masks[threadIdx.x >> 6], q);
             } else {
-                if (kInPlace && S->exact)
-                    h = trace_exact(flat, S->n_sph, ro, rd);
-                else
-                    h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
+                h = trace_filtered(flat, S->n_sph, ro, rd, q.exact);
                 q.tests = S->n_sph;
                 if (h.id >= 0 && !shadow) {
                     q.sphere = flat((uint32_t)h.id);
@@ -810,6 +806,112 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     }
 
     flush_counters(counters(), lane, tests, boxes, rays, reused);
+}
+
+// In-place launches of scenes without tiles: a lane per pixel, a wave per 8 x 8
+// pixels, both rays of a bounce in one round, so that a path's chain of dependent
+// instructions, which bounds it (the loads and square roots of one ray after the
+// other), stays short.  The persistent kernel's in-place mode, whose round is one ray
+// and which hands out pixels, took longer at every size (one frame, 13 spheres:
+// 64x64 51 us, here 32; 640x360 71 and 50; 1920x1080 214 and 96).
+// kFrames: a lane goes on to its next frame without waiting for the others and
+// keeps its primary hit (1280x720, 13 spheres, 32 frames: 1.54 ms with a loop over
+// frames around one over bounces, 1.33 with this one, 1.90 persistent).  A launch of
+// one frame has an instance of its own, 8 % shorter.
+template <bool kFrames>
+__global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
+{
+    CScene* const S = args.scenes();
+    const uint32_t lane = threadIdx.x;
+    const uint32_t px = in_place_pixel(S, blockIdx.x * 64u + lane);
+    const SphSrc flat{as_const(S->sph)};
+    uint32_t rays = 0, exact = 0;   // this lane's
+    if (px != ~0u) {
+        const f3 eye = mk(S->cam_pos[0], S->cam_pos[1], S->cam_pos[2]), dir = primary_direction(S, px);
+        const bool debug = S->dbg_hit || S->dbg_shadow;
+        const auto trace = [&](f3 o, f3 d) {
+            ++rays;
+            return S->exact ? trace_exact(flat, S->n_sph, o, d) : trace_filtered(flat, S->n_sph, o, d, exact);
+        };
+        uint32_t f = 0, seed = 0;
+        int32_t bounce = 0;
+        f3 ro, rd, tp, col;
+        bool capture = false;
+        const auto start = [&]() {   // the path of frame f
+            ro = eye;
+            rd = dir;
+            tp = mk(1.0f, 1.0f, 1.0f);
+            col = mk(0.0f, 0.0f, 0.0f);
+            seed = px * (S->frame0 + f);
+            bounce = 0;
+            capture = debug && f + 1u == S->frames;
+            for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
+                if (S->dbg_hit) S->dbg_hit[(size_t)px * S->dbg_bounces + i] = -2;
+                if (S->dbg_shadow) S->dbg_shadow[(size_t)px * S->dbg_bounces + i] = -2;
+            }
+        };
+        // one bounce; true when the path ends
+        Hit first;   // the primary ray's
+        first.id = -1;
+        first.t = FLT_MAX;
+        const auto step = [&]() -> bool {
+            if (S->max_bounces <= 0)
+                return true;
+            Hit h = first;
+            if (!kFrames || bounce != 0 || f == 0u)
+                h = trace(ro, rd);
+            if (kFrames && bounce == 0)
+                first = h;
+            const size_t at = (size_t)px * S->dbg_bounces + (uint32_t)bounce;
+            const bool record = capture && (uint32_t)bounce < S->dbg_bounces;
+            if (record && S->dbg_hit)
+                S->dbg_hit[at] = h.id;
+            if (h.id < 0) {
+                if (S->sky_light)
+                    col = add(col, mul(mk(0.6f, 0.7f, 0.9f), tp));
+                return true;
+            }
+            const int32_t mid = S->sph_mat[h.id];
+            const float4 m0 = S->mat[3 * mid], m1 = S->mat[3 * mid + 1];
+            f3 nrm, so, L, surface;
+            uint32_t lidx = 0;
+            float dist2 = 0.0f;
+            if (shade_hit(S, flat((uint32_t)h.id), mid, h, ro, rd, tp, seed, col, nrm, so, lidx, L, dist2)) {
+                const Hit sh = trace(so, L);
+                if (record && S->dbg_shadow)
+                    S->dbg_shadow[at] = sh.id;
+                if (lit_by(sh, dist2))
+                    col = add(col, light_term(m0, m1, S->light[2 * lidx + 1], nrm, rd, L, tp, S->mild != 0u));
+            }
+            if (roulette(S, m0, m1.w, tp, bounce, seed, surface))
+                return true;
+            ro = so;
+            next_direction(surface, nrm, rd, bounce, seed);
+            return false;
+        };
+        start();
+        if constexpr (!kFrames) {
+            while (!step()) {
+            }
+            add_sample(S, px, 0u, 1u, col);
+        } else {
+            while (f < S->frames) {
+                if (step()) {
+                    // a primary ray that misses does so in every frame
+                    const bool miss = bounce == 0 && first.id < 0 && !debug;
+                    const uint32_t n = miss ? S->frames - f : 1u;
+                    add_sample(S, px, f, n, col);
+                    f += n;
+                    if (f < S->frames)
+                        start();
+                }
+            }
+        }
+    }
+    const unsigned long long r = wave_sum(rays), e = wave_sum(exact);
+    const unsigned long long v = lane == kCtrRays ? r : lane == kCtrTests ? r * S->n_sph : lane == kCtrExact ? e : 0ull;
+    if (v)
+        atomicAdd(args.p.counters + (blockIdx.x % kCounterLines) * kCounterStride + lane, v);
 }
 
 // Adds every pixel's samples of the launch to its accumulation in frame order
@@ -1127,10 +1229,13 @@ hipError_t launch_in_place(const WfScene& s, const WfPass& pass, hipStream_t str
     p.refill_min = kRefillMin;
     if (p.total_chunks == 0 || p.n_scenes != 1)
         return hipErrorInvalidValue;
-    void (*const kernel)(PathArgs<true>) =
-        s.bvh.n_tiles == 0u         ? k_render_wavefront<kWfWavesInPlace, false, true, true>
-        : s.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
-                                  : k_render_wavefront<kWfWavesTree, true, true>;
+    if (s.bvh.n_tiles == 0u) {
+        hipLaunchKernelGGL(s.frames > 1u ? k_render_flat<true> : k_render_flat<false>, dim3(p.total_chunks), dim3(64), 0,
+                           stream, args);
+        return hipGetLastError();
+    }
+    void (*const kernel)(PathArgs<true>) = s.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
+                                                                   : k_render_wavefront<kWfWavesTree, true, true>;
     int dev = 0, cus = 0, blocks = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);

@@ -184,7 +184,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     const uint32_t n_launch = wf ? (uint32_t)table.size() : frames;
     WfScene plain{};
     WfPass plain_pass{};
-    if (!wf) {
+    if (!wf && frames > 0) {
         plain = entry(r->frame_index, 1);
         plain.exact = r->exact_loop ? 1u : 0u;
         if (r->exact_loop) plain.bvh.n_tiles = 0;

@@ -215,7 +215,6 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
 // 4).
 constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
-constexpr uint32_t kWfWavesInPlace = 6;   // flat scenes in place (79 VGPRs)
 constexpr uint32_t kKeepFrames = 3;       // in place with tiles: primary hits are kept from here on
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
 // The instance a launch uses: `waves` when it names a compiled instance,
