@@ -1,8 +1,8 @@
 // render_noalloc.hip -- the allocation-free render entry point.
 //
 // atx_render_frames_noalloc renders frames of one scene in place
-// (launch_in_place: every pixel's frames one after another in one lane, one
-// launch for all frames of the call), with the results of
+// (launch_in_place: every pixel's frames one after another in one lane, up to
+// kInPlaceFrames frames of the call in a launch), with the results of
 // atx_renderer_render_frames, but allocates no device memory: the caller
 // passes the accumulation, compensation and image buffers, and everything else
 // the kernel reads besides its arguments (the scene in its device layout, its
@@ -17,6 +17,7 @@
 // on a device shares its array: calls that overlap on one device (two host
 // threads, or two streams) race on it.  A call returns after its frames are
 // rendered, so consecutive calls on one thread do not overlap.
+#include <algorithm>
 #include <mutex>
 #include <string.h>
 #include <vector>
@@ -125,25 +126,24 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     if (accel != ATX_ACCEL_BVH) w.bvh.n_nodes = 0;
     const bool kahan = accumulator == ATX_ACCUM_KAHAN;
     fill_wf_view(*settings, *cam, reinterpret_cast<float4*>(accum), kahan ? reinterpret_cast<float4*>(comp) : nullptr,
-                 image, kahan, first_frame, settings->accumulation ? frames : 1u, &w);
+                 image, kahan, first_frame, settings->accumulation ? std::min(frames, kInPlaceFrames) : 1u, &w);
     WfPass p{};
     ATX_CHECK_ARG(layout_in_place(w, &p), "viewport too large");
     p.queue = reinterpret_cast<unsigned int*>(base + off_queue);
     p.counters = reinterpret_cast<unsigned long long*>(base);
-    // One launch for all frames; with accumulation off a launch per frame, the
-    // index back at 1 after the first (Renderer.cu:245-248).  The queue and the
-    // counters (both zero) go up with the scene, in one copy.
+    // One launch for up to kInPlaceFrames frames; with accumulation off a launch
+    // per frame, the index back at 1 after the first (Renderer.cu:245-248).  The
+    // queue and the counters (both zero) go up with the scene, in one copy.
     std::vector<unsigned char> block(kControlBytes, 0);
     const std::vector<unsigned char> packed = pack.block();
     block.insert(block.end(), packed.begin(), packed.end());
     hipError_t e = hipMemcpyAsync(base, block.data(), block.size(), hipMemcpyHostToDevice, stream);
-    const uint32_t launches = settings->accumulation ? 1u : frames;
-    for (uint32_t l = 0; l < launches && e == hipSuccess; ++l) {
-        if (l != 0) {
-            w.frame0 = 1u;
-            e = launch_zero_u32(p.queue, kQueueWords, stream);
-        }
-        if (e == hipSuccess) e = launch_in_place(w, p, stream);
+    for (uint32_t left = frames; left > 0 && e == hipSuccess;) {
+        e = launch_in_place(w, p, stream);
+        left -= w.frames;
+        w.frame0 = settings->accumulation ? w.frame0 + w.frames : 1u;
+        w.frames = std::min(left, w.frames);
+        if (e == hipSuccess && left > 0) e = launch_zero_u32(p.queue, kQueueWords, stream);
     }
     // the copy reads `block`, which ends with this call
     const hipError_t done = hipStreamSynchronize(stream);

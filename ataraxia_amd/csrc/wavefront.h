@@ -113,7 +113,7 @@ struct WfScene {
     const uint32_t* hit_px;
     uint32_t n_hit;
     BvhDev bvh;            // n_tiles = 0: flat loop over all spheres
-    UDiv div_group;        // by kJobGroupPx * frames (set by layout_launch)
+    UDiv div_group;        // by kJobGroupPx * frames (set by layout_launch; not used in place)
     UDiv div_light;        // by max(n_light, 1) (set by layout_launch)
 };
 
@@ -216,6 +216,9 @@ __host__ __device__ __forceinline__ uint32_t job_of(uint32_t k, uint32_t f, uint
 constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
 constexpr uint32_t kKeepFrames = 3;       // in place with tiles: primary hits are kept from here on
+// Frames of one in-place launch: the allocation-free call takes any number, and a
+// kernel should not run for minutes (1920x1080, 129 spheres: 0.5 s for as many).
+constexpr uint32_t kInPlaceFrames = 4096;
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
 // The instance a launch uses: `waves` when it names a compiled instance,
 // else the default for its scenes.

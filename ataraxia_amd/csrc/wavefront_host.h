@@ -151,8 +151,9 @@ inline bool layout_launch(WfScene* tab, size_t n, uint32_t chunk_px, float3* sam
     return true;
 }
 
-// The same for an in-place launch of one scene.  False when its jobs do not
-// fit 32 bits.
+// The same for an in-place launch of one scene, of any number of frames (its
+// jobs are pixels, not divided by div_group).  False when its jobs do not fit
+// 32 bits.
 inline bool layout_in_place(WfScene& w, WfPass* p)
 {
     const uint64_t jobs = (((uint64_t)w.width + 7) / 8) * (((uint64_t)w.height + 7) / 8) * 64;
@@ -160,7 +161,6 @@ inline bool layout_in_place(WfScene& w, WfPass* p)
         return false;
     w.chunk_begin = w.px_begin = 0;
     w.n_chunks = (uint32_t)(jobs / kInPlaceChunk);
-    w.div_group = udiv_make(kJobGroupPx * w.frames);
     w.div_light = udiv_make(w.n_light ? w.n_light : 1u);
     p->n_scenes = 1;
     p->total_chunks = w.n_chunks;
