@@ -266,16 +266,6 @@ __device__ __forceinline__ uint32_t job_pixel(CScene* S, uint32_t slots, uint32_
     return S->hit_px ? S->hit_px[slot] : slot;
 }
 
-// In-place launches: the pixel of job j, whose 64 consecutive jobs are an 8 x 8
-// tile (past the image's edge: ~0).
-__device__ __forceinline__ uint32_t in_place_pixel(CScene* S, uint32_t j)
-{
-    const uint32_t W = S->width, tiles_x = (W + 7u) / 8u;
-    const uint32_t t = j >> 6, ty = t / tiles_x, tx = t - ty * tiles_x;
-    const uint32_t x = tx * 8u + (j & 7u), y = ty * 8u + ((j >> 3) & 7u);
-    return x < W && y < S->height ? y * W + x : ~0u;
-}
-
 __device__ __forceinline__ f3 primary_direction(CScene* S, uint32_t px)
 {
     const uint32_t W = S->width;
@@ -479,7 +469,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 uint32_t cached_rays = 0;   // this lane's rays taken from the first-bounce cache
                 if constexpr (kInPlace) {
                     if (state == kIdle && rank < avail) {
-                        const uint32_t px = in_place_pixel(S, blk0 + blk_next + rank);
+                        const uint32_t px = in_place_pixel(blk0 + blk_next + rank, S->width, S->height);
                         if (px != ~0u) {
                             job = px;
                             const f3 dir = primary_direction(S, px);
@@ -631,7 +621,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 slots = (uint32_t)__builtin_amdgcn_readfirstlane((int)job_slots(S->hit_px, S->width * S->height));
             }
             pend = -1;
-            const uint32_t jobs = kInPlace ? in_place_jobs(S->width, S->height) : slots * S->frames;
+            const uint32_t jobs = kInPlace ? (uint32_t)in_place_jobs(S->width, S->height) : slots * S->frames;
             blk0 = ((uint32_t)c - S->chunk_begin) * P;
             blk_end = blk0 >= jobs ? 0u : (jobs - blk0 < P ? jobs - blk0 : P);
             blk_next = 0;
@@ -823,7 +813,7 @@ __global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
 {
     CScene* const S = args.scenes();
     const uint32_t lane = threadIdx.x;
-    const uint32_t px = in_place_pixel(S, blockIdx.x * 64u + lane);
+    const uint32_t px = in_place_pixel(blockIdx.x * 64u + lane, S->width, S->height);
     const SphSrc flat{as_const(S->sph)};
     uint32_t rays = 0, exact = 0;   // this lane's
     if (px != ~0u) {

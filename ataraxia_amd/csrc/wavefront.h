@@ -190,11 +190,32 @@ __host__ __device__ __forceinline__ void job_pixel_frame(uint32_t j, uint32_t pi
     px = kJobGroupPx * g + (w - frame * m);
 }
 
-// Jobs of an in-place launch: the pixels of whole 8 x 8 tiles.
+// Jobs of an in-place launch: 64 to an 8 x 8 tile of pixels; along the rows
+// instead for images narrower or lower than a tile, and for those whose tiles reach
+// past the right edge so far that their jobs would not fit 32 bits.
 constexpr uint32_t kInPlaceChunk = 64;
-__host__ __device__ __forceinline__ uint32_t in_place_jobs(uint32_t width, uint32_t height)
+__host__ __device__ __forceinline__ uint64_t in_place_tiles(uint32_t width, uint32_t height)
 {
-    return ((width + 7u) / 8u) * ((height + 7u) / 8u) * 64u;
+    return (((uint64_t)width + 7u) / 8u) * (((uint64_t)height + 7u) / 8u);
+}
+__host__ __device__ __forceinline__ bool in_place_rows(uint32_t width, uint32_t height)
+{
+    return width < 8u || height < 8u || in_place_tiles(width, height) >= (1u << 26) - 1u;
+}
+__host__ __device__ __forceinline__ uint64_t in_place_jobs(uint32_t width, uint32_t height)
+{
+    return in_place_rows(width, height) ? ((uint64_t)width * height + 63u) / 64u * 64u
+                                        : in_place_tiles(width, height) * 64u;
+}
+// The pixel of job j (past the image's edge: ~0).
+__host__ __device__ __forceinline__ uint32_t in_place_pixel(uint32_t j, uint32_t width, uint32_t height)
+{
+    if (in_place_rows(width, height))
+        return j < width * height ? j : ~0u;
+    const uint32_t tiles_x = (width + 7u) / 8u;
+    const uint32_t t = j >> 6, ty = t / tiles_x, tx = t - ty * tiles_x;
+    const uint32_t x = tx * 8u + (j & 7u), y = ty * 8u + ((j >> 3) & 7u);
+    return x < width && y < height ? y * width + x : ~0u;
 }
 
 // The job of slot k in the launch's frame f (the inverse of job_pixel_frame).
@@ -217,7 +238,7 @@ constexpr uint32_t kWfWavesTree = 5;
 constexpr uint32_t kWfWavesFlat = 7;
 constexpr uint32_t kKeepFrames = 3;       // in place with tiles: primary hits are kept from here on
 // Frames of one in-place launch: the allocation-free call takes any number, and a
-// kernel should not run for minutes (1920x1080, 129 spheres: 0.5 s for as many).
+// kernel should not run for minutes (1920x1080, 129 spheres: 1024 take 0.19 s).
 constexpr uint32_t kInPlaceFrames = 4096;
 constexpr uint32_t kWfWavesMin = 5, kWfWavesMax = 8;
 // The instance a launch uses: `waves` when it names a compiled instance,

@@ -156,7 +156,7 @@ inline bool layout_launch(WfScene* tab, size_t n, uint32_t chunk_px, float3* sam
 // 32 bits.
 inline bool layout_in_place(WfScene& w, WfPass* p)
 {
-    const uint64_t jobs = (((uint64_t)w.width + 7) / 8) * (((uint64_t)w.height + 7) / 8) * 64;
+    const uint64_t jobs = in_place_jobs(w.width, w.height);
     if (jobs + kInPlaceChunk >= 1ull << 32)
         return false;
     w.chunk_begin = w.px_begin = 0;
