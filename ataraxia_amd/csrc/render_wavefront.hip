@@ -78,28 +78,6 @@ __device__ __forceinline__ const ATX_CONST T* as_const(const T* p)
     return (const ATX_CONST T*)(uintptr_t)p;
 }
 
-// The path kernel's arguments.  An in-place launch has one scene, which comes
-// with them, so that a call of many launches needs no table.
-template <bool kInPlace>
-struct PathArgs {
-    WfPass p;
-    __device__ __forceinline__ CScene* scenes() const { return as_const(p.scenes); }
-};
-template <>
-struct PathArgs<true> {
-    WfPass p;
-    WfScene s;
-    __device__ __forceinline__ CScene* scenes() const
-    {
-#if defined(__HIP_DEVICE_COMPILE__)
-        return (CScene*)((const ATX_CONST char*)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(WfPass));
-#else
-        return nullptr;
-#endif
-    }
-};
-static_assert(sizeof(PathArgs<true>) == sizeof(WfPass) + sizeof(WfScene), "the scene follows the pass");
-
 struct SphSrc {
     CF4* p;
     __device__ __forceinline__ float4 operator()(uint32_t i) const { return p[i]; }
@@ -301,9 +279,9 @@ __device__ __forceinline__ uint32_t display(float4 acc, uint32_t frame)
 
 // In-place launches: the sample of pixel px, the same in n frames of the
 // launch from f on, goes to the accumulation; the last frame's also to the image.
-__device__ __forceinline__ void add_sample(CScene* S, uint32_t px, uint32_t f, uint32_t n, f3 col)
+__device__ __forceinline__ void add_sample(CScene* S, const WfPass& a, uint32_t px, uint32_t f, uint32_t n, f3 col)
 {
-    const uint32_t frame = S->frame0 + f;
+    const uint32_t frame = a.frame0 + f;
     const bool kahan = S->kahan != 0u;
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float4 acc = frame == 1u ? zero : S->accum[px];
@@ -317,7 +295,7 @@ __device__ __forceinline__ void add_sample(CScene* S, uint32_t px, uint32_t f, u
     S->accum[px] = acc;
     if (kahan)
         S->comp[px] = c;
-    if (f + n == S->frames) {
+    if (f + n == a.frames) {
         S->image[px] = display(acc, frame + n - 1u);
         if (S->dbg_radiance)
             S->dbg_radiance[px] = make_float4(col.x, col.y, col.z, 1.0f);
@@ -349,10 +327,8 @@ __device__ __forceinline__ void store_sample(CScene* S, uint32_t slots, uint32_t
 // (1280x720, 129 spheres: 1 frame 266 us without and 281 with it, 2 frames 393 and
 // 400, 4 frames 635 and 602, 8 frames 1175 and 965).
 template <uint32_t kWaves, bool kTree, bool kInPlace = false, bool kKeep = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(
-    PathArgs<kInPlace> args)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void k_render_wavefront(WfPass a)
 {
-    const WfPass& a = args.p;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t P = a.chunk_px;
     // The instances for tiles and for 7 and 8 resident waves per SIMD park the
@@ -373,7 +349,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     uint32_t(*own)[64] = own_all[threadIdx.x >> 6];
 
     // ---- wave-uniform scheduling state ----
-    CScene* scenes = args.scenes();
+    CScene* scenes = as_const(a.scenes);
     int32_t sid = -1;
     CScene* S = nullptr;
     int32_t pend = -1;              // a block of another scene, waiting for the lanes to drain
@@ -416,10 +392,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         rd = dir;
         tp = mk(1.0f, 1.0f, 1.0f);
         col = mk(0.0f, 0.0f, 0.0f);
-        seed = job * (S->frame0 + f);
+        seed = job * (a.frame0 + f);
         bounce = 0;
         state = kCont;
-        capture = (S->dbg_hit || S->dbg_shadow) && f + 1u == S->frames;
+        capture = (S->dbg_hit || S->dbg_shadow) && f + 1u == a.frames;
         for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
             if (S->dbg_hit) S->dbg_hit[(size_t)job * S->dbg_bounces + i] = -2;
             if (S->dbg_shadow) S->dbg_shadow[(size_t)job * S->dbg_bounces + i] = -2;
@@ -779,9 +755,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 // bounce ends where it is shaded
                 const bool known = kKeep && S->n_light != 0 && S->max_bounces > 0 && !S->dbg_hit && !S->dbg_shadow;
                 const bool miss = known && (int32_t)own[4][lane] < 0;
-                const uint32_t n = miss ? S->frames - f : 1u;
-                add_sample(S, job, f, n, col);
-                if (f + n < S->frames) {
+                const uint32_t n = miss ? a.frames - f : 1u;
+                add_sample(S, a, job, f, n, col);
+                if (f + n < a.frames) {
                     own[3][lane] = f + n;
                     if (known)
                         state = kAgain;
@@ -809,9 +785,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
 // frames around one over bounces, 1.33 with this one, 1.90 persistent).  A launch of
 // one frame has an instance of its own, 8 % shorter.
 template <bool kFrames>
-__global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
+__global__ __launch_bounds__(64) void k_render_flat(WfPass a)
 {
-    CScene* const S = args.scenes();
+    CScene* const S = as_const(a.scenes);
     const uint32_t lane = threadIdx.x;
     const uint32_t px = in_place_pixel(blockIdx.x * 64u + lane, S->width, S->height);
     const SphSrc flat{as_const(S->sph)};
@@ -832,9 +808,9 @@ __global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
             rd = dir;
             tp = mk(1.0f, 1.0f, 1.0f);
             col = mk(0.0f, 0.0f, 0.0f);
-            seed = px * (S->frame0 + f);
+            seed = px * (a.frame0 + f);
             bounce = 0;
-            capture = debug && f + 1u == S->frames;
+            capture = debug && f + 1u == a.frames;
             for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
                 if (S->dbg_hit) S->dbg_hit[(size_t)px * S->dbg_bounces + i] = -2;
                 if (S->dbg_shadow) S->dbg_shadow[(size_t)px * S->dbg_bounces + i] = -2;
@@ -883,16 +859,16 @@ __global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
         if constexpr (!kFrames) {
             while (!step()) {
             }
-            add_sample(S, px, 0u, 1u, col);
+            add_sample(S, a, px, 0u, 1u, col);
         } else {
-            while (f < S->frames) {
+            while (f < a.frames) {
                 if (step()) {
                     // a primary ray that misses does so in every frame
                     const bool miss = bounce == 0 && first.id < 0 && !debug;
-                    const uint32_t n = miss ? S->frames - f : 1u;
-                    add_sample(S, px, f, n, col);
+                    const uint32_t n = miss ? a.frames - f : 1u;
+                    add_sample(S, a, px, f, n, col);
                     f += n;
-                    if (f < S->frames)
+                    if (f < a.frames)
                         start();
                 }
             }
@@ -901,7 +877,7 @@ __global__ __launch_bounds__(64) void k_render_flat(PathArgs<true> args)
     const unsigned long long r = wave_sum(rays), e = wave_sum(exact);
     const unsigned long long v = lane == kCtrRays ? r : lane == kCtrTests ? r * S->n_sph : lane == kCtrExact ? e : 0ull;
     if (v)
-        atomicAdd(args.p.counters + (blockIdx.x % kCounterLines) * kCounterStride + lane, v);
+        atomicAdd(a.counters + (blockIdx.x % kCounterLines) * kCounterStride + lane, v);
 }
 
 // Adds every pixel's samples of the launch to its accumulation in frame order
@@ -1168,7 +1144,7 @@ __global__ void k_zero_u32(unsigned int* p, uint32_t n)
 }
 
 // The path kernel's instance for a launch (wf_waves).
-using PathKernel = void (*)(PathArgs<false>);
+using PathKernel = void (*)(WfPass);
 PathKernel path_kernel(bool flat_only, uint32_t waves)
 {
     if (!flat_only)
@@ -1201,7 +1177,7 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
         // no workgroup without a first chunk for a wave
         const uint32_t most = (p.total_chunks + 3u) / 4u;
         hipLaunchKernelGGL(path_kernel(l.flat_only, l.waves), dim3(l.workgroups < most ? l.workgroups : most),
-                           dim3(256), 0, stream, PathArgs<false>{p});
+                           dim3(256), 0, stream, p);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && paths_done)
@@ -1214,18 +1190,17 @@ hipError_t launch_wavefront(const WfPass& pass, const WfLaunch& l, hipStream_t s
 
 hipError_t launch_in_place(const WfScene& s, const WfPass& pass, hipStream_t stream)
 {
-    PathArgs<true> args{pass, s};
-    WfPass& p = args.p;
+    WfPass p = pass;
     p.refill_min = kRefillMin;
-    if (p.total_chunks == 0 || p.n_scenes != 1)
+    if (p.total_chunks == 0 || p.n_scenes != 1 || p.frames == 0)
         return hipErrorInvalidValue;
     if (s.bvh.n_tiles == 0u) {
-        hipLaunchKernelGGL(s.frames > 1u ? k_render_flat<true> : k_render_flat<false>, dim3(p.total_chunks), dim3(64), 0,
-                           stream, args);
+        hipLaunchKernelGGL(p.frames > 1u ? k_render_flat<true> : k_render_flat<false>, dim3(p.total_chunks), dim3(64), 0,
+                           stream, p);
         return hipGetLastError();
     }
-    void (*const kernel)(PathArgs<true>) = s.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
-                                                                   : k_render_wavefront<kWfWavesTree, true, true>;
+    const PathKernel kernel = p.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>
+                                                      : k_render_wavefront<kWfWavesTree, true, true>;
     int dev = 0, cus = 0, blocks = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1234,7 +1209,7 @@ hipError_t launch_in_place(const WfScene& s, const WfPass& pass, hipStream_t str
         return e;
     const uint32_t full = (uint32_t)(cus > 0 ? cus : 1) * (uint32_t)(blocks > 0 ? blocks : 1);
     const uint32_t most = (p.total_chunks + 3u) / 4u;   // a first chunk for each wave
-    hipLaunchKernelGGL(kernel, dim3(full < most ? full : most), dim3(256), 0, stream, args);
+    hipLaunchKernelGGL(kernel, dim3(full < most ? full : most), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

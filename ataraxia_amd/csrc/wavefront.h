@@ -130,6 +130,9 @@ struct WfPass {
     unsigned long long* totals;
     const uint32_t* n_hits;
     uint32_t refill_min;   // idle lanes a wave waits for before it hands out jobs (set by launch_wavefront)
+    // in place: this launch's frames (the table entry's are not read, so that the
+    // launches of a call share one entry)
+    uint32_t frame0, frames;
     uint32_t pad_;
 };
 
@@ -260,10 +263,10 @@ struct WfLaunch {
 // given, is recorded on the stream between the two.
 hipError_t launch_wavefront(const WfPass& p, const WfLaunch& l, hipStream_t stream,
                             hipEvent_t paths_done = nullptr);
-// In-place rendering of the scene s (p laid out by layout_in_place): every
-// pixel's frames one after another in one lane, added to the accumulation as
-// they end.  It needs neither samples nor a first-bounce cache, so no memory
-// beyond the scene's and the image's.
+// In-place rendering of the scene s, which p.scenes points to on the device (p
+// laid out by layout_in_place): every pixel's frames one after another in one
+// lane, added to the accumulation as they end.  It needs neither samples nor a
+// first-bounce cache, so no memory beyond the scene's and the image's.
 hipError_t launch_in_place(const WfScene& s, const WfPass& p, hipStream_t stream);
 hipError_t launch_zero_u32(unsigned int* p, uint32_t n, hipStream_t stream);
 // Writes the primary ray direction of every pixel of s's camera to dirs

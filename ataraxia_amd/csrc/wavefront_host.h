@@ -166,6 +166,8 @@ inline bool layout_in_place(WfScene& w, WfPass* p)
     p->total_chunks = w.n_chunks;
     p->total_px = w.width * w.height;
     p->chunk_px = kInPlaceChunk;
+    p->frame0 = w.frame0;
+    p->frames = w.frames;
     return true;
 }
 
