@@ -155,6 +155,8 @@ int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* mate
     HostBvh T;
     build_bvh(L.sph.data(), (uint32_t)n, 0, &T);
     const ScenePack pack(L, T);
+    // the block's growth frees the former scene: until this one is there, there is none
+    out->forget();
     // never an empty block: the kernels' pointers stay valid without spheres
     ATX_HIP(out->block.reserve(pack.bytes + 16));
     if (pack.bytes) ATX_HIP(hipMemcpy(out->block.get(), pack.block().data(), pack.bytes, hipMemcpyHostToDevice));

@@ -212,6 +212,15 @@ struct DevScene {
     float least_albedo = 1.0f;      // of HostSceneLayout
     bool unit_materials = false, emits = false;
     BvhDev bvh{};
+    bool loaded() const { return sph != nullptr; }
+    // Drops the scene (not its block).
+    void forget()
+    {
+        sph = mat = mat_rr = light = nullptr;
+        sph_mat = nullptr;
+        n_sph = n_mat = n_light = 0;
+        bvh = BvhDev{};
+    }
     void use_pool(DevPool* pool) { block.use_pool(pool); }
     size_t bytes() const { return block.bytes(); }
     // The tiles to hand to a kernel; for ATX_ACCEL_NONE without their boxes, so
@@ -224,7 +233,8 @@ struct DevScene {
     }
 };
 
-// Validates, converts and uploads (synchronously) a flattened scene.
+// Validates, converts and uploads (synchronously) a flattened scene.  After a
+// failure `out` holds the former scene if the arguments were refused, else none.
 int upload_scene(const atx_sphere* spheres, uint64_t n, const atx_material* materials, uint64_t m,
                  const atx_light* lights, uint64_t l, DevScene* out);
 

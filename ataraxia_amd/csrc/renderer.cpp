@@ -32,7 +32,6 @@ struct Renderer {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<hipEvent_t> wf_ev;   // per wavefront launch: path kernel start, end
     DevScene geo;
-    bool has_scene = false;
     int kernel = ATX_KERNEL_WAVEFRONT;
     int accel = ATX_ACCEL_BVH;
     DevBuf launch_dev, wf_samples, wf_dirs, wf_first;
@@ -77,7 +76,7 @@ static int renderer_launch_frames(Renderer* r, const atx_camera* cam, uint32_t f
     ATX_CHECK_ARG(cam->width == r->width && cam->height == r->height,
                   "camera viewport %ux%u does not match renderer %ux%u", cam->width, cam->height, r->width,
                   r->height);
-    if (!r->has_scene) {
+    if (!r->geo.loaded()) {
         set_error("no scene: call atx_renderer_set_scene first");
         return ATX_ERR_STATE;
     }
@@ -377,10 +376,7 @@ int atx_renderer_set_scene(atx_renderer* h, const atx_sphere* spheres, uint64_t 
     ATX_CHECK_ARG(r, "renderer is NULL");
     ATX_HIP(hipStreamSynchronize(r->stream));
     r->first_valid = r->prev_valid = false;
-    int rc = upload_scene(spheres, num_spheres, materials, num_materials, lights, num_lights, &r->geo);
-    if (rc != ATX_OK) return rc;
-    r->has_scene = true;
-    return ATX_OK;
+    return upload_scene(spheres, num_spheres, materials, num_materials, lights, num_lights, &r->geo);
 }
 
 int atx_renderer_set_kernel(atx_renderer* h, int kind)
@@ -434,7 +430,7 @@ int atx_renderer_reserve(atx_renderer* h, uint32_t frames)
         ATX_HIP(r->wf_dirs.reserve(npx * sizeof(float4)));
         r->dirs_valid = r->first_valid = false;
     }
-    if (r->has_scene && r->wf_first.bytes() < first_cache_bytes(npx, r->geo.n_light)) {
+    if (r->geo.loaded() && r->wf_first.bytes() < first_cache_bytes(npx, r->geo.n_light)) {
         ATX_HIP(r->wf_first.reserve(first_cache_bytes(npx, r->geo.n_light)));
         r->first_valid = false;
     }
