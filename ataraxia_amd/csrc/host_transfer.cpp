@@ -106,13 +106,26 @@ HostStage::~HostStage()
     if (block_) (void)hipHostFree(block_);
 }
 
-hipError_t HostStage::reserve(size_t bytes)
+// The events, on the stream's device: they are recorded there, whichever device
+// the calling thread has current.
+hipError_t HostStage::make_events(hipStream_t stream)
 {
-    for (hipEvent_t& e : ev_) {
-        if (e) continue;
-        const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-        if (r != hipSuccess) return r;
-    }
+    if (ev_[kSlots - 1]) return hipSuccess;
+    int here = 0;
+    hipDevice_t there = 0;
+    hipError_t r = hipGetDevice(&here);
+    if (r == hipSuccess) r = hipStreamGetDevice(stream, &there);
+    if (r == hipSuccess && there != here) r = hipSetDevice(there);
+    for (hipEvent_t& e : ev_)
+        if (r == hipSuccess && !e) r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+    if (there != here) (void)hipSetDevice(here);
+    return r;
+}
+
+hipError_t HostStage::reserve(size_t bytes, hipStream_t stream)
+{
+    const hipError_t made = make_events(stream);
+    if (made != hipSuccess) return made;
     if (bytes <= n_) return hipSuccess;
     if (block_) (void)hipHostFree(block_);
     block_ = nullptr;
@@ -167,7 +180,7 @@ hipError_t HostStage::copy_out(void* dst, const void* src, size_t bytes, hipStre
     if (bytes == 0) return hipSuccess;
     std::lock_guard<std::mutex> lk(mu_);
     bool staged = !known_to_runtime(dst);
-    if (staged && reserve(std::min(bytes, kSlots * kPartBytes)) != hipSuccess) {
+    if (staged && reserve(std::min(bytes, kSlots * kPartBytes), stream) != hipSuccess) {
         (void)hipGetLastError();
         staged = false;
     }

@@ -36,7 +36,8 @@ private:
     // needs.  A copy of one part is copied on by the caller alone.
     static constexpr uint32_t kSlots = 4;
     static constexpr size_t kPartBytes = size_t(1) << 20;
-    hipError_t reserve(size_t bytes);
+    hipError_t make_events(hipStream_t stream);
+    hipError_t reserve(size_t bytes, hipStream_t stream);
     hipError_t copy_parts(char* dst, const char* src, size_t bytes, hipStream_t stream);
     std::mutex mu_;
     char* block_ = nullptr;

@@ -1,6 +1,7 @@
 // The HIP calls of the library's host code over plain host memory, for host
-// checks of its error paths: allocations that fail on request.  Kernels are not
-// launched.
+// checks of its error paths: allocations that fail on request, and two devices, of
+// which an event and the stream it is recorded on have to share one.  Kernels are
+// not launched.
 #pragma once
 
 #include <cstdio>
@@ -12,12 +13,16 @@
 namespace fake {
 inline int fail_mallocs = 0;     // the next so many device allocations fail
 inline int kernel_launches = 0;
+inline thread_local int device = 0;   // the thread's current one
+struct Owned {
+    int device;
+};
 }  // namespace fake
 
 extern "C" {
-hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
-hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 2; return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = fake::device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { fake::device = d; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 4; return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "fake error"; }
@@ -38,14 +43,17 @@ hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) { return hipErrorInvalidValue; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)malloc(1); return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { free((void*)s); return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t) new fake::Owned{fake::device}; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { delete (fake::Owned*)s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* d) { *d = 0; return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) { *d = ((fake::Owned*)s)->device; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t) new fake::Owned{fake::device}; return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
-hipError_t hipEventDestroy(hipEvent_t e) { free((void*)e); return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { delete (fake::Owned*)e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
+{
+    return ((fake::Owned*)e)->device == ((fake::Owned*)s)->device ? hipSuccess : hipErrorInvalidHandle;
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0.0f; return hipSuccess; }
 }

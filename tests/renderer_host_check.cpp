@@ -3,6 +3,7 @@
 #include "fake_hip.h"
 
 #include <string>
+#include <thread>
 #include <vector>
 
 static int bad = 0;
@@ -46,6 +47,24 @@ static void upload(atx_renderer* r, const atx_camera& cam)
     CHECK(atx_renderer_render(r, &cam) == ATX_OK);
 }
 
+// Results read by a thread whose current device is another one than the
+// renderer's: the first results and later ones.
+static void devices(atx_renderer* r, const atx_camera& cam)
+{
+    CHECK(set_scene(r, 3, 1) == ATX_OK);
+    CHECK(atx_renderer_render(r, &cam) == ATX_OK);
+    std::vector<uint32_t> image(16 * 8);
+    std::vector<float> sums(4 * 16 * 8);
+    std::thread([&] {
+        (void)hipSetDevice(1);
+        CHECK(atx_renderer_get_image(r, image.data(), image.size()) == ATX_OK);
+        CHECK(atx_renderer_get_accumulation(r, sums.data(), sums.size()) == ATX_OK);
+        int now = 0;
+        CHECK(hipGetDevice(&now) == hipSuccess && now == 1);
+    }).join();
+    CHECK(atx_renderer_get_image(r, image.data(), image.size()) == ATX_OK);
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
@@ -60,6 +79,7 @@ int main(int argc, char** argv)
     cam.width = 16;
     cam.height = 8;
     if (name == "upload") upload(r, cam);
+    else if (name == "devices") devices(r, cam);
     else ++bad;
     CHECK(atx_renderer_destroy(r) == ATX_OK);
     std::printf(bad ? "%d checks failed\n" : "all checks passed\n", bad);

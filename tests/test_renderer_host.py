@@ -1,4 +1,4 @@
-"""Host checks (no GPU) of the renderer's error paths: tests/renderer_host_check.cpp
+"""Host checks (no GPU) of the renderer: tests/renderer_host_check.cpp
 with the library's host code over host memory (tests/fake_hip.h)."""
 import os
 import shutil
@@ -22,7 +22,7 @@ def check(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("name", ["upload"])
+@pytest.mark.parametrize("name", ["upload", "devices"])
 def test_renderer(check, name):
     out = subprocess.run([check, name], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and "all checks passed" in out.stdout, out.stderr
