@@ -78,6 +78,18 @@ __device__ __forceinline__ const ATX_CONST T* as_const(const T* p)
     return (const ATX_CONST T*)(uintptr_t)p;
 }
 
+// The kernel's argument where it lies: read at its use, it takes no registers
+// (in place, 2001 spheres, 8 frames: 2.76 -> 2.73 ms).
+__device__ __forceinline__ const ATX_CONST WfPass& kernel_pass()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const ATX_CONST WfPass*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+    static const WfPass none{};   // the host pass only parses the kernels
+    return none;
+#endif
+}
+
 struct SphSrc {
     CF4* p;
     __device__ __forceinline__ float4 operator()(uint32_t i) const { return p[i]; }
@@ -279,7 +291,8 @@ __device__ __forceinline__ uint32_t display(float4 acc, uint32_t frame)
 
 // In-place launches: the sample of pixel px, the same in n frames of the
 // launch from f on, goes to the accumulation; the last frame's also to the image.
-__device__ __forceinline__ void add_sample(CScene* S, const WfPass& a, uint32_t px, uint32_t f, uint32_t n, f3 col)
+__device__ __forceinline__ void add_sample(CScene* S, const ATX_CONST WfPass& a, uint32_t px, uint32_t f, uint32_t n,
+                                           f3 col)
 {
     const uint32_t frame = a.frame0 + f;
     const bool kahan = S->kahan != 0u;
@@ -385,6 +398,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     // not kept: computed where it is used
     const auto counters = [&]() { return a.counters + (wave_id % kCounterLines) * kCounterStride; };
 
+    const ATX_CONST WfPass& pass = kernel_pass();
     // in place: starts pixel `job`'s path of the launch's frame f
     const auto start_in_place = [&](uint32_t f, f3 dir) {
         own[3][lane] = f;
@@ -392,10 +406,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
         rd = dir;
         tp = mk(1.0f, 1.0f, 1.0f);
         col = mk(0.0f, 0.0f, 0.0f);
-        seed = job * (a.frame0 + f);
+        seed = job * (pass.frame0 + f);
         bounce = 0;
         state = kCont;
-        capture = (S->dbg_hit || S->dbg_shadow) && f + 1u == a.frames;
+        capture = (S->dbg_hit || S->dbg_shadow) && f + 1u == pass.frames;
         for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
             if (S->dbg_hit) S->dbg_hit[(size_t)job * S->dbg_bounces + i] = -2;
             if (S->dbg_shadow) S->dbg_shadow[(size_t)job * S->dbg_bounces + i] = -2;
@@ -755,9 +769,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                 // bounce ends where it is shaded
                 const bool known = kKeep && S->n_light != 0 && S->max_bounces > 0 && !S->dbg_hit && !S->dbg_shadow;
                 const bool miss = known && (int32_t)own[4][lane] < 0;
-                const uint32_t n = miss ? a.frames - f : 1u;
-                add_sample(S, a, job, f, n, col);
-                if (f + n < a.frames) {
+                const uint32_t n = miss ? pass.frames - f : 1u;
+                add_sample(S, pass, job, f, n, col);
+                if (f + n < pass.frames) {
                     own[3][lane] = f + n;
                     if (known)
                         state = kAgain;
@@ -788,6 +802,7 @@ template <bool kFrames>
 __global__ __launch_bounds__(64) void k_render_flat(WfPass a)
 {
     CScene* const S = as_const(a.scenes);
+    const ATX_CONST WfPass& pass = kernel_pass();
     const uint32_t lane = threadIdx.x;
     const uint32_t px = in_place_pixel(blockIdx.x * 64u + lane, S->width, S->height);
     const SphSrc flat{as_const(S->sph)};
@@ -808,9 +823,9 @@ __global__ __launch_bounds__(64) void k_render_flat(WfPass a)
             rd = dir;
             tp = mk(1.0f, 1.0f, 1.0f);
             col = mk(0.0f, 0.0f, 0.0f);
-            seed = px * (a.frame0 + f);
+            seed = px * (pass.frame0 + f);
             bounce = 0;
-            capture = debug && f + 1u == a.frames;
+            capture = debug && f + 1u == pass.frames;
             for (uint32_t i = 0; capture && i < S->dbg_bounces; ++i) {
                 if (S->dbg_hit) S->dbg_hit[(size_t)px * S->dbg_bounces + i] = -2;
                 if (S->dbg_shadow) S->dbg_shadow[(size_t)px * S->dbg_bounces + i] = -2;
@@ -859,16 +874,16 @@ __global__ __launch_bounds__(64) void k_render_flat(WfPass a)
         if constexpr (!kFrames) {
             while (!step()) {
             }
-            add_sample(S, a, px, 0u, 1u, col);
+            add_sample(S, pass, px, 0u, 1u, col);
         } else {
-            while (f < a.frames) {
+            while (f < pass.frames) {
                 if (step()) {
                     // a primary ray that misses does so in every frame
                     const bool miss = bounce == 0 && first.id < 0 && !debug;
-                    const uint32_t n = miss ? a.frames - f : 1u;
-                    add_sample(S, a, px, f, n, col);
+                    const uint32_t n = miss ? pass.frames - f : 1u;
+                    add_sample(S, pass, px, f, n, col);
                     f += n;
-                    if (f < a.frames)
+                    if (f < pass.frames)
                         start();
                 }
             }
