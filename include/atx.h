@@ -112,9 +112,13 @@ typedef struct atx_render_stats {
     uint64_t samples;        /* path samples (pixels x frames)                 */
     uint64_t rays;           /* rays of the rendered paths: primary/continuation
                                 + shadow (as the reference traces them)         */
-    uint64_t sphere_tests;   /* ray-sphere tests performed                      */
-    uint64_t exact_retraces; /* traces resolved by the exact fallback loop      */
-    uint64_t box_tests;      /* ray-box tests                                   */
+    uint64_t sphere_tests;   /* ray-sphere tests; with ATX_ACCEL_NONE every pair
+                                of a ray and a sphere, most of which a matrix
+                                product decides                                 */
+    uint64_t exact_retraces; /* traces that the interval tests left open, settled
+                                by exact distances                              */
+    uint64_t box_tests;      /* ray-box tests, of boxes around 32 spheres (those
+                                around 256 are not counted)                     */
     double gpu_ms;           /* HIP-event time of the render kernels            */
     uint64_t launches;       /* path-kernel launches                            */
     double path_ms;          /* HIP-event time of the path kernel alone, summed
