@@ -29,12 +29,15 @@ Other workloads (one JSON line each):
                          WRITE_SIZE counters
 
 The roofline entry is the VALU bound of the dominant kernel: 17 algorithmic
-FLOP per ray-sphere test and 12 per box test (6 FMA; FMA = 2), both
-counted exactly by the kernels, divided by that kernel's average launch
-duration from HIP events recorded on the renderer's stream around the path
-kernel alone (the persistent kernel's launches are each followed by a short
-accumulate kernel, which is timed in `gpu_ms_per_step` but not here), against
-MI355X's published FP32 vector peak.
+FLOP per ray-sphere test and 12 per test of a tile's box (6 FMA; FMA = 2), as the
+kernels count them, divided by that kernel's average launch duration from HIP
+events recorded on the renderer's stream around the path kernel alone (the
+persistent kernel's launches are each followed by a short accumulate kernel,
+which is timed in `gpu_ms_per_step` but not here), against MI355X's published
+FP32 vector peak.  The matrix products that rule spheres of a tile out are not in
+it.  Where every ray tests every sphere ("flat"), the count is of pairs that such
+products decide: 64 FLOP a pair (32 multiply-adds in half precision), against the
+dense matrix peak.
 """
 import argparse
 import json
@@ -48,8 +51,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FP32_VALU_PEAK_TFLOPS = 157.3   # MI355X published FP32 vector peak
+F16_MATRIX_PEAK_TFLOPS = 2500.0  # MI355X dense half-precision matrix peak
 FLOP_PER_TEST = 17
 FLOP_PER_BOX = 12
+FLOP_PER_PAIR = 64               # one entry of the tiles' products: 32 terms
 
 
 def parse():
@@ -188,16 +193,20 @@ def time_single_scene(sc, kernel, accel, steps, warmup):
     return wall, st
 
 
-def algo_flops(st):
+def algo_flops(st, products=False):
+    """products: st's sphere tests are pairs that matrix products decide."""
+    if products:
+        return FLOP_PER_PAIR * st["sphere_tests"]
     return FLOP_PER_TEST * st["sphere_tests"] + FLOP_PER_BOX * st["box_tests"]
 
 
-def roofline(st, traffic, basis=None):
+def roofline(st, traffic, basis=None, products=False):
     launches = max(1, st["launches"])
     kernel_ms = st["path_ms"] / launches
-    achieved = algo_flops(st) / launches / (kernel_ms * 1e-3) / 1e12
-    return {"bound": "valu", "achieved": achieved, "peak": FP32_VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": achieved / FP32_VALU_PEAK_TFLOPS, "traffic": traffic, "traffic_basis": basis,
+    peak = F16_MATRIX_PEAK_TFLOPS if products else FP32_VALU_PEAK_TFLOPS
+    achieved = algo_flops(st, products) / launches / (kernel_ms * 1e-3) / 1e12
+    return {"bound": "mfma" if products else "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+            "frac": achieved / peak, "traffic": traffic, "traffic_basis": basis,
             "kernel_ms": kernel_ms,
             "launches": launches, "sphere_tests_per_launch": st["sphere_tests"] / launches,
             "box_tests_per_launch": st["box_tests"] / launches, "rays_per_launch": st["rays"] / launches,
@@ -219,12 +228,14 @@ def bench_plain_1080p(args):
     for k in kernels:
         for a in accels:
             wall, st = time_single_scene(sc, kid[k], aid[a], args.steps, args.warmup)
+            # --exact-loop: the plain kernel's loop over all spheres, without products
+            products = k == "wavefront" if args.exact_loop else a == "flat"
             frames_per_launch = args.steps / max(1, st["launches"])
             traffic, basis = traffic_from_profile(f"plain_1080p_k_render_{k}_{a}", "k_render_wavefront",
                                                   int(round(frames_per_launch)))
             variants[f"{k}/{a}"] = {"value": samples / wall, "ms_per_step": wall * 1e3 / args.steps,
                                     "gpu_ms_per_step": st["gpu_ms"] / args.steps,
-                                    "roofline": roofline(st, traffic, basis)}
+                                    "roofline": roofline(st, traffic, basis, products)}
     main_variant = next(iter(variants))   # wavefront/bvh unless restricted
     v = variants[main_variant]
     out = {
@@ -304,7 +315,7 @@ def bench_batch_mix(args):
         lib.atx_device_synchronize()
         pwall += time.perf_counter() - t0
         st = r.stats()
-        pflops += algo_flops(st)
+        pflops += algo_flops(st, accel == ATX_ACCEL_NONE)
         pms += st["gpu_ms"]
     r.close()
     bv, pv = samples / bwall, (samples / pwall if pwall > 0 else float("nan"))
@@ -317,7 +328,7 @@ def bench_batch_mix(args):
                                f"1..16 lights, 2..10 bounces, spp x{args.spp_scale}", "samples": samples,
                    "accel": "flat" if accel == ATX_ACCEL_NONE else "bvh", "tuning": tuning, "autotune_s": tune_s},
         "batched": {"samples_per_s": bv, "wall_s": bwall, "gpu_ms": bst["gpu_ms"],
-                    "tflops": algo_flops(bst) / (bst["gpu_ms"] * 1e-3) / 1e12},
+                    "tflops": algo_flops(bst, accel == ATX_ACCEL_NONE) / (bst["gpu_ms"] * 1e-3) / 1e12},
         "plain": {"samples_per_s": pv, "wall_s": pwall, "gpu_ms": pms,
                   "tflops": pflops / (pms * 1e-3) / 1e12 if pms > 0 else float("nan")},
         "speedup": bv / pv,
