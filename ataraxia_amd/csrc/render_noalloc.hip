@@ -82,14 +82,9 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     HostSceneLayout L;
     int rc = build_scene_layout(spheres, num_spheres, materials, num_materials, lights, num_lights, &L);
     if (rc != ATX_OK) return rc;
-    HostBvh T;
-    build_bvh(L.sph.data(), (uint32_t)num_spheres, 0, &T);
-    // a scene that fits the scratch array only without its tiles has none
-    const size_t bare = (L.sph.size() + L.sph_mat.size() + L.mat.size() + L.light.size()) * 4;
-    if (bare + (T.tiles.size() + T.tboxes.size() + T.tsph.size() + T.tidx.size() + T.big.size()) * 4 + 16 * 256 >
-        kScratchBytes)
-        T = HostBvh();
-
+    HostBvh tiles;
+    const HostBvh none;
+    build_bvh(L.sph.data(), (uint32_t)num_spheres, 0, &tiles);
     // scratch layout: counters | queue | table entry, then from kControlBytes on
     // spheres | material ids | materials | lights | tiles
     const size_t off_queue = kCounterBytes;
@@ -97,7 +92,12 @@ extern "C" int atx_render_frames_noalloc(const atx_sphere* spheres, uint64_t num
     static_assert(kCounterBytes % 256 == 0 && kQueueWords % 64 == 0, "aligned parts");
     static_assert(kCounterBytes + kQueueWords * sizeof(unsigned int) + sizeof(WfScene) <= kControlBytes,
                   "control pages");
-    const ScenePack pack(L, T, false, 256);   // as many spheres as fit
+    // a scene that fits only without its tiles has none; without lookups, so that
+    // as many spheres as possible fit
+    const ScenePack with_tiles(L, tiles, false, 256), bare(L, none, false, 256);
+    const bool tiled = with_tiles.bytes <= kScratchBytes;
+    const HostBvh& T = tiled ? tiles : none;
+    const ScenePack& pack = tiled ? with_tiles : bare;
     const size_t total = pack.bytes;
     if (total > kScratchBytes) {
         set_error("scene needs %zu bytes of device scratch; atx_render_frames_noalloc holds at most %zu "
