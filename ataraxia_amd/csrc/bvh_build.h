@@ -69,7 +69,7 @@ inline uint32_t tile_row(uint32_t k)
 // others get neither (n_tiles = n_nodes = 0).
 void build_bvh(const float* sph4, uint32_t n, uint32_t layouts, HostBvh* out);
 
-// Device bytes of the tree of an n-sphere scene (upper bound).
+// Device bytes of the tiles of an n-sphere scene (upper bound).
 size_t bvh_device_bytes(uint64_t n);
 
 }  // namespace atx

@@ -793,10 +793,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
 // instructions, which bounds it (the loads and square roots of one ray after the
 // other), stays short.  The persistent kernel's in-place mode, whose round is one ray
 // and which hands out pixels, took longer at every size (one frame, 13 spheres:
-// 64x64 51 us, here 32; 640x360 71 and 50; 1920x1080 214 and 96).
+// 64x64 51 us, here 32; 640x360 97 and 50; 1920x1080 223 and 98).
 // kFrames: a lane goes on to its next frame without waiting for the others and
 // keeps its primary hit (1280x720, 13 spheres, 32 frames: 1.54 ms with a loop over
-// frames around one over bounces, 1.33 with this one, 1.90 persistent).  A launch of
+// frames around one over bounces, 1.33 with this one, 1.88 persistent).  A launch of
 // one frame has an instance of its own, 8 % shorter.
 template <bool kFrames>
 __global__ __launch_bounds__(64) void k_render_flat(WfPass a)
@@ -1210,8 +1210,8 @@ hipError_t launch_in_place(const WfScene& s, const WfPass& pass, hipStream_t str
     if (p.total_chunks == 0 || p.n_scenes != 1 || p.frames == 0)
         return hipErrorInvalidValue;
     if (s.bvh.n_tiles == 0u) {
-        hipLaunchKernelGGL(p.frames > 1u ? k_render_flat<true> : k_render_flat<false>, dim3(p.total_chunks), dim3(64), 0,
-                           stream, p);
+        hipLaunchKernelGGL(p.frames > 1u ? k_render_flat<true> : k_render_flat<false>, dim3(p.total_chunks), dim3(64),
+                           0, stream, p);
         return hipGetLastError();
     }
     const PathKernel kernel = p.frames >= kKeepFrames ? k_render_wavefront<kWfWavesTree, true, true, true>

@@ -6,8 +6,8 @@
 //  * rays are generated on the device from the camera's inverse matrices,
 //    so there is no per-frame W*H*12 B upload, malloc or free
 //    (Camera.cpp:197-220);
-//  * no per-frame occupancy/device-property queries or full-device syncs;
-//    work is queued on the handle's own stream and `render` waits on it;
+//  * no full-device syncs; work is queued on the handle's own stream and
+//    `render` waits on it;
 //  * the RGBA8 image stays on the device until atx_renderer_get_image;
 //  * the persistent kernel (the default) renders up to 256 frames per
 //    launch, and keeps per camera and scene the primary directions and the
